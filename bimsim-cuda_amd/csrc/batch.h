@@ -178,16 +178,18 @@ int detector_run(bimsim_ctx* ctx, int prec, int quirks, void* U, void* Uf, int u
 
 // The band-limited detector over many instances of one FFT size N (uR = vR
 // = N) in three launches per pass.  Instances qualify when det_batchable:
-// ss = 1, no zero fill, the N-point row pair fits LDS.
+// ss = 1 and the N-point row pair (N the zero-filled size, if any) fits LDS;
+// they write their images whole, so none may share its image with another.
 struct DetParams {
     long long uoff;        // element offset of U and Uf
     long long image_off;   // its D, Di, Abs images
     int padding, Nd;
-    double du, dv, NAin, NAout, lambda;
+    int nin;               // the field's side (below the FFT size: zero-filled)
+    double du, dv, NAin, NAout, lambda;   // du, dv of the FFT's frequency grid
     SumFuse fz;            // Uf + Us formed as the rows load (fused batches)
 };
 struct DetBatch {
-    int N = 0, n = 0, B = 0, B2 = 0, Bc = 0, max_nc = 0, max_nd = 0;
+    int N = 0, n = 0, B = 0, B2 = 0, Bc = 0, max_nc = 0, max_nd = 0, max_nin = 0;
     bool f32 = false, fused = false;
     void* d_inst = nullptr;
     int* d_cols = nullptr;

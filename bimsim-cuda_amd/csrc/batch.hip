@@ -17,7 +17,8 @@
 //                      launch per order bucket (us_series.hip); FP64 forms:
 //                      the per-instance entry point
 //   Uf + Us            one launch over (pixel blocks, instances)
-//   detector           per instance (its own FFT size)
+//   detector           one pass per FFT size
+#include <algorithm>
 #include <map>
 #include <vector>
 
@@ -86,7 +87,8 @@ struct bimsim_batch {
     unsigned* d_inside = nullptr;
     std::vector<long long> inside_off;
     // detectors: one batched pass per FFT size, and the instances that
-    // need their own (supersampling, zero fill, sizes without a fixed plan)
+    // need their own (supersampling, rows too long for it, an image shared
+    // with another instance)
     std::vector<DetBatch> det;
     std::vector<int> det_single;
     hipGraph_t graph = nullptr;
@@ -255,6 +257,33 @@ int enqueue(bimsim_batch* b) {
     return BIMSIM_OK;
 }
 
+// Whether instance i's detector goes with the others of its FFT size: it
+// qualifies, and its image is its own (the batched pass writes images whole;
+// an image that several instances share holds their sum).
+std::vector<char> batched_detectors(const bimsim_ctx* ctx, int prec, const bimsim_instance* inst,
+                                    int n) {
+    std::vector<int> order(n);
+    std::vector<char> ok(n);
+    for (int i = 0; i < n; ++i) {
+        order[i] = i;
+        ok[i] = det_batchable(ctx, prec, inst[i].N, inst[i].ss, inst[i].zero_fill);
+    }
+    std::sort(order.begin(), order.end(),
+              [&](int a, int b) { return inst[a].image_off < inst[b].image_off; });
+    // runs of images that overlap, each image's end against the run's
+    for (int a = 0; a < n;) {
+        long long end = inst[order[a]].image_off + (long long)inst[order[a]].Nd * inst[order[a]].Nd;
+        int b = a + 1;
+        for (; b < n && inst[order[b]].image_off < end; ++b)
+            end = std::max(end, inst[order[b]].image_off +
+                                    (long long)inst[order[b]].Nd * inst[order[b]].Nd);
+        if (b - a > 1)
+            for (int k = a; k < b; ++k) ok[order[k]] = 0;
+        a = b;
+    }
+    return ok;
+}
+
 double len3(const double* v) { return std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]); }
 
 int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphere* spheres,
@@ -279,6 +308,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     b->dv.resize(n);
     b->field_off.resize(n);
     long long coef = 0, field = 0;
+    const std::vector<char> batched = batched_detectors(ctx, b->prec, inst, n);
     for (int i = 0; i < n; ++i) {
         const bimsim_instance& I = inst[i];
         BIMSIM_CHECK_ARG(ctx, I.N > 0 && (long long)I.N * I.N <= (1LL << 28), "instance N out of range");
@@ -327,7 +357,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         }
         // images to clear each pass: those of the instances whose detector
         // adds to them (the batched detector writes its images whole)
-        const int nd2 = det_batchable(ctx, b->prec, I.N, I.ss, I.zero_fill) ? 0 : I.Nd * I.Nd;
+        const int nd2 = batched[i] ? 0 : I.Nd * I.Nd;
         sum[i] = SumInst{q, I.N, I.N, (int)sph_dev.size(), I.ns, field, I.image_off, nd2};
         for (int c = 0; c < 3; ++c) kdirs[3 * (size_t)i + c] = I.kdir[c];
         // spheres of this instance, coefficients packed
@@ -431,8 +461,8 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         // then cleared by the pre-pass launch or the incident-field launch
         b->fuse_sum = true;
         for (int i = 0; i < n; ++i)
-            b->fuse_sum = b->fuse_sum && inst[i].zero_fill <= 1 &&
-                          detector_fusable(ctx, inst[i].N, inst[i].N);
+            b->fuse_sum = b->fuse_sum && (batched[i] || (inst[i].zero_fill <= 1 &&
+                                                         detector_fusable(ctx, inst[i].N, inst[i].N)));
         if (b->fuse_sum) {
             b->sum_host = sum;
             b->pre.sum = b->d_sum;
@@ -458,7 +488,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     std::map<int, std::vector<DetParams>> by_size;
     for (int i = 0; i < n; ++i) {
         const bimsim_instance& I = inst[i];
-        if (!det_batchable(ctx, b->prec, I.N, I.ss, I.zero_fill)) {
+        if (!batched[i]) {
             b->det_single.push_back(i);
             continue;
         }
@@ -467,8 +497,10 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         q.image_off = I.image_off;
         q.padding = I.padding;
         q.Nd = I.Nd;
-        q.du = b->du[i];
-        q.dv = b->dv[i];
+        q.nin = I.N;
+        const int fill = std::max(1, I.zero_fill);
+        q.du = b->du[i] / fill;
+        q.dv = b->dv[i] / fill;
         q.NAin = I.objective[0];
         q.NAout = I.objective[1];
         q.lambda = I.lambda;
@@ -477,7 +509,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
             q.fz = SumFuse{S.q, S.uR, S.vR, S.ns, b->d_sph4 + S.s_begin,
                            b->d_inside + b->inside_off[i]};
         }
-        by_size[I.N].push_back(q);
+        by_size[I.N * fill].push_back(q);
     }
     for (auto& kv : by_size) {
         b->det.emplace_back();

@@ -1,12 +1,13 @@
 // Detector: microscopeStruct::SimulateImaging (reference microscope.cu:
 // 608-662, 722-791; fieldslice.cpp:25-94; fieldslice.cu:71-153,319-362).
 //
-// 2D FFT as two passes of batched 1D Stockham FFTs staged in LDS (one
+// Band-limited 2D FFT as batched 1D Stockham FFTs staged in LDS (one
 // workgroup owns B lines of length N; radix 4/2/3/5 stages ping-pong between
-// two LDS buffers).  The objective band-pass is applied in the store phase of
-// the forward column pass, the 1/(uR vR) scale in the store phase of the
-// inverse row pass.  A final kernel crops, forms |U|^2 averaged over ss x ss
-// into D and Di (accumulating, like resample_intensity) and -log10(D/Di).
+// two LDS buffers), any N of factors 2, 3 and 5: forward rows keep only the
+// pass-band columns, each column takes its forward transform, the objective
+// band-pass, the inverse transform and the 1/(uR vR) scale in one pass, and
+// the inverse rows end in |U|^2, averaged over ss x ss into D and Di
+// (accumulating, like resample_intensity), and -log10(D/Di).
 // FP64 instantiations run in FP64 end to end (-ffp-contract=off for the
 // whole translation unit); FP32 ones in float with FP64-accurate twiddles.
 #include <mutex>
@@ -61,7 +62,7 @@ __device__ inline C cmk(decltype(C::x) a, decltype(C::x) b) {
 
 // Post-operation applied when a pass stores its results.
 struct PostOp {
-    int kind;        // 0 none, 1 objective band-pass (freq. index = (elem, line)), 2 scale
+    int kind;        // 0 none, 1 objective band-pass (the band-limited passes), 2 scale
     int uR, vR;
     int quirks;
     double du, dv, fmin, fmax;   // fmin = NAin/lambda, fmax = NAout/lambda
@@ -86,6 +87,7 @@ __device__ inline bool passband(const PostOp& op, int iu, int iv) {
 struct DetInst {
     long long uoff, g_off, image_off;
     int cols_off, Nc, off, Nd;
+    int nin;         // the field's own side (less than the FFT size: zero-filled)
     PostOp bp;
     SumFuse fz;
 };
@@ -199,39 +201,11 @@ __global__ __launch_bounds__(kThreads) void fft_lines_kernel(
         if (lines_fast) { g = t % nb; e = t / nb; }
         else { e = t % N; g = t / N; }
         C v = src[g * P + e];
-        if (op.kind == 1) {
-            // frequency indices: elements run along v (column pass), lines along u
-            const int iu = g0 + g, iv = e;
-            if (!passband(op, iu, iv)) v = cmk<C>((R)0, (R)0);
-        } else if (op.kind == 2) {
+        if (op.kind == 2) {
             v = cmk<C>(v.x * (R)op.scale, v.y * (R)op.scale);
         }
         data[(long long)(g0 + g) * line_stride + (long long)e * elem_stride] = v;
     }
-}
-
-// crop + resample_intensity (+=) + calc_absorbance, per detector pixel
-template <class R>
-__global__ void detect_kernel(const typename C2<R>::T* __restrict__ U,
-                              const typename C2<R>::T* __restrict__ Uf, int uR, int off, int Nd,
-                              int ss, R* __restrict__ D, R* __restrict__ Di, R* __restrict__ Abs) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= Nd * Nd) return;
-    const int iv = i / Nd, iu = i - iv * Nd;
-    R I = 0, Ii = 0;
-    for (int ix = 0; ix < ss; ++ix)
-        for (int iy = 0; iy < ss; ++iy) {
-            const long long fi = (long long)(off + iv * ss + iy) * uR + (off + iu * ss + ix);
-            const auto a = U[fi], b = Uf[fi];
-            const R am = sqrt(a.x * a.x + a.y * a.y), bm = sqrt(b.x * b.x + b.y * b.y);
-            I += am * am;
-            Ii += bm * bm;
-        }
-    const R d = D[i] + I / (R)(ss * ss);
-    const R di = Di[i] + Ii / (R)(ss * ss);
-    D[i] = d;
-    Di[i] = di;
-    if (Abs) Abs[i] = -log10(d / di);
 }
 
 // ------------------------------------------------ fixed-length line FFTs
@@ -316,6 +290,105 @@ __device__ __forceinline__ typename C2<R>::T* fixed_fft(typename C2<R>::T* a,
     }
 }
 
+// ---------------------------------------- line FFTs of any supported length
+// The lengths without a fixed plan (products of 2, 3 and 5 outside the list
+// below) take the same kernels with their stage plan as an argument: the
+// divisions by a stage's span are multiplications by a host-made reciprocal
+// (t = floor(x d') 2^-32, exact for x d < 2^32; every index here is below
+// 2^15 and every divisor at most 10240), and each radix has its own unrolled
+// stage.  Bound by LDS traffic and latency, not by memory; what it replaces
+// transformed whole arrays in place, eight passes of strided lines with
+// run-time radices and integer divisions: a 720 x 720 FP64 detector with
+// 2 x 2 samples 1.25 -> 0.098 ms, 96 ragged images (sides 256 to 1024, two
+// thirds of them without a compiled length) 30.8 -> 5.7 ms a pass.
+constexpr int kRtStages = 14;   // 2^14 exceeds the longest line of the LDS
+struct RtPlan {
+    int n, nst;
+    unsigned mn;   // reciprocal of n (0: n = 1)
+    int rad[kRtStages];
+    unsigned mq[kRtStages], ms[kRtStages];   // of n / rad, and of the span before the stage
+};
+
+__host__ __device__ inline unsigned rt_magic(int d) {
+    return d <= 1 ? 0u : (unsigned)((0x100000000ull + (unsigned)d - 1) / (unsigned)d);
+}
+__device__ __forceinline__ int rt_div(int x, unsigned magic) {
+    return magic == 0u ? x : (int)__umulhi((unsigned)x, magic);
+}
+
+// The length of a kernel's lines: N, or with N = 0 the plan it carries.
+template <int N>
+struct Len {
+    __device__ __forceinline__ int n() const { return N; }
+    __device__ __forceinline__ int div(int x) const { return x / N; }
+};
+template <>
+struct Len<0> {
+    RtPlan p;
+    __device__ __forceinline__ int n() const { return p.n; }
+    __device__ __forceinline__ int div(int x) const { return rt_div(x, p.mn); }
+};
+
+template <class R, int r>
+__device__ __forceinline__ void rt_stage(const typename C2<R>::T* __restrict__ src,
+                                         typename C2<R>::T* __restrict__ dst, int nb, int N,
+                                         int Ns, unsigned mq, unsigned ms,
+                                         const typename C2<R>::T* __restrict__ tw, R sgn,
+                                         bool inverse) {
+    using C = typename C2<R>::T;
+    const int nq = N / r;
+    const int tstep = nq / Ns;
+    for (int t = threadIdx.x; t < nb * nq; t += kThreads) {
+        const int g = rt_div(t, mq), j = t - g * nq;
+        const int jd = rt_div(j, ms), k = j - jd * Ns;
+        const C* in = src + g * N + j;
+        C x[r];
+#pragma unroll
+        for (int q = 0; q < r; ++q) x[q] = in[q * nq];
+        if (Ns > 1) {
+#pragma unroll
+            for (int q = 1; q < r; ++q) {
+                C w = tw[k * q * tstep];
+                if (inverse) w.y = -w.y;
+                x[q] = cmk<C>(x[q].x * w.x - x[q].y * w.y, x[q].x * w.y + x[q].y * w.x);
+            }
+        }
+        butterfly<R>(x, r, sgn);
+        C* out = dst + g * N + jd * Ns * r + k;
+#pragma unroll
+        for (int q = 0; q < r; ++q) out[q * Ns] = x[q];
+    }
+}
+
+// nb lines' transforms, from a (b: the other buffer); returns the buffer that
+// holds them, in natural order.
+template <class R, int N>
+__device__ __forceinline__ typename C2<R>::T* line_fft(const Len<N>& L, typename C2<R>::T* a,
+                                                      typename C2<R>::T* b, int nb,
+                                                      const typename C2<R>::T* tw, bool inverse) {
+    if constexpr (N > 0) {
+        return fixed_fft<R, N>(a, b, nb, tw, inverse);
+    } else {
+        using C = typename C2<R>::T;
+        const R sgn = inverse ? (R)1 : (R)-1;
+        int Ns = 1;
+        for (int st = 0; st < L.p.nst; ++st) {
+            const int r = L.p.rad[st];
+            const unsigned mq = L.p.mq[st], ms = L.p.ms[st];
+            if (r == 4) rt_stage<R, 4>(a, b, nb, L.p.n, Ns, mq, ms, tw, sgn, inverse);
+            else if (r == 5) rt_stage<R, 5>(a, b, nb, L.p.n, Ns, mq, ms, tw, sgn, inverse);
+            else if (r == 3) rt_stage<R, 3>(a, b, nb, L.p.n, Ns, mq, ms, tw, sgn, inverse);
+            else rt_stage<R, 2>(a, b, nb, L.p.n, Ns, mq, ms, tw, sgn, inverse);
+            __syncthreads();
+            C* t = a;
+            a = b;
+            b = t;
+            Ns *= r;
+        }
+        return a;
+    }
+}
+
 // Whether pixel pix of a batch instance lies inside one of its spheres, by
 // the rule of the batch's sum kernel (d < a is inside, nfSumUf.cu:31-48).
 // Only the spheres of `near` (bit s: sphere s) are tested when fz.ns <= 64;
@@ -376,6 +449,7 @@ __global__ __launch_bounds__(kThreads) void sum_mask_kernel(SumFuse fz, unsigned
 // (beside its other first loads) and stored to a copy in LDS later.
 template <class C, int N>
 struct TwShare {
+    static_assert(N > 0, "the run-time lengths copy their twiddles in a loop");
     static constexpr int kPer = (N + kThreads - 1) / kThreads;
     C v[kPer];
     __device__ __forceinline__ void load(const C* __restrict__ tw) {
@@ -389,176 +463,170 @@ struct TwShare {
     }
 };
 
-// Forward FFT of B rows (length N) of U (f = 0) or Uf (f = 1); the
-// pass-band columns cols[0..Nc) go to the compact spectrum
-// G[(field*Nc + c)*nrows + row].  kSum: U is the scattered field alone and
-// the rows of U load as fused_sum(fz, ...).  kBoth: the rows of both
-// fields in one transform of 2 nb rows (U's, then Uf's; f unused), each Uf
-// element loaded once for both.  kTwLds: the twiddles read from a copy in
-// LDS (N more elements past the transform's buffers), not through the
-// vector caches at every stage.
+// Forward FFT of B rows of U (f = 0) or Uf (f = 1), nin elements each, zero
+// past them up to the FFT length; the pass-band columns cols[0..Nc) go to
+// the compact spectrum G[(field*Nc + c)*gs + row].  kSum: U is the scattered
+// field alone and the rows of U load as fused_sum(fz, ...).  kBoth: the rows
+// of both fields in one transform of 2 nb rows (U's, then Uf's; f unused),
+// each Uf element loaded once for both.  kTwLds: the twiddles read from a
+// copy in LDS (N more elements past the transform's buffers), not through
+// the vector caches at every stage.
 template <class R, int N, bool kSum, bool kBoth = false, bool kTwLds = false>
 __device__ __forceinline__ void rows_fwd_body(
-    const typename C2<R>::T* __restrict__ U, const typename C2<R>::T* __restrict__ Uf, int nrows,
-    int B, const int* __restrict__ cols, int Nc, typename C2<R>::T* __restrict__ G,
+    const Len<N>& L, const typename C2<R>::T* __restrict__ U,
+    const typename C2<R>::T* __restrict__ Uf, int nin, int nrows, int gs, int B,
+    const int* __restrict__ cols, int Nc, typename C2<R>::T* __restrict__ G,
     const typename C2<R>::T* __restrict__ tw, const SumFuse& fz, int blk, int f) {
     using C = typename C2<R>::T;
     constexpr int kF = kBoth ? 2 : 1;   // fields in the transform
+    const int n = L.n();
     extern __shared__ unsigned char smem_raw[];
     C* a = reinterpret_cast<C*>(smem_raw);
-    C* b = a + (size_t)kF * B * N;
+    C* b = a + (size_t)kF * B * n;
     if (kBoth) f = 0;
-    const C* F = f ? Uf : U;
     const int row0 = blk * B;
     const int nb = min(B, nrows - row0);
     const C* twp = tw;
-    TwShare<C, N> tws;
-    if constexpr (kTwLds) {
-        tws.load(tw);
-        twp = b + (size_t)kF * B * N;
-    }
+    if constexpr (kTwLds) twp = b + (size_t)kF * B * n;
+    [[maybe_unused]] TwShare<C, (kTwLds && N > 0 ? N : 1)> tws;
+    if constexpr (kTwLds && N > 0) tws.load(tw);
+    const int tot = nb * n;
+    const bool pad = nin != n;
+    // the field element of index t of the transform; false past the row's end
+    auto index = [&](int t, size_t* i) {
+        if (!pad) {
+            *i = (size_t)row0 * n + t;
+            return true;
+        }
+        const int g = L.div(t), e = t - g * n;
+        *i = (size_t)(row0 + g) * nin + min(e, nin - 1);
+        return e < nin;
+    };
+    const C zero = cmk<C>((R)0, (R)0);
     if (kBoth && !(kSum && fz.ns > 0 && !fz.inside)) {
         // fused_sum with the inside bits (or no spheres), written out so that
         // the loop body has no branch: four elements of each field (and
         // their mask words) a step, every load issued before the first
         // value is used
-        const int n = nb * N;
         const bool none = !kSum || fz.ns == 0;
-        for (int t0 = threadIdx.x; t0 < n; t0 += 4 * kThreads) {
+        for (int t0 = threadIdx.x; t0 < tot; t0 += 4 * kThreads) {
             C u[4], w[4];
             unsigned mk[4];
+            bool ok[4], in[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int t = min(t0 + k * kThreads, n - 1);
-                const size_t i = (size_t)row0 * N + t;
+                size_t i;
+                ok[k] = index(min(t0 + k * kThreads, tot - 1), &i);
                 u[k] = U[i];
                 w[k] = Uf[i];
                 mk[k] = kSum && !none ? fz.inside[i >> 5] : 0u;
+                in[k] = ((mk[k] >> (i & 31)) & 1u) != 0;
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int t = t0 + k * kThreads;
-                if (t >= n) break;
-                const int i = row0 * N + t;
+                if (t >= tot) break;
                 C v = u[k];
                 if (kSum) {
-                    const bool in = ((mk[k] >> (i & 31)) & 1u) != 0;
                     C s = v;
                     s.x = v.x + w[k].x;
                     s.y = v.y + w[k].y;
-                    v = none ? w[k] : (in ? v : s);
+                    v = none ? w[k] : (in[k] ? v : s);
                 }
-                a[t] = v;
-                a[n + t] = w[k];
+                a[t] = ok[k] ? v : zero;
+                a[tot + t] = ok[k] ? w[k] : zero;
             }
-        }
-    } else if (kSum && f == 0 && fz.inside) {
-        for (int t = threadIdx.x; t < nb * N; t += kThreads) {
-            const size_t i = (size_t)row0 * N + t;
-            a[t] = fused_sum(fz, (int)i, U[i], Uf[i]);
-        }
-    } else if (kSum && f == 0) {
-        // the spheres within their radius of these rows' bounding box (the
-        // box of the four corner pixels holds every pixel of the rows): the
-        // others cannot hold one of their pixels
-        __shared__ unsigned long long s_near;
-        if (threadIdx.x < 64) {
-            bool near = false;
-            if ((int)threadIdx.x < fz.ns && fz.ns <= 64) {
-                const double v0 = (double)row0 / (double)fz.vR;
-                const double v1 = (double)(row0 + nb - 1) / (double)fz.vR;
-                const double u1 = (double)(fz.uR - 1) / (double)fz.uR;
-                const d3 c0 = quad_at(fz.q, 0.0, v0), c1 = quad_at(fz.q, u1, v0);
-                const d3 c2 = quad_at(fz.q, 0.0, v1), c3 = quad_at(fz.q, u1, v1);
-                const double4 S = fz.sph[threadIdx.x];
-                const double cc[3] = {S.x, S.y, S.z};
-                const double q0[3] = {c0.x, c0.y, c0.z}, q1[3] = {c1.x, c1.y, c1.z};
-                const double q2[3] = {c2.x, c2.y, c2.z}, q3[3] = {c3.x, c3.y, c3.z};
-                double d2 = 0.0;
-                for (int x = 0; x < 3; ++x) {
-                    const double lo = fmin(fmin(q0[x], q1[x]), fmin(q2[x], q3[x]));
-                    const double hi = fmax(fmax(q0[x], q1[x]), fmax(q2[x], q3[x]));
-                    const double g = fmax(fmax(lo - cc[x], cc[x] - hi), 0.0);
-                    d2 += g * g;
-                }
-                near = d2 <= S.w * S.w * (1.0 + 1e-9);
-            }
-            const unsigned long long m = __ballot(near);
-            if (threadIdx.x == 0) s_near = m;
-        }
-        __syncthreads();
-        const unsigned long long near = s_near;
-        for (int t = threadIdx.x; t < nb * N; t += kThreads) {
-            const size_t i = (size_t)row0 * N + t;
-            const C w = Uf[i];
-            a[t] = fused_sum(fz, (int)i, U[i], w, near);
-            if (kBoth) a[nb * N + t] = w;
         }
     } else {
-        for (int t = threadIdx.x; t < nb * N; t += kThreads) a[t] = F[(size_t)row0 * N + t];
+        const C* F = f ? Uf : U;
+        for (int t = threadIdx.x; t < tot; t += kThreads) {
+            size_t i;
+            const bool ok = index(t, &i);
+            C v = F[i];
+            if (kBoth || (kSum && f == 0)) {
+                const C w = Uf[i];
+                if (kSum) v = fused_sum(fz, (int)i, v, w);
+                if (kBoth) a[tot + t] = ok ? w : zero;
+            }
+            a[t] = ok ? v : zero;
+        }
     }
     // (the barrier below covers the copy)
-    if constexpr (kTwLds) tws.store(b + (size_t)kF * B * N);
+    if constexpr (kTwLds && N > 0) tws.store(b + (size_t)kF * B * n);
+    if constexpr (kTwLds && N == 0)
+        for (int t = threadIdx.x; t < n; t += kThreads) b[(size_t)kF * B * n + t] = tw[t];
     // the column of the thread's first output, read before the transform
     // (the rest, if any, as they come)
     const int nout = kF * nb * Nc;
     const int col0 = (int)threadIdx.x < nout ? cols[(int)threadIdx.x % Nc] : 0;
     __syncthreads();
-    const C* res = fixed_fft<R, N>(a, b, kF * nb, twp, false);
+    const C* res = line_fft<R, N>(L, a, b, kF * nb, twp, false);
     for (int t = threadIdx.x; t < nout; t += kThreads) {
         const int h = kBoth ? t / (nb * Nc) : 0, u = t - h * (nb * Nc);
         const int g = u / Nc, c = u - g * Nc;
         const int col = t == (int)threadIdx.x ? col0 : cols[c];
-        G[((size_t)(f + h) * Nc + c) * nrows + row0 + g] = res[(h * nb + g) * N + col];
+        G[((size_t)(f + h) * Nc + c) * gs + row0 + g] = res[(h * nb + g) * n + col];
     }
 }
 
 template <class R, int N, bool kSum>
 __global__ __launch_bounds__(kThreads) void rows_fwd_kernel(
-    const typename C2<R>::T* __restrict__ U, const typename C2<R>::T* __restrict__ Uf, int nrows,
-    int B, const int* __restrict__ cols, int Nc, typename C2<R>::T* __restrict__ G,
-    const typename C2<R>::T* __restrict__ tw, SumFuse fz) {
-    rows_fwd_body<R, N, kSum>(U, Uf, nrows, B, cols, Nc, G, tw, fz, blockIdx.x, blockIdx.y);
+    Len<N> L, const typename C2<R>::T* __restrict__ U, const typename C2<R>::T* __restrict__ Uf,
+    int nin, int nrows, int gs, int B, const int* __restrict__ cols, int Nc,
+    typename C2<R>::T* __restrict__ G, const typename C2<R>::T* __restrict__ tw, SumFuse fz) {
+    rows_fwd_body<R, N, kSum>(L, U, Uf, nin, nrows, gs, B, cols, Nc, G, tw, fz, blockIdx.x,
+                              blockIdx.y);
 }
 
-// Pass-band columns of the compact spectrum, each: forward FFT along v,
-// objective band-pass, inverse FFT, scale 1/(uR vR).  In place in G.
+// Pass-band columns of the compact spectrum, each: forward FFT along v of
+// its first nin rows (zero past them), objective band-pass, inverse FFT,
+// scale 1/(uR vR), rows [w0, w0 + wn) stored.  In place in G.
 template <class R, int M>
-__device__ __forceinline__ void cols_band_body(typename C2<R>::T* __restrict__ G, int Nc, int B,
+__device__ __forceinline__ void cols_band_body(const Len<M>& L, typename C2<R>::T* __restrict__ G,
+                                               int nin, int w0, int wn, int Nc, int B,
                                                const int* __restrict__ cols, const PostOp& bp,
                                                const typename C2<R>::T* __restrict__ tw, int blk,
                                                int f) {
     using C = typename C2<R>::T;
+    const int m = L.n();
     extern __shared__ unsigned char smem_raw[];
     C* a = reinterpret_cast<C*>(smem_raw);
-    C* b = a + (size_t)B * M;
+    C* b = a + (size_t)B * m;
     const int c0 = blk * B;
     const int nb = min(B, Nc - c0);
-    C* line = G + ((size_t)f * Nc + c0) * M;
-    for (int t = threadIdx.x; t < nb * M; t += kThreads) a[t] = line[t];
+    C* line = G + ((size_t)f * Nc + c0) * m;
+    if (nin == m) {
+        for (int t = threadIdx.x; t < nb * m; t += kThreads) a[t] = line[t];
+    } else {
+        for (int t = threadIdx.x; t < nb * m; t += kThreads) {
+            C v = cmk<C>((R)0, (R)0);
+            if (t - L.div(t) * m < nin) v = line[t];
+            a[t] = v;
+        }
+    }
     __syncthreads();
-    C* res = fixed_fft<R, M>(a, b, nb, tw, false);
+    C* res = line_fft<R, M>(L, a, b, nb, tw, false);
     C* other = res == a ? b : a;
-    for (int t = threadIdx.x; t < nb * M; t += kThreads) {
-        const int g = t / M, iv = t - g * M;
+    for (int t = threadIdx.x; t < nb * m; t += kThreads) {
+        const int g = L.div(t), iv = t - g * m;
         if (!passband(bp, cols[c0 + g], iv)) res[t] = cmk<C>((R)0, (R)0);
     }
     __syncthreads();
-    res = fixed_fft<R, M>(res, other, nb, tw, true);
+    res = line_fft<R, M>(L, res, other, nb, tw, true);
     const R sc = (R)bp.scale;
-    for (int t = threadIdx.x; t < nb * M; t += kThreads) {
+    for (int t = threadIdx.x; t < nb * m; t += kThreads) {
+        const int iv = t - L.div(t) * m - w0;
+        if (iv < 0 || iv >= wn) continue;
         const C v = res[t];
         line[t] = cmk<C>(v.x * sc, v.y * sc);
     }
 }
 
 template <class R, int M>
-__global__ __launch_bounds__(kThreads) void cols_band_kernel(typename C2<R>::T* __restrict__ G,
-                                                             int Nc, int B,
-                                                             const int* __restrict__ cols,
-                                                             PostOp bp,
-                                                             const typename C2<R>::T* __restrict__ tw) {
-    cols_band_body<R, M>(G, Nc, B, cols, bp, tw, blockIdx.x, blockIdx.y);
+__global__ __launch_bounds__(kThreads) void cols_band_kernel(
+    Len<M> L, typename C2<R>::T* __restrict__ G, int nin, int w0, int wn, int Nc, int B,
+    const int* __restrict__ cols, PostOp bp, const typename C2<R>::T* __restrict__ tw) {
+    cols_band_body<R, M>(L, G, nin, w0, wn, Nc, B, cols, bp, tw, blockIdx.x, blockIdx.y);
 }
 
 // Inverse FFT of rows [row_begin, row_begin + nrows) of U/Uf from the compact
@@ -567,30 +635,31 @@ __global__ __launch_bounds__(kThreads) void cols_band_kernel(typename C2<R>::T* 
 // Uw/Ufw are given, the band-passed field itself.
 template <class R, int N>
 __global__ __launch_bounds__(kThreads) void rows_inv_kernel(
-    const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
+    Len<N> L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
     int row_begin, int nrows, int B, R* __restrict__ I, typename C2<R>::T* __restrict__ Uw,
     typename C2<R>::T* __restrict__ Ufw, const typename C2<R>::T* __restrict__ tw) {
     using C = typename C2<R>::T;
+    const int n = L.n();
     extern __shared__ unsigned char smem_raw[];
     C* a = reinterpret_cast<C*>(smem_raw);
-    C* b = a + (size_t)B * N;
+    C* b = a + (size_t)B * n;
     const int f = blockIdx.y;
     const int r0 = row_begin + blockIdx.x * B;
     const int nb = min(B, row_begin + nrows - r0);
-    for (int t = threadIdx.x; t < nb * N; t += kThreads) a[t] = cmk<C>((R)0, (R)0);
+    for (int t = threadIdx.x; t < nb * n; t += kThreads) a[t] = cmk<C>((R)0, (R)0);
     __syncthreads();
     for (int t = threadIdx.x; t < nb * Nc; t += kThreads) {
         const int g = t / Nc, c = t - g * Nc;
-        a[g * N + cols[c]] = G[((size_t)f * Nc + c) * vR + r0 + g];
+        a[g * n + cols[c]] = G[((size_t)f * Nc + c) * vR + r0 + g];
     }
     __syncthreads();
-    const C* res = fixed_fft<R, N>(a, b, nb, tw, true);
+    const C* res = line_fft<R, N>(L, a, b, nb, tw, true);
     C* W = f ? Ufw : Uw;
-    for (int t = threadIdx.x; t < nb * N; t += kThreads) {
+    for (int t = threadIdx.x; t < nb * n; t += kThreads) {
         const C v = res[t];
-        if (W) W[(size_t)r0 * N + t] = v;
+        if (W) W[(size_t)r0 * n + t] = v;
         const R m = sqrt(v.x * v.x + v.y * v.y);
-        I[((size_t)f * nrows + (r0 - row_begin)) * N + t] = m * m;
+        I[((size_t)f * nrows + (r0 - row_begin)) * n + t] = m * m;
     }
 }
 
@@ -604,21 +673,20 @@ __global__ __launch_bounds__(kThreads) void rows_inv_kernel(
 // kTwLds: the twiddles read from a copy in LDS, as in rows_fwd_body.
 template <class R, int N, bool kAdd = true, bool kTwLds = false>
 __device__ __forceinline__ void rows_inv_detect_body(
-    const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
+    const Len<N>& L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
     int row_begin, int nrows, int B, int off, int Nd, R* __restrict__ D, R* __restrict__ Di,
     R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw, int blk) {
     using C = typename C2<R>::T;
+    const int n = L.n();
     extern __shared__ unsigned char smem_raw[];
     C* a = reinterpret_cast<C*>(smem_raw);
-    C* b = a + (size_t)2 * B * N;
+    C* b = a + (size_t)2 * B * n;
     const int r0 = row_begin + blk * B;
     const int nb = min(B, row_begin + nrows - r0);
     const C* twp = tw;
-    TwShare<C, N> tws;
-    if constexpr (kTwLds) {
-        tws.load(tw);
-        twp = b + (size_t)2 * B * N;
-    }
+    if constexpr (kTwLds) twp = b + (size_t)2 * B * n;
+    [[maybe_unused]] TwShare<C, (kTwLds && N > 0 ? N : 1)> tws;
+    if constexpr (kTwLds && N > 0) tws.load(tw);
     // the spectrum element of the thread's first scatter and its column,
     // loaded beside the twiddles before the clearing (the rest, if any, as
     // they come)
@@ -626,14 +694,16 @@ __device__ __forceinline__ void rows_inv_detect_body(
     auto spec = [&](int t, int* col) {
         const int f = t / (nb * Nc), u = t - f * (nb * Nc);
         const int g = u / Nc, c = u - g * Nc;
-        *col = (f * nb + g) * N + cols[c];
+        *col = (f * nb + g) * n + cols[c];
         return G[((size_t)f * Nc + c) * vR + r0 + g];
     };
     int col0 = 0;
     C v0 = cmk<C>((R)0, (R)0);
     if ((int)threadIdx.x < nsc) v0 = spec(threadIdx.x, &col0);
-    for (int t = threadIdx.x; t < 2 * nb * N; t += kThreads) a[t] = cmk<C>((R)0, (R)0);
-    if constexpr (kTwLds) tws.store(b + (size_t)2 * B * N);
+    for (int t = threadIdx.x; t < 2 * nb * n; t += kThreads) a[t] = cmk<C>((R)0, (R)0);
+    if constexpr (kTwLds && N > 0) tws.store(b + (size_t)2 * B * n);
+    if constexpr (kTwLds && N == 0)
+        for (int t = threadIdx.x; t < n; t += kThreads) b[(size_t)2 * B * n + t] = tw[t];
     __syncthreads();
     for (int t = threadIdx.x; t < nsc; t += kThreads) {
         int col = col0;
@@ -641,10 +711,10 @@ __device__ __forceinline__ void rows_inv_detect_body(
         a[col] = v;
     }
     __syncthreads();
-    const C* res = fixed_fft<R, N>(a, b, 2 * nb, twp, true);
+    const C* res = line_fft<R, N>(L, a, b, 2 * nb, twp, true);
     for (int t = threadIdx.x; t < nb * Nd; t += kThreads) {
         const int g = t / Nd, iu = t - g * Nd;
-        const C v = res[g * N + off + iu], w = res[(nb + g) * N + off + iu];
+        const C v = res[g * n + off + iu], w = res[(nb + g) * n + off + iu];
         const R m = sqrt(v.x * v.x + v.y * v.y), mf = sqrt(w.x * w.x + w.y * w.y);
         const size_t i = (size_t)(r0 - row_begin + g) * Nd + iu;
         const R d = kAdd ? D[i] + m * m : m * m, di = kAdd ? Di[i] + mf * mf : mf * mf;
@@ -656,10 +726,10 @@ __device__ __forceinline__ void rows_inv_detect_body(
 
 template <class R, int N>
 __global__ __launch_bounds__(kThreads) void rows_inv_detect_kernel(
-    const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
+    Len<N> L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
     int row_begin, int nrows, int B, int off, int Nd, R* __restrict__ D, R* __restrict__ Di,
     R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
-    rows_inv_detect_body<R, N>(G, Nc, vR, cols, row_begin, nrows, B, off, Nd, D, Di, Abs, tw,
+    rows_inv_detect_body<R, N>(L, G, Nc, vR, cols, row_begin, nrows, B, off, Nd, D, Di, Abs, tw,
                                blockIdx.x);
 }
 
@@ -670,43 +740,43 @@ __global__ __launch_bounds__(kThreads) void rows_inv_detect_kernel(
 // columns return (uniformly per block).
 template <class R, int N, bool kSum, bool kTwLds>
 __global__ __launch_bounds__(kThreads) void rows_fwd_batch_kernel(
-    const DetInst* __restrict__ insts, int n, const typename C2<R>::T* __restrict__ U,
+    Len<N> L, const DetInst* __restrict__ insts, int n, const typename C2<R>::T* __restrict__ U,
     const typename C2<R>::T* __restrict__ Uf, int B, const int* __restrict__ cols,
     typename C2<R>::T* __restrict__ G, const typename C2<R>::T* __restrict__ tw) {
     for (int z = blockIdx.z; z < n; z += gridDim.z) {
         const DetInst& I = insts[z];
-        if (I.Nc == 0) continue;
-        rows_fwd_body<R, N, kSum, true, kTwLds>(U + I.uoff, Uf + I.uoff, N, B, cols + I.cols_off,
-                                                I.Nc, G + I.g_off, tw, I.fz, blockIdx.x, 0);
+        if (I.Nc == 0 || (int)blockIdx.x * B >= I.nin) continue;
+        rows_fwd_body<R, N, kSum, true, kTwLds>(L, U + I.uoff, Uf + I.uoff, I.nin, I.nin, L.n(), B,
+                                                cols + I.cols_off, I.Nc, G + I.g_off, tw, I.fz,
+                                                blockIdx.x, 0);
         __syncthreads();   // the block's LDS is reused by its next instance
     }
 }
 
 template <class R, int M>
 __global__ __launch_bounds__(kThreads) void cols_band_batch_kernel(
-    const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
+    Len<M> L, const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
     typename C2<R>::T* __restrict__ G, const typename C2<R>::T* __restrict__ tw) {
     for (int z = blockIdx.z; z < n; z += gridDim.z) {
         const DetInst& I = insts[z];
         if ((int)blockIdx.x * B >= I.Nc) continue;
-        cols_band_body<R, M>(G + I.g_off, I.Nc, B, cols + I.cols_off, I.bp, tw, blockIdx.x,
-                             blockIdx.y);
+        cols_band_body<R, M>(L, G + I.g_off, I.nin, I.off, I.Nd, I.Nc, B, cols + I.cols_off, I.bp,
+                             tw, blockIdx.x, blockIdx.y);
         __syncthreads();
     }
 }
 
 template <class R, int N, bool kTwLds>
 __global__ __launch_bounds__(kThreads) void rows_inv_detect_batch_kernel(
-    const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
+    Len<N> L, const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
     const typename C2<R>::T* __restrict__ G, R* __restrict__ D, R* __restrict__ Di,
     R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
     for (int z = blockIdx.z; z < n; z += gridDim.z) {
         const DetInst& I = insts[z];
         if ((int)blockIdx.x * B >= I.Nd) continue;
-        rows_inv_detect_body<R, N, false, kTwLds>(G + I.g_off, I.Nc, N, cols + I.cols_off, I.off,
-                                                  I.Nd, B, I.off, I.Nd, D + I.image_off,
-                                                  Di + I.image_off,
-                                                  Abs ? Abs + I.image_off : nullptr, tw, blockIdx.x);
+        rows_inv_detect_body<R, N, false, kTwLds>(
+            L, G + I.g_off, I.Nc, L.n(), cols + I.cols_off, I.off, I.Nd, B, I.off, I.Nd,
+            D + I.image_off, Di + I.image_off, Abs ? Abs + I.image_off : nullptr, tw, blockIdx.x);
         __syncthreads();
     }
 }
@@ -755,85 +825,53 @@ bool fixed_size(int n) {
     }
 }
 
-// The band-limited LDS FFT path: both sizes tabled and a row pair in LDS.
-bool band_path(const bimsim_ctx* ctx, size_t csize, int uR, int vR) {
-    return fixed_size(uR) && fixed_size(vR) && csize * 2 * (size_t)std::max(uR, vR) <= ctx->lds_max;
+// The stage plan of a length without a fixed one; false unless it is a
+// product of 2, 3 and 5.
+bool rt_plan(int n, RtPlan* p) {
+    FftPlan f;
+    if (make_plan(n, &f) != 0 || f.nstages > kRtStages) return false;
+    *p = RtPlan{};
+    p->n = n;
+    p->nst = f.nstages;
+    p->mn = rt_magic(n);
+    int Ns = 1;
+    for (int st = 0; st < f.nstages; ++st) {
+        p->rad[st] = f.radix[st];
+        p->mq[st] = rt_magic(n / f.radix[st]);
+        p->ms[st] = rt_magic(Ns);
+        Ns *= f.radix[st];
+    }
+    return true;
 }
 
-template <class R>
-int launch_rows_fwd(bimsim_ctx* ctx, int N, dim3 grid, size_t lds, const typename C2<R>::T* U,
-                    const typename C2<R>::T* Uf, int nrows, int B, const int* cols, int Nc,
-                    typename C2<R>::T* G, const typename C2<R>::T* tw, const SumFuse* fz) {
-    // the summing form exists for complex64 fields (the FP32 batches) only
-    constexpr bool f32 = std::is_same<R, float>::value;
-    if (fz && !f32) return set_error(ctx, BIMSIM_E_UNSUPPORTED, "fused sum needs complex64 fields");
-    switch (N) {
-#define BIMSIM_X(NN)                                                                          \
-    case NN:                                                                                  \
-        if (f32 && fz)                                                                        \
-            hipLaunchKernelGGL((rows_fwd_kernel<R, NN, f32>), grid, dim3(kThreads), lds,      \
-                               ctx->stream, U, Uf, nrows, B, cols, Nc, G, tw, *fz);           \
-        else                                                                                  \
-            hipLaunchKernelGGL((rows_fwd_kernel<R, NN, false>), grid, dim3(kThreads), lds,    \
-                               ctx->stream, U, Uf, nrows, B, cols, Nc, G, tw, SumFuse{});     \
-        break;
-        BIMSIM_FFT_SIZES(BIMSIM_X)
-#undef BIMSIM_X
-    }
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return BIMSIM_OK;
+// The band-limited LDS FFT path: both sizes products of 2, 3 and 5 and a
+// line's two buffers in LDS.  With fixed: both sizes of the compiled list.
+bool band_path(const bimsim_ctx* ctx, size_t csize, int uR, int vR, bool fixed = false) {
+    RtPlan p;
+    const bool ok = fixed ? fixed_size(uR) && fixed_size(vR) : rt_plan(uR, &p) && rt_plan(vR, &p);
+    return ok && csize * 2 * (size_t)std::max(uR, vR) <= ctx->lds_max;
 }
 
-template <class R>
-int launch_cols_band(bimsim_ctx* ctx, int M, dim3 grid, size_t lds, typename C2<R>::T* G, int Nc,
-                     int B, const int* cols, const PostOp& bp, const typename C2<R>::T* tw) {
-    switch (M) {
-#define BIMSIM_X(NN)                                                                            \
-    case NN:                                                                                    \
-        hipLaunchKernelGGL((cols_band_kernel<R, NN>), grid, dim3(kThreads), lds, ctx->stream, G, \
-                           Nc, B, cols, bp, tw);                                                \
-        break;
+// Calls f with the length as a kernel takes it: Len<n> of a compiled length,
+// else Len<0> with its stage plan.
+template <class F>
+void with_len(int n, F&& f) {
+    switch (n) {
+#define BIMSIM_X(NN)    \
+    case NN:            \
+        f(Len<NN>{});   \
+        return;
         BIMSIM_FFT_SIZES(BIMSIM_X)
 #undef BIMSIM_X
+        default: {
+            Len<0> L;
+            if (rt_plan(n, &L.p)) f(L);
+        }
     }
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return BIMSIM_OK;
 }
-
-template <class R>
-int launch_rows_inv(bimsim_ctx* ctx, int N, dim3 grid, size_t lds, const typename C2<R>::T* G,
-                    int Nc, int vR, const int* cols, int row_begin, int nrows, int B, R* I,
-                    typename C2<R>::T* Uw, typename C2<R>::T* Ufw, const typename C2<R>::T* tw) {
-    switch (N) {
-#define BIMSIM_X(NN)                                                                            \
-    case NN:                                                                                    \
-        hipLaunchKernelGGL((rows_inv_kernel<R, NN>), grid, dim3(kThreads), lds, ctx->stream, G, \
-                           Nc, vR, cols, row_begin, nrows, B, I, Uw, Ufw, tw);                  \
-        break;
-        BIMSIM_FFT_SIZES(BIMSIM_X)
-#undef BIMSIM_X
-    }
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return BIMSIM_OK;
-}
-
-template <class R>
-int launch_rows_inv_detect(bimsim_ctx* ctx, int N, dim3 grid, size_t lds,
-                           const typename C2<R>::T* G, int Nc, int vR, const int* cols,
-                           int row_begin, int nrows, int B, int off, int Nd, R* D, R* Di, R* Abs,
-                           const typename C2<R>::T* tw) {
-    switch (N) {
-#define BIMSIM_X(NN)                                                                       \
-    case NN:                                                                               \
-        hipLaunchKernelGGL((rows_inv_detect_kernel<R, NN>), grid, dim3(kThreads), lds,     \
-                           ctx->stream, G, Nc, vR, cols, row_begin, nrows, B, off, Nd, D, \
-                           Di, Abs, tw);                                                   \
-        break;
-        BIMSIM_FFT_SIZES(BIMSIM_X)
-#undef BIMSIM_X
-    }
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return BIMSIM_OK;
+template <int N>
+constexpr int len_of(const Len<N>&) {
+    return N;
 }
 
 // Pass-band columns (|f_u| <= NAout/lambda with the band-pass's own index
@@ -858,16 +896,22 @@ std::vector<int> band_column_list(const PostOp& bp, int uR) {
     return cols;
 }
 
-// Band-limited detector for FFT lengths with a fixed plan, on the given
-// work buffers: the pass-band column list colsd (Nc entries), the compact
-// spectrum G (2 Nc vR complex) and, unless the inverse row pass detects
-// on its own rows, the intensity rows I (2 nrows uR real).
+// Band-limited detector on the given work buffers: the pass-band column list
+// colsd (Nc entries), the compact spectrum G (2 Nc vR complex) and, unless
+// the inverse row pass detects on its own rows, the intensity rows I
+// (2 nrows uR real).  The fields are nin x nin_v (uR x vR, or less: zero
+// filled to that size).
 template <class R>
 int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int uR, int vR,
-                  int padding, int Nd, int ss, void* D, void* Di, void* Abs, int write_filtered,
-                  const typename C2<R>::T* tw_u, const typename C2<R>::T* tw_v,
-                  const SumFuse* fz, const int* colsd, int Nc, void* G, void* I) {
+                  int nin, int nin_v, int padding, int Nd, int ss, void* D, void* Di, void* Abs,
+                  int write_filtered, const typename C2<R>::T* tw_u,
+                  const typename C2<R>::T* tw_v, const SumFuse* fz, const int* colsd, int Nc,
+                  void* G, void* I) {
     using C = typename C2<R>::T;
+    constexpr bool f32 = std::is_same<R, float>::value;
+    // the summing form exists for complex64 fields (the FP32 batches) only
+    if (fz && !f32) return set_error(ctx, BIMSIM_E_UNSUPPORTED, "fused sum needs complex64 fields");
+    const hipStream_t st = ctx->stream;
     const int S = Nd * ss, off = padding * S;
     const int row_begin = write_filtered ? 0 : off;
     const int nrows = write_filtered ? vR : S;
@@ -879,50 +923,74 @@ int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int 
         return b;
     };
     if (Nc > 0) {
-        int B = rows_per_group(vR);
+        int B = rows_per_group(nin_v);
         size_t lds = sizeof(C) * 2 * (size_t)B * uR;
-        BIMSIM_TRY(launch_rows_fwd<R>(ctx, uR, dim3((vR + B - 1) / B, 2), lds, (const C*)Uin,
-                                      (const C*)Ufin, vR, B, colsd, Nc, (C*)G, tw_u, fz));
+        const dim3 grid((nin_v + B - 1) / B, 2);
+        with_len(uR, [&](auto L) {
+            constexpr int N = len_of(decltype(L){});
+            if (f32 && fz)
+                hipLaunchKernelGGL((rows_fwd_kernel<R, N, f32>), grid, dim3(kThreads), lds, st, L,
+                                   (const C*)Uin, (const C*)Ufin, nin, nin_v, vR, B, colsd, Nc,
+                                   (C*)G, tw_u, *fz);
+            else
+                hipLaunchKernelGGL((rows_fwd_kernel<R, N, false>), grid, dim3(kThreads), lds, st,
+                                   L, (const C*)Uin, (const C*)Ufin, nin, nin_v, vR, B, colsd, Nc,
+                                   (C*)G, tw_u, SumFuse{});
+        });
+        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
         int Bc = std::max(1, std::min(8, 2048 / vR));
         Bc = std::min(Bc, Nc);
         // a narrow pass band leaves few columns: fewer per workgroup, so
         // that the column pass still spreads over the chip
         while (Bc > 1 && (Nc + Bc - 1) / Bc < 128) Bc /= 2;
         lds = sizeof(C) * 2 * (size_t)Bc * vR;
-        BIMSIM_TRY(launch_cols_band<R>(ctx, vR, dim3((Nc + Bc - 1) / Bc, 2), lds, (C*)G, Nc, Bc,
-                                       colsd, bp, tw_v));
+        with_len(vR, [&](auto L) {
+            hipLaunchKernelGGL((cols_band_kernel<R, len_of(decltype(L){})>),
+                               dim3((Nc + Bc - 1) / Bc, 2), dim3(kThreads), lds, st, L, (C*)G,
+                               nin_v, row_begin, nrows, Nc, Bc, colsd, bp, tw_v);
+        });
+        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     }
     int B = rows_per_group(nrows);
     size_t lds = sizeof(C) * 2 * (size_t)B * uR;
     if (Nc > 0 && ss == 1 && !write_filtered && 2 * lds <= ctx->lds_max) {
         // both fields' rows per workgroup, detection on them in the same pass
-        return launch_rows_inv_detect<R>(ctx, uR, dim3((nrows + B - 1) / B), 2 * lds, (const C*)G,
-                                         Nc, vR, colsd, row_begin, nrows, B, off, Nd, (R*)D,
-                                         (R*)Di, (R*)Abs, tw_u);
+        with_len(uR, [&](auto L) {
+            hipLaunchKernelGGL((rows_inv_detect_kernel<R, len_of(decltype(L){})>),
+                               dim3((nrows + B - 1) / B), dim3(kThreads), 2 * lds, st, L,
+                               (const C*)G, Nc, vR, colsd, row_begin, nrows, B, off, Nd, (R*)D,
+                               (R*)Di, (R*)Abs, tw_u);
+        });
+        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
+        return BIMSIM_OK;
     }
     if (Nc > 0) {
-        BIMSIM_TRY(launch_rows_inv<R>(ctx, uR, dim3((nrows + B - 1) / B, 2), lds, (const C*)G, Nc,
-                                      vR, colsd, row_begin, nrows, B, (R*)I,
-                                      write_filtered ? (C*)Uin : nullptr,
-                                      write_filtered ? (C*)Ufin : nullptr, tw_u));
+        with_len(uR, [&](auto L) {
+            hipLaunchKernelGGL((rows_inv_kernel<R, len_of(decltype(L){})>),
+                               dim3((nrows + B - 1) / B, 2), dim3(kThreads), lds, st, L,
+                               (const C*)G, Nc, vR, colsd, row_begin, nrows, B, (R*)I,
+                               write_filtered ? (C*)Uin : nullptr,
+                               write_filtered ? (C*)Ufin : nullptr, tw_u);
+        });
+        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     } else {
         // nothing passes the objective: zero intensities (and fields)
         const size_t ni = 2 * (size_t)nrows * uR;
         hipLaunchKernelGGL(fill_zero<R>, dim3((unsigned)((ni + 255) / 256)), dim3(256), 0,
-                           ctx->stream, (R*)I, ni);
+                           st, (R*)I, ni);
         if (write_filtered) {
             const size_t nf = 2 * (size_t)uR * vR;   // complex values as pairs of R
             hipLaunchKernelGGL(fill_zero<R>, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0,
-                               ctx->stream, (R*)Uin, nf);
+                               st, (R*)Uin, nf);
             hipLaunchKernelGGL(fill_zero<R>, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0,
-                               ctx->stream, (R*)Ufin, nf);
+                               st, (R*)Ufin, nf);
         }
         BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     }
     const R* Ic = (const R*)I + (size_t)(off - row_begin) * uR;
     // detect_from_intensity indexes rows relative to the crop start
     hipLaunchKernelGGL(detect_from_intensity<R>, dim3((Nd * Nd + 255) / 256), dim3(256), 0,
-                       ctx->stream, Ic, nrows, uR, off, Nd, ss, (R*)D, (R*)Di, (R*)Abs);
+                       st, Ic, nrows, uR, off, Nd, ss, (R*)D, (R*)Di, (R*)Abs);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
 }
@@ -952,59 +1020,26 @@ int run_fft_pass(bimsim_ctx* ctx, typename C2<R>::T* data, int nlines, int n, lo
     return BIMSIM_OK;
 }
 
+// The detector of nin x nin_v fields at FFT size uR x vR (the fields' own, or
+// more: zero-filled).
 template <class R>
-int detector_impl(bimsim_ctx* ctx, void* Uin, void* Ufin, int uR, int vR, double du, double dv,
-                  double NAin, double NAout, double lambda, int padding, int Nd, int ss, void* D,
-                  void* Di, void* Abs, int write_filtered, int quirks, const SumFuse* fz) {
+int detector_impl(bimsim_ctx* ctx, void* U, void* Uf, int uR, int vR, int nin, int nin_v,
+                  double du, double dv, double NAin, double NAout, double lambda, int padding,
+                  int Nd, int ss, void* D, void* Di, void* Abs, int write_filtered, int quirks,
+                  const SumFuse* fz) {
     using C = typename C2<R>::T;
-    const size_t npix = (size_t)uR * vR;
-    C* U = (C*)Uin;
-    C* Uf = (C*)Ufin;
-    if (band_path(ctx, sizeof(C), uR, vR)) {
-        const double *twd_u, *twd_v;
-        const float *twf_u, *twf_v;
-        BIMSIM_TRY(twiddles_get(ctx, uR, &twd_u, &twf_u));
-        BIMSIM_TRY(twiddles_get(ctx, vR, &twd_v, &twf_v));
-        PostOp bp{};
-        bp.kind = 1;
-        bp.uR = uR;
-        bp.vR = vR;
-        bp.quirks = quirks;
-        bp.du = du;
-        bp.dv = dv;
-        bp.fmin = NAin / lambda;
-        bp.fmax = NAout / lambda;
-        bp.scale = 1.0 / ((unsigned)uR * (unsigned)vR);   // ScaleField(1.0/(R0*R1))
-        const bool dbl = std::is_same<R, double>::value;
-        const std::vector<int> cols = band_column_list(bp, uR);
-        const int Nc = (int)cols.size();
-        const int nrows = write_filtered ? vR : Nd * ss;
-        const int* colsd = nullptr;
-        void *G = nullptr, *I = nullptr;
-        BIMSIM_TRY(int_table_get(ctx, cols, &colsd));
-        BIMSIM_TRY(scratch_get(ctx, kSlotFftA, sizeof(C) * 2 * (size_t)std::max(Nc, 1) * vR, &G));
-        BIMSIM_TRY(scratch_get(ctx, kSlotFftB, sizeof(R) * 2 * (size_t)nrows * uR, &I));
-        return detector_band<R>(ctx, bp, Uin, Ufin, uR, vR, padding, Nd, ss, D, Di, Abs,
-                                write_filtered, dbl ? (const C*)twd_u : (const C*)twf_u,
-                                dbl ? (const C*)twd_v : (const C*)twf_v, fz, colsd, Nc, G, I);
-    }
-    if (fz) return set_error(ctx, BIMSIM_E_UNSUPPORTED, "fused sum needs the band-limited detector");
-    if (!write_filtered) {
-        void *a = nullptr, *b = nullptr;
-        BIMSIM_TRY(scratch_get(ctx, kSlotFftA, sizeof(C) * npix, &a));
-        BIMSIM_TRY(scratch_get(ctx, kSlotFftB, sizeof(C) * npix, &b));
-        BIMSIM_HIP_CHECK(ctx, hipMemcpyAsync(a, U, sizeof(C) * npix, hipMemcpyDeviceToDevice, ctx->stream));
-        BIMSIM_HIP_CHECK(ctx, hipMemcpyAsync(b, Uf, sizeof(C) * npix, hipMemcpyDeviceToDevice, ctx->stream));
-        U = (C*)a;
-        Uf = (C*)b;
+    for (int n : {uR, vR}) {
+        RtPlan p;
+        if (!rt_plan(n, &p))
+            return set_error(ctx, BIMSIM_E_UNSUPPORTED,
+                             "FFT length %d is not a product of 2, 3 and 5", n);
+        if (sizeof(C) * 2 * (size_t)n > ctx->lds_max)
+            return set_error(ctx, BIMSIM_E_UNSUPPORTED, "FFT length %d does not fit in LDS", n);
     }
     const double *twd_u, *twd_v;
     const float *twf_u, *twf_v;
     BIMSIM_TRY(twiddles_get(ctx, uR, &twd_u, &twf_u));
     BIMSIM_TRY(twiddles_get(ctx, vR, &twd_v, &twf_v));
-    const C* tw_u = std::is_same<R, double>::value ? (const C*)twd_u : (const C*)twf_u;
-    const C* tw_v = std::is_same<R, double>::value ? (const C*)twd_v : (const C*)twf_v;
-    PostOp none{};
     PostOp bp{};
     bp.kind = 1;
     bp.uR = uR;
@@ -1014,62 +1049,32 @@ int detector_impl(bimsim_ctx* ctx, void* Uin, void* Ufin, int uR, int vR, double
     bp.dv = dv;
     bp.fmin = NAin / lambda;
     bp.fmax = NAout / lambda;
-    PostOp sc{};
-    sc.kind = 2;
-    sc.scale = 1.0 / ((unsigned)uR * (unsigned)vR);   // ScaleField(1.0/(R0*R1))
-    C* fields[2] = {U, Uf};
-    for (C* F : fields) {
-        // forward: rows (length uR), then columns (length vR) + band-pass
-        BIMSIM_TRY(run_fft_pass<R>(ctx, F, vR, uR, uR, 1, tw_u, 0, none));
-        BIMSIM_TRY(run_fft_pass<R>(ctx, F, uR, vR, 1, uR, tw_v, 0, bp));
-        // inverse: columns, then rows + 1/(uR vR)
-        BIMSIM_TRY(run_fft_pass<R>(ctx, F, uR, vR, 1, uR, tw_v, 1, none));
-        BIMSIM_TRY(run_fft_pass<R>(ctx, F, vR, uR, uR, 1, tw_u, 1, sc));
-    }
-    const int off = padding * Nd * ss;
-    hipLaunchKernelGGL(detect_kernel<R>, dim3((Nd * Nd + 255) / 256), dim3(256), 0, ctx->stream,
-                       (const C*)U, (const C*)Uf, uR, off, Nd, ss, (R*)D, (R*)Di, (R*)Abs);
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return BIMSIM_OK;
+    bp.scale = 1.0 / ((unsigned)uR * (unsigned)vR);   // ScaleField(1.0/(R0*R1))
+    const bool dbl = std::is_same<R, double>::value;
+    const std::vector<int> cols = band_column_list(bp, uR);
+    const int Nc = (int)cols.size();
+    const int nrows = write_filtered ? vR : Nd * ss;
+    const int* colsd = nullptr;
+    void *G = nullptr, *I = nullptr;
+    BIMSIM_TRY(int_table_get(ctx, cols, &colsd));
+    BIMSIM_TRY(scratch_get(ctx, kSlotFftA, sizeof(C) * 2 * (size_t)std::max(Nc, 1) * vR, &G));
+    BIMSIM_TRY(scratch_get(ctx, kSlotFftB, sizeof(R) * 2 * (size_t)nrows * uR, &I));
+    return detector_band<R>(ctx, bp, U, Uf, uR, vR, nin, nin_v, padding, Nd, ss, D, Di, Abs,
+                            write_filtered, dbl ? (const C*)twd_u : (const C*)twf_u,
+                            dbl ? (const C*)twd_v : (const C*)twf_v, fz, colsd, Nc, G, I);
 }
 
-// dst (M x Mv) = src (uR x vR) at the corner, zeros elsewhere.
-template <class C>
-__global__ void embed_kernel(const C* __restrict__ src, int uR, int vR, C* __restrict__ dst, int M,
-                             int Mv) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)M * Mv) return;
-    const int iv = (int)(i / M), iu = (int)(i - (long long)iv * M);
-    C v;
-    v.x = 0;
-    v.y = 0;
-    if (iu < uR && iv < vR) v = src[(long long)iv * uR + iu];
-    dst[i] = v;
-}
-
-// The detector on the near field zero-filled to (fill uR) x (fill vR): both
-// fields embedded at the corner of scratch arrays, the FFT and band-pass on
-// the finer frequency grid (du/fill, dv/fill), the crop of the field's own
-// uR x uR samples at the corner.
+// The detector on the near field zero-filled to (fill uR) x (fill vR): the
+// fields at the corner of zero arrays (the zeros enter in the LDS lines, no
+// filled copy), the FFT and band-pass on the finer frequency grid (du/fill,
+// dv/fill), the crop of the field's own uR x uR samples at the corner.
 template <class R>
 int detector_zero_filled_impl(bimsim_ctx* ctx, const void* U, const void* Uf, int uR, int vR,
                               int fill, double du, double dv, double NAin, double NAout,
                               double lambda, void* D, void* Di, void* Abs, int quirks) {
-    using C = typename C2<R>::T;
-    const int M = fill * uR, Mv = fill * vR;
-    const size_t n = (size_t)M * Mv;
-    void *a = nullptr, *b = nullptr;
-    BIMSIM_TRY(scratch_get(ctx, kSlotDet, sizeof(C) * 2 * n, &a));
-    b = (char*)a + sizeof(C) * n;
-    const dim3 grid((unsigned)((n + 255) / 256));
-    hipLaunchKernelGGL(embed_kernel<C>, grid, dim3(256), 0, ctx->stream, (const C*)U, uR, vR, (C*)a,
-                       M, Mv);
-    hipLaunchKernelGGL(embed_kernel<C>, grid, dim3(256), 0, ctx->stream, (const C*)Uf, uR, vR,
-                       (C*)b, M, Mv);
-    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    // the embedded copies are ours: the transform may run in place on them
-    return detector_impl<R>(ctx, a, b, M, Mv, du / fill, dv / fill, NAin, NAout, lambda, 0, uR, 1,
-                            D, Di, Abs, 1, quirks, nullptr);
+    return detector_impl<R>(ctx, const_cast<void*>(U), const_cast<void*>(Uf), fill * uR, fill * vR,
+                            uR, vR, du / fill, dv / fill, NAin, NAout, lambda, 0, uR, 1, D, Di,
+                            Abs, 0, quirks, nullptr);
 }
 
 // fieldslice::toAngularSpectrum / fromAngularSpectrum (fieldslice.cpp:
@@ -1136,10 +1141,10 @@ int detector_run(bimsim_ctx* ctx, int prec, int quirks, void* U, void* Uf, int u
     const int tmr = timer_begin(ctx, kStageDet);
     int rc;
     if (prec == BIMSIM_FP32_FAST)
-        rc = detector_impl<float>(ctx, U, Uf, uR, vR, du, dv, NAin, NAout, lambda, padding, Nd, ss,
+        rc = detector_impl<float>(ctx, U, Uf, uR, vR, uR, vR, du, dv, NAin, NAout, lambda, padding, Nd, ss,
                                   D, Di, Abs, write_filtered, quirks, fz);
     else
-        rc = detector_impl<double>(ctx, U, Uf, uR, vR, du, dv, NAin, NAout, lambda, padding, Nd,
+        rc = detector_impl<double>(ctx, U, Uf, uR, vR, uR, vR, du, dv, NAin, NAout, lambda, padding, Nd,
                                    ss, D, Di, Abs, write_filtered, quirks, fz);
     if (rc != BIMSIM_OK) return rc;
     timer_end(ctx, tmr);
@@ -1168,36 +1173,29 @@ int det_batch_launch_impl(bimsim_ctx* ctx, const DetBatch& b, const void* U, con
     const hipStream_t st = ctx->stream;
     constexpr bool f32 = std::is_same<R, float>::value;
     const bool sum = f32 && b.fused;
-    const dim3 grid_r((N + b.B - 1) / b.B, 1, nz), grid_i((b.max_nd + b.B2 - 1) / b.B2, 1, nz);
-    switch (N) {
-#define BIMSIM_FWD(NN, S, T)                                                                       \
-    hipLaunchKernelGGL((rows_fwd_batch_kernel<R, NN, S, T>), grid_r, dim3(kThreads),               \
-                       lds_r + (T ? lds_tw : 0), st, I, b.n, (const C*)U, (const C*)Uf, b.B,       \
-                       b.d_cols, (C*)b.d_G, tw)
-#define BIMSIM_INV(NN, T)                                                                          \
-    hipLaunchKernelGGL((rows_inv_detect_batch_kernel<R, NN, T>), grid_i, dim3(kThreads),           \
-                       lds_i + (T ? lds_tw : 0), st, I, b.n, b.B2, b.d_cols, (const C*)b.d_G,      \
-                       (R*)D, (R*)Di, (R*)Abs, tw)
-#define BIMSIM_X(NN)                                                                               \
-    case NN:                                                                                       \
-        if (sum && tw_r) BIMSIM_FWD(NN, f32, true);                                                \
-        else if (sum) BIMSIM_FWD(NN, f32, false);                                                  \
-        else if (tw_r) BIMSIM_FWD(NN, false, true);                                                \
-        else BIMSIM_FWD(NN, false, false);                                                         \
-        if (b.max_nc > 0)                                                                          \
-            hipLaunchKernelGGL((cols_band_batch_kernel<R, NN>),                                    \
-                               dim3((b.max_nc + b.Bc - 1) / b.Bc, 2, nz), dim3(kThreads), lds_c,   \
-                               st, I, b.n, b.Bc, b.d_cols, (C*)b.d_G, tw);                        \
-        if (tw_i) BIMSIM_INV(NN, true);                                                            \
-        else BIMSIM_INV(NN, false);                                                                \
-        break;
-        BIMSIM_FFT_SIZES(BIMSIM_X)
-#undef BIMSIM_X
-#undef BIMSIM_INV
-#undef BIMSIM_FWD
-        default:
-            return set_error(ctx, BIMSIM_E_UNSUPPORTED, "no batched detector for N = %d", N);
-    }
+    const dim3 grid_r((b.max_nin + b.B - 1) / b.B, 1, nz);
+    const dim3 grid_i((b.max_nd + b.B2 - 1) / b.B2, 1, nz);
+    with_len(N, [&](auto L) {
+        constexpr int NN = len_of(decltype(L){});
+        auto fwd = [&](auto kernel, size_t lds) {
+            hipLaunchKernelGGL(kernel, grid_r, dim3(kThreads), lds, st, L, I, b.n, (const C*)U,
+                               (const C*)Uf, b.B, b.d_cols, (C*)b.d_G, tw);
+        };
+        auto inv = [&](auto kernel, size_t lds) {
+            hipLaunchKernelGGL(kernel, grid_i, dim3(kThreads), lds, st, L, I, b.n, b.B2, b.d_cols,
+                               (const C*)b.d_G, (R*)D, (R*)Di, (R*)Abs, tw);
+        };
+        if (sum && tw_r) fwd(rows_fwd_batch_kernel<R, NN, f32, true>, lds_r + lds_tw);
+        else if (sum) fwd(rows_fwd_batch_kernel<R, NN, f32, false>, lds_r);
+        else if (tw_r) fwd(rows_fwd_batch_kernel<R, NN, false, true>, lds_r + lds_tw);
+        else fwd(rows_fwd_batch_kernel<R, NN, false, false>, lds_r);
+        if (b.max_nc > 0)
+            hipLaunchKernelGGL((cols_band_batch_kernel<R, NN>),
+                               dim3((b.max_nc + b.Bc - 1) / b.Bc, 2, nz), dim3(kThreads), lds_c,
+                               st, L, I, b.n, b.Bc, b.d_cols, (C*)b.d_G, tw);
+        if (tw_i) inv(rows_inv_detect_batch_kernel<R, NN, true>, lds_i + lds_tw);
+        else inv(rows_inv_detect_batch_kernel<R, NN, false>, lds_i);
+    });
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
 }
@@ -1206,8 +1204,10 @@ int det_batch_launch_impl(bimsim_ctx* ctx, const DetBatch& b, const void* U, con
 
 bool det_batchable(const bimsim_ctx* ctx, int prec, int N, int ss, int zero_fill) {
     const size_t cs = prec == BIMSIM_FP32_FAST ? sizeof(float2) : sizeof(double2);
-    return ss == 1 && zero_fill <= 1 && band_path(ctx, cs, N, N) &&
-           2 * cs * 2 * (size_t)rows_per_wg(N) * N <= ctx->lds_max;
+    if (N < 1 || N > (1 << 14) || zero_fill > 8) return false;
+    const int M = N * std::max(1, zero_fill);
+    return ss == 1 && band_path(ctx, cs, M, M) &&
+           2 * cs * 2 * (size_t)rows_per_wg(M) * M <= ctx->lds_max;
 }
 
 int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::vector<DetParams>& p,
@@ -1218,14 +1218,15 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
     std::vector<DetInst> insts;
     std::vector<int> cols;
     long long g = 0;
-    int max_nc = 0, max_nd = 0;
+    int max_nc = 0, max_nd = 0, max_nin = 0;
     for (const DetParams& q : p) {
         DetInst I{};
         I.uoff = q.uoff;
         I.image_off = q.image_off;
         I.Nd = q.Nd;
         I.off = q.padding * q.Nd;
-        BIMSIM_CHECK_ARG(ctx, I.off + q.Nd <= N, "detector crop exceeds the near-field grid");
+        I.nin = q.nin;
+        BIMSIM_CHECK_ARG(ctx, I.off + q.Nd <= q.nin && q.nin <= N, "detector crop exceeds the near-field grid");
         PostOp& bp = I.bp;
         bp.kind = 1;
         bp.uR = N;
@@ -1246,6 +1247,7 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
         g += 2LL * I.Nc * N;
         max_nc = std::max(max_nc, I.Nc);
         max_nd = std::max(max_nd, I.Nd);
+        max_nin = std::max(max_nin, I.nin);
         insts.push_back(I);
     }
     out->N = N;
@@ -1254,11 +1256,12 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
     out->fused = fused && f32;
     out->max_nc = max_nc;
     out->max_nd = max_nd;
+    out->max_nin = max_nin;
     // rows (columns) per workgroup, fewer when the batch is small so that
     // each pass still spreads over the chip
     const int n = (int)insts.size();
     int B = rows_per_wg(N), B2 = B, Bc = std::max(1, std::min(8, 2048 / N));
-    while (B > 1 && (long long)n * ((N + B - 1) / B) < 512) B /= 2;
+    while (B > 1 && (long long)n * ((max_nin + B - 1) / B) < 512) B /= 2;
     while (B2 > 1 && (long long)n * ((max_nd + B2 - 1) / B2) < 512) B2 /= 2;
     while (Bc > 1 && (long long)n * ((max_nc + Bc - 1) / Bc) < 128) Bc /= 2;
     out->B = B;
@@ -1380,8 +1383,8 @@ int detector_noalloc_impl(bimsim_ctx* ctx, unsigned char* work, int quirks, cons
         hipLaunchKernelGGL(band_cols_kernel, dim3((Nc + 255) / 256), dim3(256), 0, ctx->stream,
                            cols, n1, n2, uR);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    return detector_band<R>(ctx, bp, const_cast<void*>(U), const_cast<void*>(Uf), uR, vR, padding,
-                            Nd, ss, D, Di, Abs, 0, tu, tv, nullptr, cols, Nc, work + o_G,
+    return detector_band<R>(ctx, bp, const_cast<void*>(U), const_cast<void*>(Uf), uR, vR, uR, vR,
+                            padding, Nd, ss, D, Di, Abs, 0, tu, tv, nullptr, cols, Nc, work + o_G,
                             work + o_I);
 }
 
@@ -1417,7 +1420,7 @@ extern "C" int bimsim_detector_noalloc(bimsim_ctx* ctx, int prec, int quirks, co
     BIMSIM_CHECK_ARG(ctx, lambda > 0.0 && du > 0.0 && dv > 0.0, "lambda, du and dv must be positive");
     BIMSIM_CHECK_ARG(ctx, prec >= BIMSIM_FP64_PARITY && prec <= BIMSIM_FP32_FAST, "unknown precision");
     const bool f32 = prec == BIMSIM_FP32_FAST;
-    if (!band_path(ctx, f32 ? sizeof(float2) : sizeof(double2), uR, vR))
+    if (!band_path(ctx, f32 ? sizeof(float2) : sizeof(double2), uR, vR, true))
         return set_error(ctx, BIMSIM_E_UNSUPPORTED,
                          "the allocation-free detector takes FFT sizes of 64..4096 from "
                          "{2^k, 3 2^k} whose rows fit LDS (got %d x %d)",
