@@ -109,9 +109,14 @@ struct SumInst {
 };
 
 // Mie coefficients of n spheres, sphere i at wavenumber kmag[i]; writes
-// A/B at each sphere's coeff_off.  work: n * 8 * (lmax + 2) complex doubles.
+// A/B at each sphere's coeff_off.  closed: all n are mie_closed_spheres.
+// work: n * 8 * (lmax + 2) complex doubles (unless closed).
 int mie_batch_launch(bimsim_ctx* ctx, const SphereDev* d_sph, const double* d_kmag, int n,
-                     int lmax, int quirks, void* work, double2* A, double2* B);
+                     int lmax, int quirks, bool closed, void* work, double2* A, double2* B);
+
+// Whether the closed form of the coefficients takes all n spheres (host
+// tables) in one launch.
+bool mie_closed_spheres(const bimsim_ctx* ctx, const SphereDev* sph, const double* kmag, int n);
 
 // Pixel-invariant table of the incident-field series for the complex64
 // form: for l = 0..m the four values (i^l sign) * D_l, (2l-1)/l, (l-1)/l
@@ -191,10 +196,11 @@ struct DetParams {
 struct DetBatch {
     int N = 0, n = 0, B = 0, B2 = 0, Bc = 0, max_nc = 0, max_nd = 0, max_nin = 0;
     bool f32 = false, fused = false;
+    bool wide = false;       // FP32 images, FP64 from the pass-band columns on
     void* d_inst = nullptr;
     int* d_cols = nullptr;
-    void* d_G = nullptr;
-    const void* tw = nullptr;
+    void *d_G = nullptr, *d_H = nullptr;   // pass-band columns, and filtered (one, or complex128)
+    const void *tw = nullptr, *tw2 = nullptr;   // twiddles of the forward rows, and past them
 };
 bool det_batchable(const bimsim_ctx* ctx, int prec, int N, int ss, int zero_fill);
 int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::vector<DetParams>& p,

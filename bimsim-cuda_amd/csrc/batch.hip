@@ -8,9 +8,9 @@
 //                      tables and records, joined before the scattered
 //                      fields (beside those persistent launches the fields
 //                      ran starved of CUs, and slowed them)
-//   FP32 pre-pass      with one harmonic plan and few spheres instead: the
-//                      Legendre tables, then coefficients, records and
-//                      incident fields in one launch (series_plan_launch_prepass);
+//   FP32 pre-pass      with one harmonic plan of few rows instead: the
+//                      coefficients, wave tables and incident fields in one
+//                      launch (series_plan_launch_prepass);
 //                      with band-limited detectors the sum is then formed by
 //                      their first row pass and the images cleared here
 //   scattered fields   FP32: coefficient kernel + one persistent work-queue
@@ -50,6 +50,7 @@ struct bimsim_batch {
     SphereDev* d_sph = nullptr;
     double* d_kmag = nullptr;
     void* d_work = nullptr;
+    bool mie_closed = false;    // the coefficients' closed form takes every sphere
     double2 *d_A = nullptr, *d_B = nullptr;
     UfInst* d_uf = nullptr;
     double* d_uftab = nullptr;      // incident-field tables of complex64 batches
@@ -72,9 +73,9 @@ struct bimsim_batch {
     // before the sums)
     hipStream_t side = nullptr, side_f = nullptr;
     hipEvent_t ev_fork = nullptr, ev_coef = nullptr, ev_fields = nullptr;
-    // FP32 passes of one harmonic plan whose coefficient blocks fit
-    // kPrepassLds: coefficients, records and incident fields in one launch
-    // on the one stream instead
+    // FP32 passes of one harmonic plan with few rows (series_few_rows), whose
+    // launches would not fill the chip: coefficients, wave tables and incident
+    // fields in one launch on the one stream instead
     bool prepass = false;
     PrepassArgs pre{};
     // and with every detector on the band-limited path, the Uf + Us sum
@@ -138,7 +139,7 @@ void release(bimsim_batch* b) {
 int enqueue_fp64_fields(bimsim_batch* b) {
     bimsim_ctx* ctx = b->ctx;
     const size_t fb = sizeof(double2);
-    BIMSIM_TRY(mie_batch_launch(ctx, b->d_sph, b->d_kmag, b->n_sph, b->lmax, b->quirks, b->d_work,
+    BIMSIM_TRY(mie_batch_launch(ctx, b->d_sph, b->d_kmag, b->n_sph, b->lmax, b->quirks, b->mie_closed, b->d_work,
                                 b->d_A, b->d_B));
     BIMSIM_TRY(uf_batch_launch(ctx, b->d_uf, b->n, b->uf_items, b->f32, b->d_uftab, b->waves,
                                b->d_Uf));
@@ -193,7 +194,7 @@ int enqueue(bimsim_batch* b) {
         const hipStream_t main = ctx->stream;
         ctx->stream = b->side;
         int rc = mie_batch_launch(ctx, b->d_sph, b->d_kmag, b->n_sph, b->lmax, b->quirks,
-                                  b->d_work, b->d_A, b->d_B);
+                                  b->mie_closed, b->d_work, b->d_A, b->d_B);
         if (rc == BIMSIM_OK && hipEventRecord(b->ev_coef, b->side) != hipSuccess)
             rc = set_error(ctx, BIMSIM_E_HIP, "hipEventRecord failed");
         ctx->stream = b->side_f;
@@ -426,7 +427,9 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     BIMSIM_TRY(dev_upload(ctx, &b->d_kdirs, kdirs));
     BIMSIM_TRY(dev_upload(ctx, &b->d_mc_list, mc_list));
     b->n_mc_uf = (int)mc_list.size();
-    BIMSIM_TRY(dev_alloc(ctx, &b->d_work, sizeof(double2) * 8 * (size_t)(b->lmax + 2) * std::max(1, b->n_sph)));
+    b->mie_closed = mie_closed_spheres(ctx, sph_dev.data(), sph_k.data(), b->n_sph);
+    if (!b->mie_closed)
+        BIMSIM_TRY(dev_alloc(ctx, &b->d_work, sizeof(double2) * 8 * (size_t)(b->lmax + 2) * std::max(1, b->n_sph)));
     BIMSIM_TRY(dev_alloc(ctx, (void**)&b->d_A, sizeof(double2) * (size_t)std::max<long long>(1, coef)));
     BIMSIM_TRY(dev_alloc(ctx, (void**)&b->d_B, sizeof(double2) * (size_t)std::max<long long>(1, coef)));
     BIMSIM_TRY(dev_alloc(ctx, &b->d_Uf, fb * (size_t)field));
@@ -441,7 +444,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         // the series plans are timed on real inputs: coefficients first
         const size_t budget = (size_t)8 << 30;
         BIMSIM_TRY(mie_batch_launch(ctx, b->d_sph, b->d_kmag, b->n_sph, b->lmax, b->quirks,
-                                    b->d_work, b->d_A, b->d_B));
+                                    b->mie_closed, b->d_work, b->d_A, b->d_B));
         if (!mc.inst.empty()) {
             BIMSIM_TRY(series_plan_create_tuned(ctx, mc, budget, b->waves, b->d_A, b->d_B, &b->plan_mc));
             b->have_mc = true;
@@ -451,12 +454,12 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
             b->have_pw = true;
         }
         const int wstride = b->lmax + 2;
-        b->pre = PrepassArgs{b->d_sph, b->d_kmag, b->n_sph, mie::mie_spheres_per_block(wstride),
-                             wstride, b->quirks, b->d_A, b->d_B, b->d_uf, b->n,
-                             (b->uf_items + 255) / 256, b->d_uftab, b->waves, (float2*)b->d_Uf};
+        b->pre = PrepassArgs{b->d_sph, b->d_kmag, b->n_sph, wstride, b->quirks, b->d_A, b->d_B, b->d_uf, b->n,
+                             (b->uf_items + 255) / 256, b->d_uftab, b->waves, (float2*)b->d_Uf,
+                             nullptr, nullptr, nullptr};
         const SeriesPlan& P = b->have_mc ? b->plan_mc : b->plan_pw;
-        b->prepass = b->have_mc != b->have_pw && P.harmonic && b->n_sph > 0 &&
-                     prepass_lds(b->pre) <= kPrepassLds;
+        b->prepass = b->have_mc != b->have_pw && P.harmonic && b->n_sph > 0 && b->mie_closed &&
+                     series_few_rows(ctx, P) && prepass_lds(b->pre) <= kPrepassLds;
         // the Uf + Us sum in the detectors' first row pass: the images are
         // then cleared by the pre-pass launch or the incident-field launch
         b->fuse_sum = true;

@@ -9,7 +9,13 @@
 // the inverse rows end in |U|^2, averaged over ss x ss into D and Di
 // (accumulating, like resample_intensity), and -log10(D/Di).
 // FP64 instantiations run in FP64 end to end (-ffp-contract=off for the
-// whole translation unit); FP32 ones in float with FP64-accurate twiddles.
+// whole translation unit).  FP32 ones transform the rows forward in float
+// with FP64-accurate twiddles and, up to the lengths whose lines fit LDS,
+// work in FP64 from the pass-band columns on: the band-pass keeps a small
+// part of the forward pass's rounding (its noise spreads over every
+// frequency), while the inverse transforms' rounding reaches every pixel, and
+// the absorbance of the dark ones with it (its error on a 512 x 512 image
+// 8e-6 with the inverse in float, of which the fields' own 2e-7).
 #include <mutex>
 #include <type_traits>
 
@@ -580,10 +586,11 @@ __global__ __launch_bounds__(kThreads) void rows_fwd_kernel(
 
 // Pass-band columns of the compact spectrum, each: forward FFT along v of
 // its first nin rows (zero past them), objective band-pass, inverse FFT,
-// scale 1/(uR vR), rows [w0, w0 + wn) stored.  In place in G.
-template <class R, int M>
-__device__ __forceinline__ void cols_band_body(const Len<M>& L, typename C2<R>::T* __restrict__ G,
-                                               int nin, int w0, int wn, int Nc, int B,
+// scale 1/(uR vR), rows [w0, w0 + wn) stored in H (which may be G itself).
+// Computed in R, from columns in RI.
+template <class RI, class R, int M>
+__device__ __forceinline__ void cols_band_body(const Len<M>& L, const typename C2<RI>::T* G,
+                                               typename C2<R>::T* H, int nin, int w0, int wn, int Nc, int B,
                                                const int* __restrict__ cols, const PostOp& bp,
                                                const typename C2<R>::T* __restrict__ tw, int blk,
                                                int f) {
@@ -594,13 +601,14 @@ __device__ __forceinline__ void cols_band_body(const Len<M>& L, typename C2<R>::
     C* b = a + (size_t)B * m;
     const int c0 = blk * B;
     const int nb = min(B, Nc - c0);
-    C* line = G + ((size_t)f * Nc + c0) * m;
+    const typename C2<RI>::T* in = G + ((size_t)f * Nc + c0) * m;
+    C* const out = H + ((size_t)f * Nc + c0) * m;
     if (nin == m) {
-        for (int t = threadIdx.x; t < nb * m; t += kThreads) a[t] = line[t];
+        for (int t = threadIdx.x; t < nb * m; t += kThreads) a[t] = cmk<C>(in[t].x, in[t].y);
     } else {
         for (int t = threadIdx.x; t < nb * m; t += kThreads) {
             C v = cmk<C>((R)0, (R)0);
-            if (t - L.div(t) * m < nin) v = line[t];
+            if (t - L.div(t) * m < nin) v = cmk<C>(in[t].x, in[t].y);
             a[t] = v;
         }
     }
@@ -618,26 +626,26 @@ __device__ __forceinline__ void cols_band_body(const Len<M>& L, typename C2<R>::
         const int iv = t - L.div(t) * m - w0;
         if (iv < 0 || iv >= wn) continue;
         const C v = res[t];
-        line[t] = cmk<C>(v.x * sc, v.y * sc);
+        out[t] = cmk<C>(v.x * sc, v.y * sc);
     }
 }
 
-template <class R, int M>
+template <class RI, class R, int M>
 __global__ __launch_bounds__(kThreads) void cols_band_kernel(
-    Len<M> L, typename C2<R>::T* __restrict__ G, int nin, int w0, int wn, int Nc, int B,
+    Len<M> L, const typename C2<RI>::T* G, typename C2<R>::T* H, int nin, int w0, int wn, int Nc, int B,
     const int* __restrict__ cols, PostOp bp, const typename C2<R>::T* __restrict__ tw) {
-    cols_band_body<R, M>(L, G, nin, w0, wn, Nc, B, cols, bp, tw, blockIdx.x, blockIdx.y);
+    cols_band_body<RI, R, M>(L, G, H, nin, w0, wn, Nc, B, cols, bp, tw, blockIdx.x, blockIdx.y);
 }
 
 // Inverse FFT of rows [row_begin, row_begin + nrows) of U/Uf from the compact
 // spectrum (zeros outside the pass band).  Writes |.|^2 (as |.| squared, like
 // resample_intensity) into I[(field*nrows + row - row_begin)*N + iu] and, when
 // Uw/Ufw are given, the band-passed field itself.
-template <class R, int N>
+template <class R, class RO, int N>
 __global__ __launch_bounds__(kThreads) void rows_inv_kernel(
     Len<N> L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
-    int row_begin, int nrows, int B, R* __restrict__ I, typename C2<R>::T* __restrict__ Uw,
-    typename C2<R>::T* __restrict__ Ufw, const typename C2<R>::T* __restrict__ tw) {
+    int row_begin, int nrows, int B, RO* __restrict__ I, typename C2<RO>::T* __restrict__ Uw,
+    typename C2<RO>::T* __restrict__ Ufw, const typename C2<R>::T* __restrict__ tw) {
     using C = typename C2<R>::T;
     const int n = L.n();
     extern __shared__ unsigned char smem_raw[];
@@ -654,12 +662,13 @@ __global__ __launch_bounds__(kThreads) void rows_inv_kernel(
     }
     __syncthreads();
     const C* res = line_fft<R, N>(L, a, b, nb, tw, true);
-    C* W = f ? Ufw : Uw;
+    using CO = typename C2<RO>::T;
+    CO* W = f ? Ufw : Uw;
     for (int t = threadIdx.x; t < nb * n; t += kThreads) {
         const C v = res[t];
-        if (W) W[(size_t)r0 * n + t] = v;
+        if (W) W[(size_t)r0 * n + t] = cmk<CO>((RO)v.x, (RO)v.y);
         const R m = sqrt(v.x * v.x + v.y * v.y);
-        I[((size_t)f * nrows + (r0 - row_begin)) * n + t] = m * m;
+        I[((size_t)f * nrows + (r0 - row_begin)) * n + t] = (RO)(m * m);
     }
 }
 
@@ -671,11 +680,11 @@ __global__ __launch_bounds__(kThreads) void rows_inv_kernel(
 // kAdd false: D = |U|^2 and Di = |Uf|^2 (the same bits as adding to
 // cleared images), for the batches, whose passes then clear nothing.
 // kTwLds: the twiddles read from a copy in LDS, as in rows_fwd_body.
-template <class R, int N, bool kAdd = true, bool kTwLds = false>
+template <class R, class RO, int N, bool kAdd = true, bool kTwLds = false>
 __device__ __forceinline__ void rows_inv_detect_body(
     const Len<N>& L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
-    int row_begin, int nrows, int B, int off, int Nd, R* __restrict__ D, R* __restrict__ Di,
-    R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw, int blk) {
+    int row_begin, int nrows, int B, int off, int Nd, RO* __restrict__ D, RO* __restrict__ Di,
+    RO* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw, int blk) {
     using C = typename C2<R>::T;
     const int n = L.n();
     extern __shared__ unsigned char smem_raw[];
@@ -717,19 +726,19 @@ __device__ __forceinline__ void rows_inv_detect_body(
         const C v = res[g * n + off + iu], w = res[(nb + g) * n + off + iu];
         const R m = sqrt(v.x * v.x + v.y * v.y), mf = sqrt(w.x * w.x + w.y * w.y);
         const size_t i = (size_t)(r0 - row_begin + g) * Nd + iu;
-        const R d = kAdd ? D[i] + m * m : m * m, di = kAdd ? Di[i] + mf * mf : mf * mf;
+        const RO d = (RO)(kAdd ? D[i] + m * m : m * m), di = (RO)(kAdd ? Di[i] + mf * mf : mf * mf);
         D[i] = d;
         Di[i] = di;
         if (Abs) Abs[i] = -log10(d / di);
     }
 }
 
-template <class R, int N>
+template <class R, class RO, int N>
 __global__ __launch_bounds__(kThreads) void rows_inv_detect_kernel(
     Len<N> L, const typename C2<R>::T* __restrict__ G, int Nc, int vR, const int* __restrict__ cols,
-    int row_begin, int nrows, int B, int off, int Nd, R* __restrict__ D, R* __restrict__ Di,
-    R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
-    rows_inv_detect_body<R, N>(L, G, Nc, vR, cols, row_begin, nrows, B, off, Nd, D, Di, Abs, tw,
+    int row_begin, int nrows, int B, int off, int Nd, RO* __restrict__ D, RO* __restrict__ Di,
+    RO* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
+    rows_inv_detect_body<R, RO, N>(L, G, Nc, vR, cols, row_begin, nrows, B, off, Nd, D, Di, Abs, tw,
                                blockIdx.x);
 }
 
@@ -753,28 +762,28 @@ __global__ __launch_bounds__(kThreads) void rows_fwd_batch_kernel(
     }
 }
 
-template <class R, int M>
+template <class RI, class R, int M>
 __global__ __launch_bounds__(kThreads) void cols_band_batch_kernel(
     Len<M> L, const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
-    typename C2<R>::T* __restrict__ G, const typename C2<R>::T* __restrict__ tw) {
+    const typename C2<RI>::T* G, typename C2<R>::T* H, const typename C2<R>::T* __restrict__ tw) {
     for (int z = blockIdx.z; z < n; z += gridDim.z) {
         const DetInst& I = insts[z];
         if ((int)blockIdx.x * B >= I.Nc) continue;
-        cols_band_body<R, M>(L, G + I.g_off, I.nin, I.off, I.Nd, I.Nc, B, cols + I.cols_off, I.bp,
-                             tw, blockIdx.x, blockIdx.y);
+        cols_band_body<RI, R, M>(L, G + I.g_off, H + I.g_off, I.nin, I.off, I.Nd, I.Nc, B,
+                                 cols + I.cols_off, I.bp, tw, blockIdx.x, blockIdx.y);
         __syncthreads();
     }
 }
 
-template <class R, int N, bool kTwLds>
+template <class R, class RO, int N, bool kTwLds>
 __global__ __launch_bounds__(kThreads) void rows_inv_detect_batch_kernel(
     Len<N> L, const DetInst* __restrict__ insts, int n, int B, const int* __restrict__ cols,
-    const typename C2<R>::T* __restrict__ G, R* __restrict__ D, R* __restrict__ Di,
-    R* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
+    const typename C2<R>::T* __restrict__ G, RO* __restrict__ D, RO* __restrict__ Di,
+    RO* __restrict__ Abs, const typename C2<R>::T* __restrict__ tw) {
     for (int z = blockIdx.z; z < n; z += gridDim.z) {
         const DetInst& I = insts[z];
         if ((int)blockIdx.x * B >= I.Nd) continue;
-        rows_inv_detect_body<R, N, false, kTwLds>(
+        rows_inv_detect_body<R, RO, N, false, kTwLds>(
             L, G + I.g_off, I.Nc, L.n(), cols + I.cols_off, I.off, I.Nd, B, I.off, I.Nd,
             D + I.image_off, Di + I.image_off, Abs ? Abs + I.image_off : nullptr, tw, blockIdx.x);
         __syncthreads();
@@ -896,18 +905,34 @@ std::vector<int> band_column_list(const PostOp& bp, int uR) {
     return cols;
 }
 
+// Whether an FP32 detector works in FP64 from its pass-band columns on: both
+// fields' lines of an inverse row pass fit LDS in double.
+bool det_wide(const bimsim_ctx* ctx, int uR, int vR) {
+    return 4 * sizeof(double2) * (size_t)std::max(uR, vR) <= ctx->lds_max;
+}
+
+// f<R>() with the type a detector of fields in RI computes in past its
+// columns.
+template <class RI, class F>
+int with_compute(bool wide, F&& f) {
+    if (std::is_same<RI, double>::value || wide) return f(double());
+    return f(RI());
+}
+
 // Band-limited detector on the given work buffers: the pass-band column list
-// colsd (Nc entries), the compact spectrum G (2 Nc vR complex) and, unless
-// the inverse row pass detects on its own rows, the intensity rows I
+// colsd (Nc entries), the compact spectrum G (2 Nc vR complex), the filtered
+// columns H (as many, complex128 when wide, det_wide, else G itself) and,
+// unless the inverse row pass detects on its own rows, the intensity rows I
 // (2 nrows uR real).  The fields are nin x nin_v (uR x vR, or less: zero
 // filled to that size).
 template <class R>
 int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int uR, int vR,
                   int nin, int nin_v, int padding, int Nd, int ss, void* D, void* Di, void* Abs,
-                  int write_filtered, const typename C2<R>::T* tw_u,
-                  const typename C2<R>::T* tw_v, const SumFuse* fz, const int* colsd, int Nc,
-                  void* G, void* I) {
+                  int write_filtered, const typename C2<R>::T* tw_u, const void* tw2_u,
+                  const void* tw2_v, const SumFuse* fz, const int* colsd, int Nc, void* G, void* H,
+                  bool wide, void* I) {
     using C = typename C2<R>::T;
+    const size_t cs2 = wide ? sizeof(double2) : sizeof(C);   // past the forward rows
     constexpr bool f32 = std::is_same<R, float>::value;
     // the summing form exists for complex64 fields (the FP32 batches) only
     if (fz && !f32) return set_error(ctx, BIMSIM_E_UNSUPPORTED, "fused sum needs complex64 fields");
@@ -917,13 +942,13 @@ int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int 
     const int nrows = write_filtered ? vR : S;
     // rows per workgroup: at most 1024 points, and at least 512 workgroups
     // per field where the rows allow it
-    auto rows_per_group = [&](int nr) {
-        int b = std::max(1, std::min(8, 1024 / uR));
+    auto rows_per_group = [&](int nr, size_t cs) {
+        int b = std::max(1, std::min(8, (int)(8192 / cs) / uR));
         while (b > 1 && (nr + b - 1) / b < 512) b /= 2;
         return b;
     };
     if (Nc > 0) {
-        int B = rows_per_group(nin_v);
+        int B = rows_per_group(nin_v, f32 ? sizeof(C) : sizeof(C) / 2);
         size_t lds = sizeof(C) * 2 * (size_t)B * uR;
         const dim3 grid((nin_v + B - 1) / B, 2);
         with_len(uR, [&](auto L) {
@@ -943,34 +968,50 @@ int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int 
         // a narrow pass band leaves few columns: fewer per workgroup, so
         // that the column pass still spreads over the chip
         while (Bc > 1 && (Nc + Bc - 1) / Bc < 128) Bc /= 2;
-        lds = sizeof(C) * 2 * (size_t)Bc * vR;
-        with_len(vR, [&](auto L) {
-            hipLaunchKernelGGL((cols_band_kernel<R, len_of(decltype(L){})>),
-                               dim3((Nc + Bc - 1) / Bc, 2), dim3(kThreads), lds, st, L, (C*)G,
-                               nin_v, row_begin, nrows, Nc, Bc, colsd, bp, tw_v);
+        lds = cs2 * 2 * (size_t)Bc * vR;
+        with_compute<R>(wide, [&](auto r2) {
+            using R2 = decltype(r2);
+            using C2T = typename C2<R2>::T;
+            with_len(vR, [&](auto L) {
+                hipLaunchKernelGGL((cols_band_kernel<R, R2, len_of(decltype(L){})>),
+                                   dim3((Nc + Bc - 1) / Bc, 2), dim3(kThreads), lds, st, L,
+                                   (const C*)G, (C2T*)H, nin_v, row_begin, nrows, Nc, Bc, colsd, bp,
+                                   (const C2T*)tw2_v);
+            });
+            return BIMSIM_OK;
         });
         BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     }
-    int B = rows_per_group(nrows);
-    size_t lds = sizeof(C) * 2 * (size_t)B * uR;
+    const int B = rows_per_group(nrows, f32 ? cs2 : cs2 / 2);
+    const size_t lds = cs2 * 2 * (size_t)B * uR;
     if (Nc > 0 && ss == 1 && !write_filtered && 2 * lds <= ctx->lds_max) {
         // both fields' rows per workgroup, detection on them in the same pass
-        with_len(uR, [&](auto L) {
-            hipLaunchKernelGGL((rows_inv_detect_kernel<R, len_of(decltype(L){})>),
-                               dim3((nrows + B - 1) / B), dim3(kThreads), 2 * lds, st, L,
-                               (const C*)G, Nc, vR, colsd, row_begin, nrows, B, off, Nd, (R*)D,
-                               (R*)Di, (R*)Abs, tw_u);
+        with_compute<R>(wide, [&](auto r2) {
+            using R2 = decltype(r2);
+            using C2T = typename C2<R2>::T;
+            with_len(uR, [&](auto L) {
+                hipLaunchKernelGGL((rows_inv_detect_kernel<R2, R, len_of(decltype(L){})>),
+                                   dim3((nrows + B - 1) / B), dim3(kThreads), 2 * lds, st, L,
+                                   (const C2T*)H, Nc, vR, colsd, row_begin, nrows, B, off, Nd,
+                                   (R*)D, (R*)Di, (R*)Abs, (const C2T*)tw2_u);
+            });
+            return BIMSIM_OK;
         });
         BIMSIM_HIP_CHECK(ctx, hipGetLastError());
         return BIMSIM_OK;
     }
     if (Nc > 0) {
-        with_len(uR, [&](auto L) {
-            hipLaunchKernelGGL((rows_inv_kernel<R, len_of(decltype(L){})>),
-                               dim3((nrows + B - 1) / B, 2), dim3(kThreads), lds, st, L,
-                               (const C*)G, Nc, vR, colsd, row_begin, nrows, B, (R*)I,
-                               write_filtered ? (C*)Uin : nullptr,
-                               write_filtered ? (C*)Ufin : nullptr, tw_u);
+        with_compute<R>(wide, [&](auto r2) {
+            using R2 = decltype(r2);
+            using C2T = typename C2<R2>::T;
+            with_len(uR, [&](auto L) {
+                hipLaunchKernelGGL((rows_inv_kernel<R2, R, len_of(decltype(L){})>),
+                                   dim3((nrows + B - 1) / B, 2), dim3(kThreads), lds, st, L,
+                                   (const C2T*)H, Nc, vR, colsd, row_begin, nrows, B, (R*)I,
+                                   write_filtered ? (C*)Uin : nullptr,
+                                   write_filtered ? (C*)Ufin : nullptr, (const C2T*)tw2_u);
+            });
+            return BIMSIM_OK;
         });
         BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     } else {
@@ -1055,13 +1096,19 @@ int detector_impl(bimsim_ctx* ctx, void* U, void* Uf, int uR, int vR, int nin, i
     const int Nc = (int)cols.size();
     const int nrows = write_filtered ? vR : Nd * ss;
     const int* colsd = nullptr;
-    void *G = nullptr, *I = nullptr;
+    void *G = nullptr, *H = nullptr, *I = nullptr;
+    const bool wide = !dbl && det_wide(ctx, uR, vR);
     BIMSIM_TRY(int_table_get(ctx, cols, &colsd));
     BIMSIM_TRY(scratch_get(ctx, kSlotFftA, sizeof(C) * 2 * (size_t)std::max(Nc, 1) * vR, &G));
+    H = G;
+    if (wide)
+        BIMSIM_TRY(scratch_get(ctx, kSlotDet, sizeof(double2) * 2 * (size_t)std::max(Nc, 1) * vR, &H));
     BIMSIM_TRY(scratch_get(ctx, kSlotFftB, sizeof(R) * 2 * (size_t)nrows * uR, &I));
     return detector_band<R>(ctx, bp, U, Uf, uR, vR, nin, nin_v, padding, Nd, ss, D, Di, Abs,
                             write_filtered, dbl ? (const C*)twd_u : (const C*)twf_u,
-                            dbl ? (const C*)twd_v : (const C*)twf_v, fz, colsd, Nc, G, I);
+                            dbl || wide ? (const void*)twd_u : (const void*)twf_u,
+                            dbl || wide ? (const void*)twd_v : (const void*)twf_v, fz, colsd, Nc, G,
+                            H, wide, I);
 }
 
 // The detector on the near field zero-filled to (fill uR) x (fill vR): the
@@ -1155,6 +1202,9 @@ int detector_run(bimsim_ctx* ctx, int prec, int quirks, void* U, void* Uf, int u
 namespace {
 
 int rows_per_wg(int n) { return std::max(1, std::min(8, 1024 / n)); }
+// of the inverse row pass in FP64 (an FP32 batch's, whose lines take twice
+// the LDS)
+int rows_per_wg_wide(int n) { return std::max(1, std::min(8, 512 / n)); }
 
 template <class R>
 int det_batch_launch_impl(bimsim_ctx* ctx, const DetBatch& b, const void* U, const void* Uf,
@@ -1165,11 +1215,12 @@ int det_batch_launch_impl(bimsim_ctx* ctx, const DetBatch& b, const void* U, con
     const C* tw = (const C*)b.tw;
     const unsigned nz = (unsigned)std::min(b.n, 65535);
     const size_t lds_r = sizeof(C) * 2 * 2 * (size_t)b.B * N;   // both fields' rows
-    const size_t lds_c = sizeof(C) * 2 * (size_t)b.Bc * N;
-    const size_t lds_i = sizeof(C) * 2 * 2 * (size_t)b.B2 * N;
+    const size_t cs2 = b.wide ? sizeof(double2) : sizeof(C);   // past the forward rows
+    const size_t lds_c = cs2 * 2 * (size_t)b.Bc * N;
+    const size_t lds_i = cs2 * 2 * 2 * (size_t)b.B2 * N;
     // the row passes read their twiddles from LDS where the N more elements fit
-    const size_t lds_tw = sizeof(C) * (size_t)N;
-    const bool tw_r = lds_r + lds_tw <= ctx->lds_max, tw_i = lds_i + lds_tw <= ctx->lds_max;
+    const size_t lds_tw = sizeof(C) * (size_t)N, lds_tw2 = cs2 * (size_t)N;
+    const bool tw_r = lds_r + lds_tw <= ctx->lds_max, tw_i = lds_i + lds_tw2 <= ctx->lds_max;
     const hipStream_t st = ctx->stream;
     constexpr bool f32 = std::is_same<R, float>::value;
     const bool sum = f32 && b.fused;
@@ -1181,20 +1232,27 @@ int det_batch_launch_impl(bimsim_ctx* ctx, const DetBatch& b, const void* U, con
             hipLaunchKernelGGL(kernel, grid_r, dim3(kThreads), lds, st, L, I, b.n, (const C*)U,
                                (const C*)Uf, b.B, b.d_cols, (C*)b.d_G, tw);
         };
-        auto inv = [&](auto kernel, size_t lds) {
-            hipLaunchKernelGGL(kernel, grid_i, dim3(kThreads), lds, st, L, I, b.n, b.B2, b.d_cols,
-                               (const C*)b.d_G, (R*)D, (R*)Di, (R*)Abs, tw);
-        };
         if (sum && tw_r) fwd(rows_fwd_batch_kernel<R, NN, f32, true>, lds_r + lds_tw);
         else if (sum) fwd(rows_fwd_batch_kernel<R, NN, f32, false>, lds_r);
         else if (tw_r) fwd(rows_fwd_batch_kernel<R, NN, false, true>, lds_r + lds_tw);
         else fwd(rows_fwd_batch_kernel<R, NN, false, false>, lds_r);
-        if (b.max_nc > 0)
-            hipLaunchKernelGGL((cols_band_batch_kernel<R, NN>),
-                               dim3((b.max_nc + b.Bc - 1) / b.Bc, 2, nz), dim3(kThreads), lds_c,
-                               st, L, I, b.n, b.Bc, b.d_cols, (C*)b.d_G, tw);
-        if (tw_i) inv(rows_inv_detect_batch_kernel<R, NN, true>, lds_i + lds_tw);
-        else inv(rows_inv_detect_batch_kernel<R, NN, false>, lds_i);
+        with_compute<R>(b.wide, [&](auto r2) {
+            using R2 = decltype(r2);
+            using C2T = typename C2<R2>::T;
+            const C2T* tw2 = (const C2T*)b.tw2;
+            auto inv = [&](auto kernel, size_t lds) {
+                hipLaunchKernelGGL(kernel, grid_i, dim3(kThreads), lds, st, L, I, b.n, b.B2,
+                                   b.d_cols, (const C2T*)b.d_H, (R*)D, (R*)Di, (R*)Abs, tw2);
+            };
+            if (b.max_nc > 0)
+                hipLaunchKernelGGL((cols_band_batch_kernel<R, R2, NN>),
+                                   dim3((b.max_nc + b.Bc - 1) / b.Bc, 2, nz), dim3(kThreads),
+                                   lds_c, st, L, I, b.n, b.Bc, b.d_cols, (const C*)b.d_G,
+                                   (C2T*)b.d_H, tw2);
+            if (tw_i) inv(rows_inv_detect_batch_kernel<R2, R, NN, true>, lds_i + lds_tw2);
+            else inv(rows_inv_detect_batch_kernel<R2, R, NN, false>, lds_i);
+            return BIMSIM_OK;
+        });
     });
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
@@ -1260,7 +1318,8 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
     // rows (columns) per workgroup, fewer when the batch is small so that
     // each pass still spreads over the chip
     const int n = (int)insts.size();
-    int B = rows_per_wg(N), B2 = B, Bc = std::max(1, std::min(8, 2048 / N));
+    const bool wide = f32 && det_wide(ctx, N, N);
+    int B = rows_per_wg(N), B2 = wide ? rows_per_wg_wide(N) : B, Bc = std::max(1, std::min(8, 2048 / N));
     while (B > 1 && (long long)n * ((max_nin + B - 1) / B) < 512) B /= 2;
     while (B2 > 1 && (long long)n * ((max_nd + B2 - 1) / B2) < 512) B2 /= 2;
     while (Bc > 1 && (long long)n * ((max_nc + Bc - 1) / Bc) < 128) Bc /= 2;
@@ -1271,14 +1330,19 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
     const float* twf;
     BIMSIM_TRY(twiddles_get(ctx, N, &twd, &twf));
     out->tw = f32 ? (const void*)twf : (const void*)twd;
+    out->tw2 = f32 && !wide ? (const void*)twf : (const void*)twd;
+    out->wide = wide;
     if (cols.empty()) cols.push_back(0);
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     if (hipMalloc(&out->d_inst, sizeof(DetInst) * insts.size()) != hipSuccess ||
         hipMalloc((void**)&out->d_cols, sizeof(int) * cols.size()) != hipSuccess ||
-        hipMalloc(&out->d_G, cs * (size_t)std::max<long long>(1, g)) != hipSuccess) {
+        hipMalloc(&out->d_G, cs * (size_t)std::max<long long>(1, g)) != hipSuccess ||
+        (wide && hipMalloc(&out->d_H, sizeof(double2) * (size_t)std::max<long long>(1, g)) !=
+                     hipSuccess)) {
         det_batch_destroy(out);
         return set_error(ctx, BIMSIM_E_NOMEM, "out of device memory for the batched detector");
     }
+    if (!wide) out->d_H = out->d_G;
     BIMSIM_HIP_CHECK(ctx, hipMemcpy(out->d_inst, insts.data(), sizeof(DetInst) * insts.size(),
                                     hipMemcpyHostToDevice));
     BIMSIM_HIP_CHECK(ctx, hipMemcpy(out->d_cols, cols.data(), sizeof(int) * cols.size(),
@@ -1300,6 +1364,7 @@ int det_batch_launch(bimsim_ctx* ctx, const DetBatch& b, const void* U, const vo
 void det_batch_destroy(DetBatch* b) {
     if (b->d_inst) (void)hipFree(b->d_inst);
     if (b->d_cols) (void)hipFree(b->d_cols);
+    if (b->d_H && b->d_H != b->d_G) (void)hipFree(b->d_H);
     if (b->d_G) (void)hipFree(b->d_G);
     *b = DetBatch();
 }
@@ -1367,6 +1432,13 @@ int detector_noalloc_impl(bimsim_ctx* ctx, unsigned char* work, int quirks, cons
     const size_t o_G = o_cols + align256(sizeof(int) * std::max(Nc, 1));
     const size_t o_I = o_G + align256(sizeof(C) * 2 * (size_t)std::max(Nc, 1) * vR);
     const size_t need = o_I + sizeof(R) * 2 * (size_t)nrows * uR;
+    // in FP64 past the columns where their filtered copy and the FP64
+    // twiddles fit as well
+    constexpr bool f32 = std::is_same<R, float>::value;
+    const size_t o_H = align256(need);
+    const size_t o_t2u = o_H + align256(sizeof(double2) * 2 * (size_t)std::max(Nc, 1) * vR);
+    const size_t o_t2v = o_t2u + align256(sizeof(double2) * uR);
+    const bool wide = f32 && det_wide(ctx, uR, vR) && o_t2v + sizeof(double2) * vR <= kNoAllocBytes;
     if (need > kNoAllocBytes)
         return set_error(ctx, BIMSIM_E_INVALID,
                          "the detector needs %zu bytes of work memory; the allocation-free "
@@ -1379,13 +1451,22 @@ int detector_noalloc_impl(bimsim_ctx* ctx, unsigned char* work, int quirks, cons
                        tu, uR);
     hipLaunchKernelGGL(twiddle_fill_kernel<C>, dim3((vR + 255) / 256), dim3(256), 0, ctx->stream,
                        tv, vR);
+    double2 *t2u = (double2*)tu, *t2v = (double2*)tv;
+    if (wide) {
+        t2u = (double2*)(work + o_t2u);
+        t2v = (double2*)(work + o_t2v);
+        hipLaunchKernelGGL(twiddle_fill_kernel<double2>, dim3((uR + 255) / 256), dim3(256), 0,
+                           ctx->stream, t2u, uR);
+        hipLaunchKernelGGL(twiddle_fill_kernel<double2>, dim3((vR + 255) / 256), dim3(256), 0,
+                           ctx->stream, t2v, vR);
+    }
     if (Nc > 0)
         hipLaunchKernelGGL(band_cols_kernel, dim3((Nc + 255) / 256), dim3(256), 0, ctx->stream,
                            cols, n1, n2, uR);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return detector_band<R>(ctx, bp, const_cast<void*>(U), const_cast<void*>(Uf), uR, vR, uR, vR,
-                            padding, Nd, ss, D, Di, Abs, 0, tu, tv, nullptr, cols, Nc, work + o_G,
-                            work + o_I);
+                            padding, Nd, ss, D, Di, Abs, 0, tu, t2u, t2v, nullptr, cols, Nc,
+                            work + o_G, wide ? work + o_H : work + o_G, wide, work + o_I);
 }
 
 }  // namespace

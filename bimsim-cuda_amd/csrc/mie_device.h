@@ -3,6 +3,15 @@
 // each, and the coefficient formula per (sphere, order).  Shared by the
 // coefficient kernels and the batch's fused pre-pass launch; every file
 // that includes it is built with -ffp-contract=off.
+//
+// Two forms.  The general one runs the reference's CJYVA (power series or
+// asymptotic expansions for the start values, start orders by its secant
+// search), for any order and argument.  The closed form below it covers the
+// spheres whose order belongs to their size (mie_closed_form): at half-odd
+// orders the start values are sin z / z and cos z / z, so a sphere is three
+// short recurrences and one quotient per order.  Both are bound by the
+// latency of one sphere's chain, not by throughput; the general form's was
+// mostly instruction fetch of its long straight-line code.
 #pragma once
 
 #include <algorithm>
@@ -112,6 +121,176 @@ __device__ __forceinline__ void mie_block(const SphereDev* sh, const double* kh,
     for (int idx = t; idx < cnt * per; idx += (int)blockDim.x) {
         const int i = idx / per, l = idx - i * per;
         if (l <= sh[i].Nl) mie_order(sh[i], l, lds + (size_t)8 * i * wstride, wstride, A, B);
+    }
+}
+
+// ---------------------------------------------------------- closed form
+// Spheres per block: few, so that the quotients (one per order) spread over
+// the chip as well.
+constexpr int kClosedSph = 8;
+constexpr int kClosedThreads = 256;
+
+// One sphere's input to the coefficients.
+struct MieSph {
+    double x, zr, zi;   // k a and n k a
+    double nr, ni;
+    int Nl, coeff_off;
+};
+
+__host__ __device__ inline MieSph mie_sph(const SphereDev& S, double kmag) {
+    const zc z = zj::zsc(S.a, zj::zsc(kmag, zc{S.n[0], S.n[1]}));
+    return MieSph{kmag * S.a, z.r, z.i, S.n[0], S.n[1], S.Nl, S.coeff_off};
+}
+
+// The spheres the closed form takes: the order within 20 of the size's own
+// (sphere::calcNl: x + 4 x^(1/3) + 2), so that no order leaves the range of
+// a double, and arguments whose sinh and cosh stay far from overflow.
+__host__ __device__ inline bool mie_closed_form(const MieSph& m) {
+    const double az = sqrt(m.zr * m.zr + m.zi * m.zi);
+    return m.Nl >= 2 && m.x >= 1e-2 && m.x <= 4096.0 && az >= 1e-2 && az <= 4096.0 &&
+           m.zr >= 0.0 && fabs(m.zi) <= 100.0 &&
+           (double)m.Nl <= m.x + 4.05 * cbrt(m.x) + 20.0;
+}
+
+// First order of the downward recurrence for orders up to n of argument
+// magnitude az: far enough past both that what the start leaves out of
+// order n (the ratio of j to y at the start against that at n, which falls
+// as exp(-(2 sqrt(2)/3) 2 (d/az^(1/3))^(3/2)) past the turning point, d
+// orders beyond it) is below 1e-18.
+__device__ inline int mie_start_order(int n, double az) {
+    const double c = cbrt(az);
+    return (int)(fmax((double)n, az) + 8.0 * c + 16.0);
+}
+
+// LDS of a sphere in doubles: orders 0 .. Nl of j (of ka, unscaled), y (of
+// ka), j (of n ka, complex, unscaled), w = lmax + 2 each, and the scales.
+__host__ __device__ inline int mie_closed_doubles(int w) { return 4 * w + 4; }
+
+// Coefficients of cnt <= kClosedSph spheres sh (in LDS); lds as above per
+// sphere.  Waves 0, 1 and 2 run a part each (j of ka, y of ka, j of n ka;
+// lane s: sphere s), then the block's threads take the (sphere, order)
+// quotients.
+__device__ __forceinline__ void mie_closed_block(const MieSph* sh, int cnt, int quirks, double* lds,
+                                                 int w, double2* A, double2* B) {
+    const int t = (int)threadIdx.x;
+    const int s = t % kWave, role = t / kWave;
+    const int per = mie_closed_doubles(w);
+    if (s < cnt && role < 3) {
+        const MieSph m = sh[s];
+        const int n = m.Nl;
+        double* const o = lds + s * per;
+        if (role == 2) {
+            // j_k = (2k + 3)/z j_{k+1} - j_{k+2}, scaled to the larger of
+            // sin z / z and (sin z / z - cos z) / z at the end
+            const double az2 = m.zr * m.zr + m.zi * m.zi, inv = 1.0 / az2;
+            const double ur = m.zr * inv, ui = -(m.zi * inv);
+            double sr, cr;
+            sincos(m.zr, &sr, &cr);
+            const double e = exp(m.zi), ei = 1.0 / e;
+            const double ch = 0.5 * (e + ei);
+            // sinh near zero by its series (the difference would cancel)
+            const double q = m.zi * m.zi;
+            const double sh_s =
+                m.zi * (1.0 + q * (1.0 / 6.0 + q * (1.0 / 120.0 + q * (1.0 / 5040.0 +
+                                                                      q * (1.0 / 362880.0)))));
+            const double shi = fabs(m.zi) < 0.25 ? sh_s : 0.5 * (e - ei);
+            const zc u = {ur, ui};
+            const zc j0 = zj::zmul(zc{sr * ch, cr * shi}, u);
+            const zc j1 = zj::zsub(zj::zmul(j0, u), zj::zmul(zc{cr * ch, -(sr * shi)}, u));
+            double fr = 1e-100, fi = 0.0, gr = 0.0, gi = 0.0;   // orders k + 1 and k + 2
+            const int top = mie_start_order(n, sqrt(az2));
+            double c = 2.0 * top + 3.0;
+#pragma clang loop unroll_count(2)
+            for (int k = top; k >= 0; --k) {
+                const double ar = c * ur, ai = c * ui;
+                const double hr = fma(ar, fr, fma(-ai, fi, -gr));
+                const double hi = fma(ar, fi, fma(ai, fr, -gi));
+                if (k <= n) {
+                    o[2 * w + 2 * k] = hr;
+                    o[2 * w + 2 * k + 1] = hi;
+                }
+                gr = fr;
+                gi = fi;
+                fr = hr;
+                fi = hi;
+                c -= 2.0;
+            }
+            const bool use0 = j0.r * j0.r + j0.i * j0.i > j1.r * j1.r + j1.i * j1.i;
+            const zc sc = use0 ? zj::zdiv(j0, zc{fr, fi}) : zj::zdiv(j1, zc{gr, gi});
+            o[4 * w + 1] = sc.r;
+            o[4 * w + 2] = sc.i;
+        } else {
+            const double inv = 1.0 / m.x;
+            double sn, cs;
+            sincos(m.x, &sn, &cs);
+            if (role == 0) {
+                const double j0 = sn * inv, j1 = fma(j0, inv, -(cs * inv));
+                double f = 1e-100, g = 0.0;
+                const int top = mie_start_order(n, m.x);
+                double c = 2.0 * top + 3.0;
+#pragma clang loop unroll_count(2)
+                for (int k = top; k >= 0; --k) {
+                    const double h = fma(c * inv, f, -g);
+                    if (k <= n) o[k] = h;
+                    g = f;
+                    f = h;
+                    c -= 2.0;
+                }
+                o[4 * w] = fabs(j0) > fabs(j1) ? j0 / f : j1 / g;
+            } else {
+                // y_0 above 12: with quirks the reference's expansion adds
+                // cos(x - pi/2) = sin x (its q is zero at this order)
+                const double yt = -(cs * inv);
+                double g = quirks && m.x > 12.0 ? (sn - cs) * inv : yt;
+                double f = fma(yt, inv, -(sn * inv));
+                o[w] = g;
+                o[w + 1] = f;
+                double c = 3.0;
+#pragma clang loop unroll_count(2)
+                for (int k = 2; k <= n; ++k) {
+                    const double h = fma(c * inv, f, -g);
+                    o[w + k] = h;
+                    g = f;
+                    f = h;
+                    c += 2.0;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    int lm = 0;
+    for (int i = 0; i < cnt; ++i) lm = max(lm, sh[i].Nl);
+    const int nl = lm + 1;
+    for (int idx = t; idx < cnt * nl; idx += (int)blockDim.x) {
+        const int i = idx / nl, l = idx - i * nl;
+        const MieSph& m = sh[i];
+        if (l > m.Nl) continue;
+        const double* const o = lds + i * per;
+        const double* const Y = o + w;
+        const double* const K = o + 2 * w;
+        const double js = o[4 * w], ix = 1.0 / m.x;
+        const zc ks = {o[4 * w + 1], o[4 * w + 2]};
+        // the derivatives f_l' = f_{l-1} - (l + 1)/z f_l (f_0' = -f_1)
+        const int lo = l > 0 ? l - 1 : 1;
+        const double sg = l > 0 ? 1.0 : -1.0, c = l > 0 ? l + 1.0 : 0.0;
+        const double j1 = o[l] * js, y1 = Y[l];
+        const double jp1 = fma(-(c * ix), j1, sg * (o[lo] * js));
+        const double yp1 = fma(-(c * ix), y1, sg * Y[lo]);
+        const zc j2 = zj::zmul(zc{K[2 * l], K[2 * l + 1]}, ks);
+        const zc jl = zj::zmul(zc{K[2 * lo], K[2 * lo + 1]}, ks);
+        const zc jp2 = zj::zsub(zj::zsc(sg, jl), zj::zmul(zj::rdiv(c, zc{m.zr, m.zi}), j2));
+        const zc nc = {m.nr, m.ni};
+        const zc h = {j1, y1}, hp = {jp1, yp1};
+        const zc den = zj::zsub(zj::zmul(j2, hp), zj::zmul(zj::zmul(h, jp2), nc));
+        // j1 h' - j1' h = i (j1 y1' - j1' y1)
+        const zc num_a = {0.0, fma(j1, yp1, -(jp1 * y1))};
+        const zc num_b = zj::zsub(zj::zmul(zj::zsc(j1, jp2), nc), zj::zsc(jp1, j2));
+        const double f = 2.0 * l + 1.0;
+        const zc il = {(l & 1) ? 0.0 : ((l & 2) ? -f : f), (l & 1) ? ((l & 2) ? -f : f) : 0.0};
+        const zc An = zj::zmul(il, zj::zdiv(num_a, den));
+        const zc Bn = zj::zmul(il, zj::zdiv(num_b, den));
+        A[m.coeff_off + l] = make_double2(An.r, An.i);
+        B[m.coeff_off + l] = make_double2(Bn.r, Bn.i);
     }
 }
 

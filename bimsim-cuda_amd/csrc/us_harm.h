@@ -589,7 +589,7 @@ __device__ __forceinline__ void quad_load(__amdgpu_buffer_rsrc_t rs, const int* 
 // and row m + 1's, or the one packed register).  Block gb of the bucket
 // (= L0/4 + b) runs from row 4 gb on and up to the block of order Nl, as
 // in harm_planar_chunk.  The chunk's first row pair runs every block (the
-// blocks past Nl there take the zero records the fold writes, which start
+// blocks past Nl there take the zero records of the table, which start
 // their sums at zero; no later product or read touches them).
 template <int L, int C, int L0, int k, bool kSeed>
 __device__ __forceinline__ void quad_groups(const float* a, float zar, float zai, float zbr,

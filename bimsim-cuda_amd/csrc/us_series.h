@@ -82,16 +82,16 @@ struct UfInst;
 struct SumInst;
 
 // The other work of an FP32 batch's pre-pass, run in one launch with a
-// harmonic plan's records (series_plan_launch_prepass): the Mie
-// coefficients of n_mie_sph spheres (sphere i at mie_kmag[i]) in blocks of
-// spb, Bessel arrays of wstride in LDS, and the complex64 incident fields
+// harmonic plan's wave tables (series_plan_launch_prepass): the Mie
+// coefficients of n_mie_sph spheres (sphere i at mie_kmag[i], all of the
+// closed form, wstride orders in LDS), and the complex64 incident fields
 // of n_uf instances, uf_blocks blocks of 256 pixels each; with sum, also
 // the clearing of each instance's detector images in D and Di (sum[i] for
 // instance i), which the batch's sum kernel does otherwise.
 struct PrepassArgs {
     const SphereDev* mie_sph;
     const double* mie_kmag;
-    int n_mie_sph, spb, wstride, quirks;
+    int n_mie_sph, wstride, quirks;
     double2* A;
     double2* B;
     const UfInst* uf;
@@ -245,7 +245,7 @@ struct SeriesPlan {
     double* d_pl = nullptr;       // normalised Legendre values per (m, wave, l)
     double2* d_e = nullptr;       // exp(i m phi_k) per (m, wave)
     double2* d_phi = nullptr;     // wave weights (1/nk) subA exp(i k k.c) per sphere
-    float4* d_rec = nullptr;      // harmonic records per (sphere, m, l), then times B_l
+    float4* d_rec = nullptr;      // harmonic records per (sphere, m, l) times B_l
     float4* d_rec_in = nullptr;   // the same records times A_l
     float* d_cst = nullptr;       // scaled Legendre recurrence constants per (m, l)
     int* d_perm = nullptr;        // pixel orders of the instances with perm_off >= 0
@@ -272,21 +272,25 @@ void series_plan_destroy(SeriesPlan* plan);
 
 // Launches the plan on the context stream; allocation- and
 // synchronisation-free, so it can be captured into a graph.  The two halves
-// can run apart: the wave tables (harmonic sums or wave records, from the
-// waves only) and the per-pixel sums (which read A and B).
+// can run apart: the wave tables (from the waves only), and the records'
+// coefficients and the per-pixel sums (which read A and B).
 int series_plan_launch(bimsim_ctx* ctx, const SeriesPlan& plan, const double* waves,
                        const double2* A, const double2* B, float2* U);
 int series_plan_launch_waves(bimsim_ctx* ctx, const SeriesPlan& plan, const double* waves);
-// Legendre tables, then one launch of the records of P beside the
-// coefficients and incident fields of a (instead of
-// series_plan_launch_waves, the Mie launch and the incident-field launch).
-// P must be a harmonic plan and prepass_lds(a) <= kPrepassLds.
+// One launch of P's wave tables beside the coefficients and incident fields
+// of a (instead of series_plan_launch_waves, the Mie launch and the
+// incident-field launch).  P must be a harmonic plan and prepass_lds(a) <=
+// kPrepassLds.
 int series_plan_launch_prepass(bimsim_ctx* ctx, const SeriesPlan& P, const double* waves,
                                const PrepassArgs& a);
-// after_fold: an event the sums (not the records' coefficient fold before
-// them) wait for.
+// after_records: an event the sums (not the records before them) wait for.
 int series_plan_launch_sums(bimsim_ctx* ctx, const SeriesPlan& plan, const double2* A,
-                            const double2* B, float2* U, hipEvent_t after_fold = nullptr);
+                            const double2* B, float2* U, hipEvent_t after_records = nullptr);
+
+// Whether a harmonic plan has too few (instance, azimuth) rows to fill the
+// chip with a block each.
+bool series_few_rows(const bimsim_ctx* ctx, const SeriesPlan& plan);
+
 
 // Order capacity for Nl + 1 orders, or -1.
 int series_capacity(int nl1);

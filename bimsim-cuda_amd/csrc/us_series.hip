@@ -347,11 +347,37 @@ __host__ __device__ inline long long tri_off(int m, int lh) {
     return (long long)m * lh - (long long)m * (m - 1) / 2;
 }
 
-// Pn_lm(cos th_w) in pl[pl_off + (tri_off(m) + (l - m)) * nk + w],
-// e^{i m phi_w} in e[e_off + m * nk + w] and, at m = 0, the wave weights
-// phi_w = (1/nk) subA exp(i kmag k.c) of every sphere of the instance in
-// phi[woff + w] (FP64); block 0 also clears the work-queue counters.
-// Grid: (wave blocks, instances, m).
+// Row m of instance i's wave tables, waves w0, w0 + step, ...: Pn_lm(cos
+// th_w) in pl[pl_off + (tri_off(m) + (l - m)) * nk + w], e^{i m phi_w} in
+// e[e_off + m * nk + w], and of the instance's spheres every lh-th from the
+// m-th the wave weights phi_w = (1/nk) subA exp(i kmag k.c) in phi[woff + w]
+// (FP64).
+__device__ __forceinline__ void harm_legendre_row(int m, int i, int w0, int step,
+                                                  const SeriesInst* __restrict__ insts,
+                                                  const SeriesSph* __restrict__ sph,
+                                                  const double* __restrict__ waves,
+                                                  const double* __restrict__ h64,
+                                                  double* __restrict__ pl,
+                                                  double2* __restrict__ e,
+                                                  double2* __restrict__ phi) {
+    const SeriesInst& I = insts[i];
+    if (m >= I.lh) return;
+    for (int w = w0; w < I.nk; w += step) {
+        const d3 k = mk(waves + 3 * (I.wave_off + w));
+        legendre_column(m, I.lh, k.z, pl + I.pl_off + tri_off(m, I.lh) * I.nk + w, I.nk, h64);
+        const double az = atan2(k.y, k.x);
+        e[I.e_off + (long long)m * I.nk + w] = make_double2(cos(m * az), sin(m * az));
+        for (int s = I.s_begin + m; s < I.s_begin + I.ns; s += I.lh) {
+            const SeriesSph& SS = sph[s];
+            const d3 c = sub(mk(SS.s.p), I.f);
+            const dc ph = cscl(cexp_i(I.kmag * dot(k, c)), I.sA);
+            phi[SS.woff + w] = make_double2(ph.r, ph.i);
+        }
+    }
+}
+
+// The wave tables of every instance; block 0 also clears the work-queue
+// counters.  Grid: (wave blocks, instances, m).
 __global__ void harm_legendre_kernel(const SeriesInst* __restrict__ insts,
                                      const SeriesSph* __restrict__ sph, int n_inst,
                                      const double* __restrict__ waves,
@@ -361,24 +387,25 @@ __global__ void harm_legendre_kernel(const SeriesInst* __restrict__ insts,
     const int m = blockIdx.z;
     if (blockIdx.x == 0 && blockIdx.y == 0 && m == 0)
         for (int i = threadIdx.x; i < n_counters; i += blockDim.x) counters[i] = 0;
-    for (int i = blockIdx.y; i < n_inst; i += gridDim.y) {
-        const SeriesInst& I = insts[i];
-        if (m >= I.lh) continue;
-        for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < I.nk; w += gridDim.x * blockDim.x) {
-            const d3 k = mk(waves + 3 * (I.wave_off + w));
-            legendre_column(m, I.lh, k.z, pl + I.pl_off + tri_off(m, I.lh) * I.nk + w, I.nk, h64);
-            const double az = atan2(k.y, k.x);
-            e[I.e_off + (long long)m * I.nk + w] = make_double2(cos(m * az), sin(m * az));
-            if (m == 0) {
-                for (int s = I.s_begin; s < I.s_begin + I.ns; ++s) {
-                    const SeriesSph& SS = sph[s];
-                    const d3 c = sub(mk(SS.s.p), I.f);
-                    const dc ph = cscl(cexp_i(I.kmag * dot(k, c)), I.sA);
-                    phi[SS.woff + w] = make_double2(ph.r, ph.i);
-                }
-            }
-        }
-    }
+    for (int i = blockIdx.y; i < n_inst; i += gridDim.y)
+        harm_legendre_row(m, i, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x,
+                          insts, sph, waves, h64, pl, e, phi);
+}
+
+// A record (U1, U2) times the order's coefficients: B_l into rec, A_l into
+// rec_in (the pixels outside and inside the sphere read one each).
+__device__ __forceinline__ void harm_record_store(const SeriesSph& SS, int l, long long o,
+                                                  double x1, double y1, double x2, double y2,
+                                                  const double2* __restrict__ A,
+                                                  const double2* __restrict__ B,
+                                                  float4* __restrict__ rec,
+                                                  float4* __restrict__ rec_in) {
+    auto mul = [&](double2 c) {
+        return make_float4((float)(x1 * c.x - y1 * c.y), (float)(x1 * c.y + y1 * c.x),
+                           (float)(x2 * c.x - y2 * c.y), (float)(x2 * c.y + y2 * c.x));
+    };
+    rec[SS.toff + o] = mul(B[SS.s.coeff_off + l]);
+    rec_in[SS.toff + o] = mul(A[SS.s.coeff_off + l]);
 }
 
 // Records per (sphere, m, l) from the wave tables.  Block (m, instance)
@@ -575,7 +602,8 @@ __device__ __forceinline__ void harm_records_tile(
     int m, int tile, int s_first, int s_step, const SeriesInst* __restrict__ insts,
     const SeriesSph* __restrict__ sph, int n_sph, const double* __restrict__ pl,
     const double2* __restrict__ e, const double2* __restrict__ phi,
-    const double* __restrict__ h64, float4* __restrict__ rec) {
+    const double* __restrict__ h64, const double2* __restrict__ A, const double2* __restrict__ B,
+    float4* __restrict__ rec, float4* __restrict__ rec_in) {
     __shared__ double red[kRecThreads / 64][4 * kRecTile];
     for (int s = s_first; s < n_sph; s += s_step) {
         const SeriesSph& SS = sph[s];
@@ -635,7 +663,7 @@ __device__ __forceinline__ void harm_records_tile(
             const int j = threadIdx.x;
             const int k = kRecTile * tile + j;
             if (k < width) {
-                float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+                const long long o = (long long)m * width + k;
                 if (need[j]) {
                     dc tp = {0.0, 0.0}, tm = {0.0, 0.0};
                     for (int q = 0; q < kRecThreads / 64; ++q) {
@@ -656,12 +684,13 @@ __device__ __forceinline__ void harm_records_tile(
                         f = 4.0 * M_PI / (2.0 * l + 1.0) * h64[kHK + m * kH + l];
                     }
                     if (m == 0)
-                        r = make_float4((float)(f * tp.r), (float)(f * tp.i), 0.f, 0.f);
+                        harm_record_store(SS, l, o, f * tp.r, f * tp.i, 0.0, 0.0, A, B, rec, rec_in);
                     else
-                        r = make_float4((float)(f * (tp.r + tm.r)), (float)(f * (tp.i + tm.i)),
-                                        (float)(f * (tp.i - tm.i)), (float)(f * (tm.r - tp.r)));
+                        harm_record_store(SS, l, o, f * (tp.r + tm.r), f * (tp.i + tm.i),
+                                          f * (tp.i - tm.i), f * (tm.r - tp.r), A, B, rec, rec_in);
+                } else {
+                    rec[SS.toff + o] = rec_in[SS.toff + o] = make_float4(0.f, 0.f, 0.f, 0.f);
                 }
-                rec[SS.toff + (long long)m * width + k] = r;
             }
         }
     }
@@ -693,16 +722,18 @@ RecTiles rec_tiles(int max_nlv, int max_ns, int l_cap, int s_cap, int kW) {
 __global__ __launch_bounds__(kRecThreads) void harm_records_tile_kernel(
     const SeriesInst* __restrict__ insts, const SeriesSph* __restrict__ sph, int n_sph,
     const double* __restrict__ pl, const double2* __restrict__ e, const double2* __restrict__ phi,
-    const double* __restrict__ h64, float4* __restrict__ rec) {
+    const double* __restrict__ h64, const double2* __restrict__ A, const double2* __restrict__ B,
+    float4* __restrict__ rec, float4* __restrict__ rec_in) {
     harm_records_tile(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, insts, sph, n_sph, pl, e, phi,
-                      h64, rec);
+                      h64, A, B, rec, rec_in);
 }
 
-// The records times the sphere's coefficients, once both are formed:
-// rec (in place) times B_l, rec_in times A_l, l the record's order; the
-// records of orders below the row or past Nl stay zero.  Rows 0 .. tl - 1
-// of each table (tl / 2 records each for a planar sphere, else tl) hold
-// every record the pixel kernel reads.  Grid: (record blocks, spheres).
+// The row form's records times the sphere's coefficients, once both are
+// formed: rec (in place) times B_l, rec_in times A_l, l the record's order;
+// the records of orders below the row or past Nl stay zero.  (Folded into
+// the row form itself, as the tile form has it, the scattered stores of both
+// tables cost more than this launch: 145 + 20 -> 300 us on a 64-image
+// sweep.)  Grid: (record blocks, spheres).
 __global__ __launch_bounds__(kRecThreads) void harm_fold_kernel(const SeriesSph* __restrict__ sph,
                                                                 int n_sph,
                                                                 const double2* __restrict__ A,
@@ -719,64 +750,50 @@ __global__ __launch_bounds__(kRecThreads) void harm_fold_kernel(const SeriesSph*
              o += gridDim.x * kRecThreads) {
             const int m = o / width, k = o - m * width;
             const int l = planar ? 2 * k + (m & 1) : k;
-            float4 ob = make_float4(0.f, 0.f, 0.f, 0.f), oa = ob;
-            if (l >= m && l <= SS.s.Nl) {
-                const float4 r = rec[SS.toff + o];
-                const double2 b = B[SS.s.coeff_off + l], a = A[SS.s.coeff_off + l];
-                // U1 = (r.x, r.y) and U2 = (r.z, r.w), each times the coefficient
-                auto mul = [](double x, double y, double2 c) {
-                    return make_float2((float)(x * c.x - y * c.y), (float)(x * c.y + y * c.x));
-                };
-                const float2 b1 = mul(r.x, r.y, b), b2 = mul(r.z, r.w, b);
-                const float2 a1 = mul(r.x, r.y, a), a2 = mul(r.z, r.w, a);
-                ob = make_float4(b1.x, b1.y, b2.x, b2.y);
-                oa = make_float4(a1.x, a1.y, a2.x, a2.y);
-            }
-            rec[SS.toff + o] = ob;
-            rec_in[SS.toff + o] = oa;
+            if (l < m || l > SS.s.Nl) continue;
+            const float4 r = rec[SS.toff + o];
+            harm_record_store(SS, l, o, r.x, r.y, r.z, r.w, A, B, rec, rec_in);
         }
     }
 }
 
 // The FP32 batch's pre-pass as one launch: Mie coefficients (blocks
-// [0, n_mie), mie_block over spb spheres each, Bessel arrays in dynamic
-// LDS), the harmonic records (the next n_rec blocks, one per (m, instance)
-// as harm_records_kernel) and the incident fields (the rest, 256
-// pixels of one instance each, which also clear its detector images when
-// a.sum is given).  None reads what another writes, and the
-// records read only the Legendre tables of the launch before, so the long
-// dependent chains of the coefficients run on a few compute units while
-// the records and fields fill the others.  The role is uniform per block.
+// [0, n_mie), mie_closed_block over kClosedSph spheres each), the wave
+// tables (the next n_leg blocks: harm_legendre_row, kRecThreads waves of one
+// (row, instance) each) and the incident fields (the rest, 256 pixels of
+// one instance each, which also clear its detector images when a.sum is
+// given).  None reads what another writes; the records of the next launch
+// read the first two.  The role is uniform per block.
 __global__ __launch_bounds__(kRecThreads) void prepass_kernel(
-    PrepassArgs a, int n_mie, int n_rec, int rec_m, int rec_tiles,
-    const SeriesInst* __restrict__ insts, const SeriesSph* __restrict__ sph, int n_sph,
-    const double* __restrict__ pl, const double2* __restrict__ e, const double2* __restrict__ phi,
-    const double* __restrict__ h64, float4* __restrict__ rec) {
-    static_assert(kRecThreads >= mie::kMieThreads, "the coefficient waves fit the block");
-    extern __shared__ mie::zc mie_lds[];
-    __shared__ SphereDev msph[mie::kSphPerLaunch];
-    __shared__ double mk[mie::kSphPerLaunch];
+    PrepassArgs a, int n_mie, int n_leg, int leg_w, int n_inst,
+    const SeriesInst* __restrict__ insts, const SeriesSph* __restrict__ sph,
+    const double* __restrict__ waves, const double* __restrict__ h64, double* __restrict__ pl,
+    double2* __restrict__ e, double2* __restrict__ phi, int* __restrict__ counters,
+    int n_counters) {
+    static_assert(kRecThreads == mie::kClosedThreads, "the coefficient block's size");
+    extern __shared__ double mie_lds[];
+    __shared__ mie::MieSph msph[mie::kClosedSph];
     int b = (int)blockIdx.x;
     const int t = (int)threadIdx.x;
+    if (b == 0)   // the work-queue counters of the sums
+        for (int i = t; i < n_counters; i += kRecThreads) counters[i] = 0;
     if (b < n_mie) {
-        const int s0 = b * a.spb;
-        const int cnt = min(a.spb, a.n_mie_sph - s0);
-        if (t < cnt) {
-            msph[t] = a.mie_sph[s0 + t];
-            mk[t] = a.mie_kmag[s0 + t];
-        }
+        const int s0 = b * mie::kClosedSph;
+        const int cnt = min(mie::kClosedSph, a.n_mie_sph - s0);
+        if (t < cnt) msph[t] = mie::mie_sph(a.mie_sph[s0 + t], a.mie_kmag[s0 + t]);
         __syncthreads();
-        mie::mie_block(msph, mk, cnt, a.quirks, mie_lds, a.wstride, a.A, a.B);
+        mie::mie_closed_block(msph, cnt, a.quirks, mie_lds, a.wstride, a.A, a.B);
         return;
     }
     b -= n_mie;
-    if (b < n_rec) {
-        const int per_s = rec_m * rec_tiles;
-        const int s = b / per_s, r = b - s * per_s;
-        harm_records_tile(r % rec_m, r / rec_m, s, n_sph, insts, sph, n_sph, pl, e, phi, h64, rec);
+    if (b < n_leg) {
+        const int w = b % leg_w, r = b / leg_w;
+        const int i = r % n_inst, m = r / n_inst;
+        harm_legendre_row(m, i, w * kRecThreads + t, leg_w * kRecThreads, insts, sph, waves, h64,
+                          pl, e, phi);
         return;
     }
-    b -= n_rec;
+    b -= n_leg;
     const int i = b / a.uf_blocks, pix = (b - i * a.uf_blocks) * kRecThreads + t;
     const UfInst& I = a.uf[i];
     if (pix < ufd::uf_batch_work(I)) ufd::uf_batch_item(I, pix, a.uf_tabs, a.uf_waves, a.Uf);
@@ -1201,12 +1218,12 @@ int series_plan_launch_waves(bimsim_ctx* ctx, const SeriesPlan& P, const double*
     const dim3 wgrid((P.nk_max + 255) / 256, std::min(P.n_sph, 65535));
     if (P.harmonic) {
         // per-wave Legendre values, azimuth phases and wave weights (and the
-        // counters cleared), then the records from them
+        // counters cleared), and the row form's records from them
         const dim3 lgrid((P.nk_max + 63) / 64, std::min(P.n_inst, 65535), P.max_lh);
         hipLaunchKernelGGL(harm_legendre_kernel, lgrid, dim3(64), 0, st, P.d_inst, P.d_sph,
                            P.n_inst, waves, P.d_h64, P.d_pl, P.d_e, P.d_phi, P.d_counters,
                            P.n_counters);
-        if ((long long)P.max_lh * P.n_inst >= 2LL * ctx->cu_count) {
+        if (!series_few_rows(ctx, P)) {
             // one block per (row, instance) over all its spheres
             const dim3 rgrid(P.max_lh, std::min(P.n_inst, 65535));
             if (P.max_rec_combos <= 2 * kRecPer * 64) {
@@ -1220,13 +1237,6 @@ int series_plan_launch_waves(bimsim_ctx* ctx, const SeriesPlan& P, const double*
                                    dim3(kRecThreads), T.lds, st, P.d_inst, P.d_sph, P.n_inst,
                                    P.d_pl, P.d_e, P.d_phi, P.d_h64, P.d_rec, T.tl, T.ts);
             }
-        } else {
-            // few instances: blocks per (row, four records, sphere)
-            const dim3 rgrid(P.max_tl, (P.max_tl + kRecTile - 1) / kRecTile,
-                             std::min(P.n_sph, 65535));
-            hipLaunchKernelGGL(harm_records_tile_kernel, rgrid, dim3(kRecThreads), 0, st,
-                               P.d_inst, P.d_sph, P.n_sph, P.d_pl, P.d_e, P.d_phi, P.d_h64,
-                               P.d_rec);
         }
     } else {
         hipLaunchKernelGGL(series_waves_kernel, wgrid, dim3(256), 0, st, P.d_inst, P.d_sph, P.n_sph,
@@ -1236,45 +1246,57 @@ int series_plan_launch_waves(bimsim_ctx* ctx, const SeriesPlan& P, const double*
     return BIMSIM_OK;
 }
 
+bool series_few_rows(const bimsim_ctx* ctx, const SeriesPlan& P) {
+    return (long long)P.max_lh * P.n_inst < 2LL * ctx->cu_count;
+}
+
 size_t prepass_lds(const PrepassArgs& a) {
-    return sizeof(mie::zc) * 8 * (size_t)a.wstride * (size_t)std::min(a.spb, a.n_mie_sph);
+    return sizeof(double) * (size_t)mie::mie_closed_doubles(a.wstride) *
+           std::min(mie::kClosedSph, a.n_mie_sph);
 }
 
 int series_plan_launch_prepass(bimsim_ctx* ctx, const SeriesPlan& P, const double* waves,
                                const PrepassArgs& a) {
     if (!P.harmonic || P.n_inst == 0 || P.n_sph == 0 || a.n_mie_sph <= 0 || a.n_uf <= 0 ||
-        a.spb < 1 || a.spb > mie::kSphPerLaunch || a.uf_blocks < 1 || prepass_lds(a) > kPrepassLds)
+        a.uf_blocks < 1 || prepass_lds(a) > kPrepassLds)
         return set_error(ctx, BIMSIM_E_INVALID, "pre-pass launch outside its limits");
     const hipStream_t st = ctx->stream;
-    const dim3 lgrid((P.nk_max + 63) / 64, std::min(P.n_inst, 65535), P.max_lh);
-    hipLaunchKernelGGL(harm_legendre_kernel, lgrid, dim3(64), 0, st, P.d_inst, P.d_sph, P.n_inst,
-                       waves, P.d_h64, P.d_pl, P.d_e, P.d_phi, P.d_counters, P.n_counters);
-    const int n_mie = (a.n_mie_sph + a.spb - 1) / a.spb;
-    const int tiles = (P.max_tl + kRecTile - 1) / kRecTile;
-    const long long n_rec = (long long)P.max_tl * tiles * P.n_sph;
-    const long long total = n_mie + n_rec + (long long)a.uf_blocks * a.n_uf;
+    const int n_mie = (a.n_mie_sph + mie::kClosedSph - 1) / mie::kClosedSph;
+    const int leg_w = (P.nk_max + kRecThreads - 1) / kRecThreads;
+    const long long n_leg = (long long)leg_w * P.n_inst * P.max_lh;
+    const long long total = n_mie + n_leg + (long long)a.uf_blocks * a.n_uf;
     if (total > INT_MAX)
         return set_error(ctx, BIMSIM_E_INVALID, "pre-pass launch outside its limits");
     hipLaunchKernelGGL(prepass_kernel, dim3((unsigned)total), dim3(kRecThreads), prepass_lds(a), st,
-                       a, n_mie, (int)n_rec, P.max_tl, tiles, P.d_inst, P.d_sph, P.n_sph, P.d_pl,
-                       P.d_e, P.d_phi, P.d_h64, P.d_rec);
+                       a, n_mie, (int)n_leg, leg_w, P.n_inst, P.d_inst, P.d_sph, waves, P.d_h64,
+                       P.d_pl, P.d_e, P.d_phi, P.d_counters, P.n_counters);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
 }
 
 namespace {
 
-// One bucket's persistent launch (the counter must be zero).
-// The coefficients into the records (harm_fold_kernel).
-int fold_launch(bimsim_ctx* ctx, const SeriesPlan& P, const double2* A, const double2* B) {
-    const dim3 grid((P.max_tl * P.max_tl / 2 + kRecThreads - 1) / kRecThreads,
-                    std::min(P.n_sph, 65535));
-    hipLaunchKernelGGL(harm_fold_kernel, grid, dim3(kRecThreads), 0, ctx->stream, P.d_sph,
-                       P.n_sph, A, B, P.d_rec, P.d_rec_in);
+// The records times the coefficients: the tile form's from the wave tables,
+// the row form's from its plain records.
+int records_launch(bimsim_ctx* ctx, const SeriesPlan& P, const double2* A, const double2* B) {
+    const hipStream_t st = ctx->stream;
+    if (series_few_rows(ctx, P)) {
+        // few instances: blocks per (row, four records, sphere)
+        const dim3 rgrid(P.max_tl, (P.max_tl + kRecTile - 1) / kRecTile, std::min(P.n_sph, 65535));
+        hipLaunchKernelGGL(harm_records_tile_kernel, rgrid, dim3(kRecThreads), 0, st, P.d_inst,
+                           P.d_sph, P.n_sph, P.d_pl, P.d_e, P.d_phi, P.d_h64, A, B, P.d_rec,
+                           P.d_rec_in);
+    } else {
+        const dim3 grid((P.max_tl * P.max_tl / 2 + kRecThreads - 1) / kRecThreads,
+                        std::min(P.n_sph, 65535));
+        hipLaunchKernelGGL(harm_fold_kernel, grid, dim3(kRecThreads), 0, st, P.d_sph, P.n_sph, A,
+                           B, P.d_rec, P.d_rec_in);
+    }
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
 }
 
+// One bucket's persistent launch (the counter must be zero).
 int launch_one_bucket(bimsim_ctx* ctx, const SeriesPlan& P, const SeriesPlan::Bucket& K,
                       const double2* A, const double2* B, float2* U) {
     const hipStream_t st = ctx->stream;
@@ -1313,14 +1335,14 @@ int launch_one_bucket(bimsim_ctx* ctx, const SeriesPlan& P, const SeriesPlan::Bu
 }  // namespace
 
 int series_plan_launch_sums(bimsim_ctx* ctx, const SeriesPlan& P, const double2* A,
-                            const double2* B, float2* U, hipEvent_t after_fold) {
+                            const double2* B, float2* U, hipEvent_t after_records) {
     const hipStream_t st = ctx->stream;
     if (P.n_inst == 0 || P.n_sph == 0) {
-        if (after_fold) BIMSIM_HIP_CHECK(ctx, hipStreamWaitEvent(st, after_fold, 0));
+        if (after_records) BIMSIM_HIP_CHECK(ctx, hipStreamWaitEvent(st, after_records, 0));
         return BIMSIM_OK;
     }
-    if (P.harmonic) BIMSIM_TRY(fold_launch(ctx, P, A, B));
-    if (after_fold) BIMSIM_HIP_CHECK(ctx, hipStreamWaitEvent(st, after_fold, 0));
+    if (P.harmonic) BIMSIM_TRY(records_launch(ctx, P, A, B));
+    if (after_records) BIMSIM_HIP_CHECK(ctx, hipStreamWaitEvent(st, after_records, 0));
     for (const SeriesPlan::Chunk& ch : P.chunks) {
         if (!P.harmonic) {
             const dim3 cgrid((P.max_npix + kThreads - 1) / kThreads, std::min(ch.sph_count, 65535));
@@ -1396,7 +1418,7 @@ int harm_tune(bimsim_ctx* ctx, const std::string& shape, const double* waves, co
     ctx->timing = false;
     int rc = zero_launch(ctx, tmp, sizeof(float2) * (size_t)std::max<long long>(1, field));
     if (rc == BIMSIM_OK) rc = series_plan_launch_waves(ctx, *P, waves);
-    if (rc == BIMSIM_OK) rc = fold_launch(ctx, *P, A, B);
+    if (rc == BIMSIM_OK) rc = records_launch(ctx, *P, A, B);
     std::vector<int> chosen;
     for (SeriesPlan::Bucket* K : bks) {
         if (rc != BIMSIM_OK) break;
