@@ -764,7 +764,7 @@ __device__ __forceinline__ void quad_chunks(__amdgpu_buffer_rsrc_t rs, const int
     }
 }
 
-// Per-pixel harmonic sum, persistent over (instance, pixel block) items.
+// Harmonic sum per pixel, node or near-tile pixel, persistent over the items.
 // Row m of the order sums runs the scaled recurrence
 //   q_mm = Pn_mm,  q_lm = 2x q_{l-1,m} - c_lm q_{l-2,m}
 // (Pn_lm = K_lm q_lm, K_lm = prod_{j=m+1..l} a_jm / 2, folded into the
@@ -785,8 +785,8 @@ __global__ __launch_bounds__(kHarmThreads, kWaves) void series_harm_kernel(
     const SeriesInst* __restrict__ insts, const SeriesSph* __restrict__ sph,
     const SeriesGroup* __restrict__ grps, const SeriesItem* __restrict__ items, int n_items,
     const float4* __restrict__ rec, const float4* __restrict__ rec_in,
-    const float* __restrict__ cst, const int* __restrict__ perm, float2* __restrict__ U,
-    int* __restrict__ counter) {
+    const float* __restrict__ cst, const int* __restrict__ perm, HarmNodes nodes,
+    float2* __restrict__ U, int* __restrict__ counter) {
     static_assert(!kMfma || (kPlanar && kChunk > 0), "matrix-core sums: planar chunks only");
     __shared__ int s_item;
     int qoff[QuadRegs<L, (kChunk > 0 ? kChunk : 4)>::NR];
@@ -803,25 +803,67 @@ __global__ __launch_bounds__(kHarmThreads, kWaves) void series_harm_kernel(
         if (it >= n_items) break;
         const SeriesItem item = items[it];
         const SeriesInst& I = insts[item.inst];
-        const int npix = I.uR * I.vR;
-        const int j0 = item.pix0 + (int)threadIdx.x;
-        // lanes past the instance's pixels repeat its last one and store
+        const int kind = item.split & (kItemAdd - 1);
+        // lanes past the instance's points repeat its last one and store
         // nothing: every lane stays active (the matrix-core sums broadcast
         // record operands from lanes of the wave)
-        const bool live = j0 < npix;
-        const int j = live ? j0 : npix - 1;
-        // pixels in the instance's order of uniform waves (inside each
-        // sphere, then outside every sphere), so that a wave takes one
-        // radial path
-        const int pix = I.perm_off >= 0 ? perm[I.perm_off + j] : j;
-        const int iv = pix / I.uR, iu = pix - iv * I.uR;
-        const d3 p = quad_at(I.q, (double)iu / (double)I.uR, (double)iv / (double)I.vR);
+        bool live;
+        int pix;        // where the result goes, within the instance's values
+        double u, v;    // the point, in edges of the slice
+        // the spheres wanted at the wave's tile (a wave holds points of one)
+        const unsigned long long* __restrict__ want = nullptr;
+        if (kind == kItemPixels) {
+            const int npix = I.uR * I.vR;
+            const int j0 = item.pix0 + (int)threadIdx.x;
+            live = j0 < npix;
+            const int j = live ? j0 : npix - 1;
+            // pixels in the instance's order of uniform waves (inside each
+            // sphere, then outside every sphere), so that a wave takes one
+            // radial path
+            pix = I.perm_off >= 0 ? perm[I.perm_off + j] : j;
+            const int iv = pix / I.uR, iu = pix - iv * I.uR;
+            u = (double)iu / (double)I.uR;
+            v = (double)iv / (double)I.vR;
+        } else {
+            const NodeInst& N = nodes.inst[item.inst];
+            int tile;
+            if (kind == kItemNodes) {
+                const int w0 = __builtin_amdgcn_readfirstlane(item.pix0 + ((int)threadIdx.x >> 6));
+                const int w = min(w0, N.n_waves - 1);
+                int l = 0;
+                while (l + 1 < N.n_lev && w >= N.lev[l + 1].wave0) ++l;
+                const NodeLevel& Lv = N.lev[l];
+                const int q = Lv.q, t = (w - Lv.wave0) / Lv.wpt;
+                const int e0 = 64 * (w - Lv.wave0 - t * Lv.wpt) + ((int)threadIdx.x & 63);
+                live = w0 == w && e0 < q * q;
+                const int e = min(e0, q * q - 1), b = e / q, a = e - b * q;
+                pix = Lv.node0 + t * q * q + e;
+                tile = Lv.tile0 + t;
+                const int2 t0 = nodes.tiles[tile];
+                u = ((double)t0.x + nodes.X[Lv.x0 + a]) / (double)I.uR;
+                v = ((double)t0.y + nodes.X[Lv.x0 + b]) / (double)I.vR;
+            } else {
+                tile = N.near0 + item.pix0;
+                const int2 t0 = nodes.tiles[tile];
+                const int iu = t0.x + ((int)threadIdx.x & 15), iv = t0.y + ((int)threadIdx.x >> 4);
+                live = iu < I.uR && iv < I.vR;
+                pix = item.pix0 * kHarmThreads + (int)threadIdx.x;
+                u = (double)min(iu, I.uR - 1) / (double)I.uR;
+                v = (double)min(iv, I.vR - 1) / (double)I.vR;
+            }
+            want = nodes.mask + N.mask0 + (long long)(tile - N.tile_first) * N.words;
+        }
+        const d3 p = quad_at(I.q, u, v);
         const SeriesGroup G = grps[item.grp];
         const double inv_kmag = 1.0 / I.kmag;
         float acc_r = 0.f, acc_i = 0.f;
         for (int s = G.s_begin; s < G.s_begin + G.ns; ++s) {
             const SeriesSph& SS = sph[s];
             const SphereDev S = SS.s;
+            if (kind != kItemPixels) {
+                const int b = s - I.s_begin;
+                if (((want[b >> 6] >> (b & 63)) & 1) == 0) continue;
+            }
             const int nl1 = S.Nl + 1;
             d3 r = sub(p, mk(S.p));
             double d, inv_d;
@@ -952,8 +994,14 @@ __global__ __launch_bounds__(kHarmThreads, kWaves) void series_harm_kernel(
         }
         if (live) {
             float2* o = U + I.u_off + pix;
+            bool add = G.accumulate != 0;
+            if (kind != kItemPixels) {
+                const NodeInst& N = nodes.inst[item.inst];
+                o = kind == kItemNodes ? nodes.V + N.v0 + pix : nodes.W + N.w0 + pix;
+                add = (item.split & kItemAdd) != 0;
+            }
             float2 v = make_float2(0.f, 0.f);
-            if (G.accumulate) v = *o;
+            if (add) v = *o;
             *o = make_float2(v.x + acc_r, v.y + acc_i);
         }
     }

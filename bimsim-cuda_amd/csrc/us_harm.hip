@@ -20,11 +20,11 @@ void launch_variant(const HarmLaunch& a) {
     if (a.planar)
         hipLaunchKernelGGL((harm::series_harm_kernel<L, true, W, 0>), a.grid,
                            dim3(harm::kHarmThreads), 0, a.stream, a.inst, a.sph, a.grp, a.items,
-                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.U, a.counter);
+                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.nodes, a.U, a.counter);
     else
         hipLaunchKernelGGL((harm::series_harm_kernel<L, false, W, 0>), a.grid,
                            dim3(harm::kHarmThreads), 0, a.stream, a.inst, a.sph, a.grp, a.items,
-                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.U, a.counter);
+                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.nodes, a.U, a.counter);
 }
 
 #else
@@ -36,7 +36,7 @@ int launch_chunked(const HarmLaunch& a) {
         if (!a.planar) return -1;
         hipLaunchKernelGGL((harm::series_harm_kernel<L, true, W, C, kMfma>), a.grid,
                            dim3(harm::kHarmThreads), 0, a.stream, a.inst, a.sph, a.grp, a.items,
-                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.U, a.counter);
+                           a.n_items, a.rec, a.rec_in, a.cst, a.perm, a.nodes, a.U, a.counter);
         return 0;
     }
     return -1;

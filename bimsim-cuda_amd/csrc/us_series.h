@@ -54,11 +54,49 @@ struct SeriesSph {
     int tl;             // harmonic form: record stride (its order bucket)
     int planar;         // harmonic form: the slice contains the centre and is normal
                         // to z, so every pixel has x = r-hat.z = 0
+    int reach;          // the caller's bound on the orders whose cut j_l shows outside the
+                        // sphere (us_nodes.h), or 0: Nl
 };
 
+// A work item: 256 pixels of an instance from pix0 (and one of its wave
+// splits), or in the harmonic form the waves of its nodes from wave pix0, or
+// its near tile pix0 (us_nodes.h).
 struct SeriesItem {
-    int inst, pix0, split;
+    int inst, pix0, split;   // harmonic form: split = kind, plus kItemAdd to add to the nodes' or
+                             // the tile's values
     int grp;            // harmonic form: its sphere group
+};
+enum { kItemPixels = 0, kItemNodes = 1, kItemNear = 2, kItemAdd = 4 };
+
+// One tile size of an instance's nodes (us_nodes.h): T pixels and q nodes per
+// edge, tiles [tile0, tile0 + n_tiles) of the plan's tile table, q x q nodes
+// each from node0 of the instance, evaluated by wpt waves each from wave0 of
+// the instance, the grid of tile numbers (gw per row, -1:
+// none) at idx0, the interpolation matrix [q][T] at e0, the node positions at
+// x0.
+struct NodeLevel {
+    int T, q, tile0, n_tiles, node0, wave0, wpt, gw, e0, x0;
+    long long idx0;
+};
+// An instance's nodes: tiles of words mask words each from tile_first (mask
+// at mask0), its node values at v0, its near tiles [near0, near0 + n_near)
+// with their values at w0.  n_lev = 0: none, its pixels are items.
+struct NodeInst {
+    int n_lev, words, n_nodes, n_waves, tile_first;
+    int near0, n_near, near_gw;
+    long long near_idx0, mask0, v0, w0;
+    NodeLevel lev[4];
+};
+// The plan's node tables as the kernels take them.
+struct HarmNodes {
+    const NodeInst* inst;
+    const int2* tiles;
+    const unsigned long long* mask;
+    const int* idx;
+    const float* E;
+    const double* X;
+    float2* V;
+    float2* W;
 };
 
 // Harmonic form: the spheres of one instance in one order bucket, a
@@ -125,6 +163,7 @@ struct HarmLaunch {
     const float4* rec_in;   // records times A_l
     const float* cst;
     const int* perm;
+    HarmNodes nodes;
     float2* U;
     int* counter;
     int planar;   // every sphere of the bucket's groups is planar
@@ -251,6 +290,9 @@ struct SeriesPlan {
     int* d_perm = nullptr;        // pixel orders of the instances with perm_off >= 0
     SeriesGroup* d_grp = nullptr; // sphere groups of the harmonic form
     double* d_h64 = nullptr;      // FP64 Legendre constants and scales of the wave sums
+    HarmNodes nodes{};            // node tables (null where no instance has nodes)
+    int4* d_xblocks = nullptr;    // 64 x 64 pixel blocks of the instances with nodes
+    int n_xblocks = 0;
 };
 
 // Chooses splits and chunks, builds and uploads the tables and allocates

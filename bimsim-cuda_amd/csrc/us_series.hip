@@ -24,7 +24,7 @@
 #include "mie_device.h"
 #include "refmath.h"
 #include "uf_device.h"
-#include "us_series.h"
+#include "us_nodes.h"
 
 namespace bimsim {
 namespace {
@@ -32,6 +32,8 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kW = 2;   // waves in flight per thread
 constexpr int kBuckets[] = {16, 24, 32, 40, 48, 64, 80, 96, 112};
+// Waves of pixels per CU up to which a harmonic plan takes one bucket.
+constexpr long long kOneBucketWaves = 16;
 
 __device__ inline dc ld2(const double2* p, int i) {
     const double2 v = p[i];
@@ -867,7 +869,10 @@ void series_plan_destroy(SeriesPlan* P) {
     (void)hipFree(P->d_part);
     (void)hipFree(P->d_coef);
     (void)hipFree(P->d_rhat);
-    void* harm[] = {P->d_pl, P->d_e, P->d_phi, P->d_rec, P->d_rec_in, P->d_cst, P->d_h64};
+    void* harm[] = {P->d_pl, P->d_e, P->d_phi, P->d_rec, P->d_rec_in, P->d_cst, P->d_h64,
+                    P->d_xblocks, (void*)P->nodes.inst, (void*)P->nodes.tiles,
+                    (void*)P->nodes.mask, (void*)P->nodes.idx, (void*)P->nodes.E,
+                    (void*)P->nodes.X, P->nodes.V, P->nodes.W};
     for (void* q : harm) (void)hipFree(q);
     *P = SeriesPlan();
 }
@@ -876,6 +881,37 @@ void series_plan_destroy(SeriesPlan* P) {
 // = 0 and A.z = c.z have r.z = 0 exactly, so x = 0 at every pixel.
 static bool harm_planar(const QuadArg& q, const SphereDev& S) {
     return q.X.z == 0.0 && q.Y.z == 0.0 && q.A.z == S.p[2];
+}
+
+// The items of instance i's sphere group g (spheres [s0, s0 + ns) of the
+// instance): its near tiles that have one of them, and the waves of nodes
+// that do, four to an item (for the instance's first group every one, whose
+// nodes it writes; later groups add, as near tiles of an earlier group are
+// added to).
+static void node_items(const NodeTables& nt, int i, int g, int s0, int ns, bool first,
+                       std::vector<char>* near_done, std::vector<SeriesItem>* items) {
+    const NodeInst& N = nt.inst[i];
+    const unsigned long long* mask = nt.mask.data() + N.mask0;
+    auto wants = [&](int tile) {
+        return node_mask_any(mask + (long long)(tile - N.tile_first) * N.words, s0, ns);
+    };
+    near_done->resize(N.n_near, 0);
+    for (int t = 0; t < N.n_near; ++t) {
+        if (!wants(N.near0 + t)) continue;
+        items->push_back(SeriesItem{i, t, kItemNear | ((*near_done)[t] ? kItemAdd : 0), g});
+        (*near_done)[t] = 1;
+    }
+    constexpr int kW4 = kThreads / 64;   // waves of an item
+    for (int w0 = 0; w0 < N.n_waves; w0 += kW4) {
+        bool any = first;
+        for (int l = 0; l < N.n_lev && !any; ++l) {
+            const NodeLevel& L = N.lev[l];
+            const int lo = std::max(w0, L.wave0) - L.wave0;
+            const int hi = std::min(w0 + kW4, L.wave0 + L.n_tiles * L.wpt) - L.wave0;
+            for (int w = lo; w < hi && !any; ++w) any = wants(L.tile0 + w / L.wpt);
+        }
+        if (any) items->push_back(SeriesItem{i, w0, kItemNodes | (first ? 0 : kItemAdd), g});
+    }
 }
 
 int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, SeriesPlan* P,
@@ -920,14 +956,26 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     for (const SeriesInst& I : batch.inst) min_nk = std::min(min_nk, I.nk);
     P->harmonic = ctx->series_algo == kSeriesHarmonic ||
                   (ctx->series_algo == kSeriesAuto && min_nk >= 16);
+    // a plan of few waves is bound by the latency of its launches, one per
+    // order bucket: its spheres all take the largest one's (its kernel skips
+    // the orders a sphere lacks)
+    int one_bucket = 0;
     if (P->harmonic) {
         split_mult = 1;
+        const int top = *std::max_element(bucket.begin(), bucket.end());
+        if ((blocks_all + 0LL) * (kThreads / 64) <= kOneBucketWaves * ctx->cu_count && top <= 64)
+            one_bucket = top;
+    }
+    auto order_bucket = [&](const SeriesSph& S) {
+        return one_bucket > 0 ? one_bucket : series_capacity(S.s.Nl + 1);
+    };
+    if (P->harmonic) {
         // each instance's spheres sorted by their own order bucket, so that
         // a bucket's spheres form one consecutive group per instance
         for (const SeriesInst& I : batch.inst)
             std::stable_sort(batch.sph.begin() + I.s_begin, batch.sph.begin() + I.s_begin + I.ns,
-                             [](const SeriesSph& a, const SeriesSph& b) {
-                                 return series_capacity(a.s.Nl + 1) < series_capacity(b.s.Nl + 1);
+                             [&](const SeriesSph& a, const SeriesSph& b) {
+                                 return order_bucket(a) < order_bucket(b);
                              });
     }
     // harmonic form: the sphere groups of each instance, in bucket order
@@ -937,14 +985,27 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
         for (int i = 0; i < ni; ++i) {
             const SeriesInst& I = batch.inst[i];
             for (int s = I.s_begin; s < I.s_begin + I.ns;) {
-                const int L = series_capacity(batch.sph[s].s.Nl + 1);
+                const int L = order_bucket(batch.sph[s]);
                 int e = s + 1;
-                while (e < I.s_begin + I.ns && series_capacity(batch.sph[e].s.Nl + 1) == L) ++e;
+                while (e < I.s_begin + I.ns && order_bucket(batch.sph[e]) == L) ++e;
                 inst_groups[i].push_back((int)groups.size());
                 groups.push_back(SeriesGroup{s, e - s,
                                              inst_groups[i].size() == 1 ? I.accumulate : 1, L});
                 s = e;
             }
+        }
+    }
+    // harmonic form: the nodes of the instances they pay for
+    NodeTables nt;
+    bool any_nodes = false;
+    if (P->harmonic) {
+        for (const SeriesInst& I : batch.inst) {
+            node_plan_instance(I, batch.sph.data() + I.s_begin, &nt);
+            any_nodes = any_nodes || nt.inst.back().n_lev > 0;
+        }
+        if (nt.n_v + nt.n_w >= (1LL << 31) || !any_nodes) {   // (node numbers are ints)
+            any_nodes = false;
+            nt = NodeTables();
         }
     }
     // split the waves until the queue holds several items per CU (each
@@ -987,6 +1048,7 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     P->n_part = poff;
     // chunks of whole instances within the coefficient budget
     std::vector<SeriesItem> items;
+    std::vector<std::vector<char>> near_done(ni);   // near tiles an earlier group writes
     int i0 = 0;
     while (i0 < ni) {
         long long celems = 0, relems = 0;
@@ -1028,8 +1090,12 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
                         if (G.L != L) continue;
                         for (int t = G.s_begin; t < G.s_begin + G.ns; ++t)
                             if (!harm_planar(I.q, batch.sph[t].s)) all_planar = 0;
-                        for (int p0 = 0; p0 < npix; p0 += kThreads)
-                            items.push_back(SeriesItem{i, p0, 0, g});
+                        if (any_nodes && nt.inst[i].n_lev > 0)
+                            node_items(nt, i, g, G.s_begin - I.s_begin, G.ns,
+                                       g == inst_groups[i][0], &near_done[i], &items);
+                        else
+                            for (int p0 = 0; p0 < npix; p0 += kThreads)
+                                items.push_back(SeriesItem{i, p0, kItemPixels, g});
                     }
                     continue;
                 }
@@ -1077,7 +1143,7 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
         for (int t = 0; t < P->n_sph; ++t) {
             SeriesSph& S = batch.sph[t];
             const SeriesInst& I = batch.inst[S.inst];
-            S.tl = series_capacity(S.s.Nl + 1);
+            S.tl = order_bucket(S);
             P->max_tl = std::max(P->max_tl, S.tl);
             S.planar = harm_planar(I.q, S.s) ? 1 : 0;
             S.toff = nrec;
@@ -1130,13 +1196,18 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     for (SeriesInst& I : batch.inst) I.perm_off = -1;
     if (P->harmonic) {
         long long npx = 0, tests = 0;
-        for (const SeriesInst& I : batch.inst) {
+        auto has_nodes = [&](size_t i) { return any_nodes && nt.inst[i].n_lev > 0; };
+        for (size_t i = 0; i < batch.inst.size(); ++i) {
+            if (has_nodes(i)) continue;
+            const SeriesInst& I = batch.inst[i];
             npx += (long long)I.uR * I.vR;
             tests += (long long)I.uR * I.vR * I.ns;
         }
         if (npx <= kPermMaxPixels && tests <= kPermMaxTests) {
             std::vector<int> cls, start;
-            for (SeriesInst& I : batch.inst) {
+            for (size_t i = 0; i < batch.inst.size(); ++i) {
+                if (has_nodes(i)) continue;
+                SeriesInst& I = batch.inst[i];
                 const int npix = I.uR * I.vR;
                 cls.assign(npix, 0);
                 bool any = false;
@@ -1184,6 +1255,34 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
          (rc = alloc(ctx, &P->d_rec_in, P->n_rec)) != BIMSIM_OK)) {
         series_plan_destroy(P);
         return rc;
+    }
+    if (any_nodes) {
+        NodeInst* d_ninst = nullptr;
+        int2* d_tiles = nullptr;
+        unsigned long long* d_mask = nullptr;
+        int* d_idx = nullptr;
+        float* d_E = nullptr;
+        double* d_X = nullptr;
+        rc = upload(ctx, &d_ninst, nt.inst);
+        P->nodes.inst = d_ninst;
+        if (rc == BIMSIM_OK) rc = upload(ctx, &d_tiles, nt.tiles);
+        P->nodes.tiles = d_tiles;
+        if (rc == BIMSIM_OK) rc = upload(ctx, &d_mask, nt.mask);
+        P->nodes.mask = d_mask;
+        if (rc == BIMSIM_OK) rc = upload(ctx, &d_idx, nt.idx);
+        P->nodes.idx = d_idx;
+        if (rc == BIMSIM_OK) rc = upload(ctx, &d_E, nt.E);
+        P->nodes.E = d_E;
+        if (rc == BIMSIM_OK) rc = upload(ctx, &d_X, nt.X);
+        P->nodes.X = d_X;
+        if (rc == BIMSIM_OK) rc = alloc(ctx, &P->nodes.V, nt.n_v);
+        if (rc == BIMSIM_OK) rc = alloc(ctx, &P->nodes.W, nt.n_w);
+        if (rc == BIMSIM_OK) rc = upload(ctx, &P->d_xblocks, nt.blocks);
+        if (rc != BIMSIM_OK) {
+            series_plan_destroy(P);
+            return rc;
+        }
+        P->n_xblocks = (int)nt.blocks.size();
     }
     // the records kernel writes only the records the spheres use: the rest
     // of each table stays zero, as the pixel kernel's blocks may read past Nl
@@ -1303,7 +1402,7 @@ int launch_one_bucket(bimsim_ctx* ctx, const SeriesPlan& P, const SeriesPlan::Bu
     // resident workgroups: the queue keeps them busy until it drains
     const dim3 grid(std::min(K.item_count, P.groups_per_cu * ctx->cu_count));
     const HarmLaunch hl{grid, st, P.d_inst, P.d_sph, P.d_grp, P.d_items + K.item_begin,
-                        K.item_count, P.d_rec, P.d_rec_in, P.d_cst, P.d_perm, U,
+                        K.item_count, P.d_rec, P.d_rec_in, P.d_cst, P.d_perm, P.nodes, U,
                         P.d_counters + K.counter, K.planar};
     int hv = 0;
     switch (K.L) {
@@ -1352,6 +1451,7 @@ int series_plan_launch_sums(bimsim_ctx* ctx, const SeriesPlan& P, const double2*
         }
         const int tmr = timer_begin(ctx, kStageSeries);
         for (const SeriesPlan::Bucket& K : ch.buckets) BIMSIM_TRY(launch_one_bucket(ctx, P, K, A, B, U));
+        if (P.harmonic) BIMSIM_TRY(node_expand_launch(ctx, P, U));
         timer_end(ctx, tmr);
     }
     if (!P.split_insts.empty()) {
