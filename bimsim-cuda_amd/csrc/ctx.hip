@@ -43,6 +43,25 @@ int scratch_get(bimsim_ctx* ctx, int slot, size_t bytes, void** out) {
     return BIMSIM_OK;
 }
 
+void* scratch_try(bimsim_ctx* ctx, int slot, size_t bytes) {
+    auto& s = ctx->scratch[slot];
+    if (s.second < bytes) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        (void)hipStreamIsCapturing(ctx->stream, &cap);
+        if (cap != hipStreamCaptureStatusNone) return nullptr;
+        const size_t want = bytes + bytes / 8 + 256;
+        void* ptr = nullptr;
+        if (hipMalloc(&ptr, want) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (s.first) ctx->scratch_retired.push_back(s.first);
+        s.first = ptr;
+        s.second = want;
+    }
+    return s.first;
+}
+
 namespace {
 
 template <class T>

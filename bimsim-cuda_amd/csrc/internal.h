@@ -53,7 +53,7 @@ namespace bimsim {
 
 enum ScratchSlot {
     kSlotCoef = 0,    // per-pixel series coefficients
-    kSlotRhat = 1,    // per-pixel unit vectors
+    kSlotSums = 1,    // FP64 scattered field: sums of single spheres
     kSlotWaves = 2,   // per-sphere wave tables
     kSlotSph = 3,     // device sphere records
     kSlotPartial = 4, // split partial sums
@@ -70,6 +70,10 @@ int set_error(bimsim_ctx* ctx, int code, const char* fmt, ...);
 // Device scratch of at least `bytes` in `slot` (grown with hipMalloc; an
 // outgrown buffer stays allocated until the context ends).
 int scratch_get(bimsim_ctx* ctx, int slot, size_t bytes, void** out);
+
+// The same for a caller that can do without: null where the memory is not
+// there, or would have to be allocated while the context's stream is captured.
+void* scratch_try(bimsim_ctx* ctx, int slot, size_t bytes);
 
 // Device copy of an int table (cached by content; uploaded once).
 int int_table_get(bimsim_ctx* ctx, const std::vector<int>& v, const int** out);

@@ -12,6 +12,7 @@ constexpr int kUsBatch = 32;
 
 struct UsSphereBatch {
     SphereDev s[kUsBatch];
+    int slot[kUsBatch];   // place of s[i] in the caller's order
 };
 
 // One Monte-Carlo wave as seen by the FP32 series kernel: 2*k (so that the
@@ -22,7 +23,7 @@ struct WaveF {
 };
 
 // The scattered field of an FP32 call whose orders exceed the FP32 series
-// kernels (Nl + 1 > 112): the hoisted FP64 form into context scratch, then
+// kernels (Nl + 1 > 112): the FP64 form into context scratch, then
 // U (+)= that field rounded to complex64.
 int us_wide_fp32(bimsim_ctx* ctx, const bimsim_quad* pos, int uR, int vR, const double focus[3],
                  double kmag, const bimsim_sphere* spheres, int ns, const void* A, const void* B,
