@@ -12,6 +12,7 @@
 // rotation).  Built with -ffp-contract=off.
 #include "geometry.h"
 #include "internal.h"
+#include "mie_device.h"
 #include "refmath.h"
 #include "zj_device.h"
 
@@ -117,27 +118,32 @@ __global__ __launch_bounds__(kThreads) void uf_lut_kernel(QuadArg q, int uR, int
 }
 
 // -------------------------------------------------------- sphere radial LUTs
+// Where a radial table holds (radius, order): p[row radius + col order].
+struct RadialOut {
+    double2* p;
+    long long row, col;
+};
+
 // h[ir][l] = (j_l, y_l)(k r), r in [max(a, dmin), dmax] over dR samples
 __global__ void hankel_lut_kernel(int nl, double kmag, double lo, double dr, int dR,
-                                  double* __restrict__ work, int wstride,
-                                  double2* __restrict__ h) {
+                                  double* __restrict__ work, int wstride, RadialOut h) {
     const int ir = blockIdx.x * blockDim.x + threadIdx.x;
     if (ir >= dR) return;
     const double r = ir * dr + lo;
     const double kr = kmag * r;
     double* j = work + (size_t)ir * 4 * wstride;
     zj::sph_jy_real(nl, kr, true, j, j + wstride, j + 2 * wstride, j + 3 * wstride);
-    for (int l = 0; l <= nl; ++l) h[(size_t)ir * (nl + 1) + l] = make_double2(j[l], j[wstride + l]);
+    for (int l = 0; l <= nl; ++l)
+        h.p[ir * h.row + l * h.col] = make_double2(j[l], j[wstride + l]);
 }
 
 // j[ir][l] = j_l(k n r), r = ir * a/(aR-1); r = 0 -> delta_l0
 __global__ void bessel_lut_kernel(int nl, double kmag, double nr, double ni, double a, int aR,
-                                  zj::zc* __restrict__ work, int wstride,
-                                  double2* __restrict__ jl) {
+                                  zj::zc* __restrict__ work, int wstride, RadialOut jl) {
     const int ir = blockIdx.x * blockDim.x + threadIdx.x;
     if (ir >= aR) return;
     if (ir == 0) {
-        for (int l = 0; l <= nl; ++l) jl[l] = make_double2(l == 0 ? 1.0 : 0.0, 0.0);
+        for (int l = 0; l <= nl; ++l) jl.p[l * jl.col] = make_double2(l == 0 ? 1.0 : 0.0, 0.0);
         return;
     }
     const double dr = a / (aR - 1);
@@ -146,44 +152,163 @@ __global__ void bessel_lut_kernel(int nl, double kmag, double nr, double ni, dou
     const zj::zc knr = {(kmag * nr) * r, (kmag * ni) * r};
     zj::zc* j = work + (size_t)ir * 4 * wstride;
     zj::sph_jy_cplx(nl, knr, true, j, j + wstride, j + 2 * wstride, j + 3 * wstride, false);
-    for (int l = 0; l <= nl; ++l) jl[(size_t)ir * (nl + 1) + l] = make_double2(j[l].r, j[l].i);
+    for (int l = 0; l <= nl; ++l)
+        jl.p[ir * jl.row + l * jl.col] = make_double2(j[l].r, j[l].i);
 }
 
-// L[it][ir] = sum_l C_l rad[ir][l] P_l(cos(it * dtheta)) (sphere.cu:4-99)
+// Both radial tables where lut_closed_radii allows: j and y of the real
+// arguments and the complex j, a row of blocks each (blockIdx.y), one radius
+// a lane.  j runs down from mie_start_order and is scaled to sin z / z (or
+// order 1), y runs up from its closed form.  A lane's chain of two dependent
+// operations an order bounds it: 18 us for 2048 radii of 20 to 30 orders and
+// both tables, where two launches of the general form, whose arrays pass
+// through memory, took 65 and 48.
+__global__ __launch_bounds__(64) void lut_radial_kernel(int nl, double kmag, double lo, double dr,
+                                                        int dR, RadialOut h, double nr, double ni,
+                                                        double a, int aR, RadialOut jl) {
+    const int ir = blockIdx.x * 64 + threadIdx.x;
+    // j and y carry sqrt(3.14159 / pi) (the cylindrical functions' scaling)
+    const double quirk = sqrt(3.14159 / M_PI);
+    if (blockIdx.y == 2) {
+        if (ir >= aR) return;
+        double2* const o = jl.p + ir * jl.row;
+        if (ir == 0) {   // r = 0: delta_l0
+            for (int l = 0; l <= nl; ++l) o[l * jl.col] = make_double2(l == 0 ? 1.0 : 0.0, 0.0);
+            return;
+        }
+        // k*n*r as (k*n)*r with k*n scaling each component
+        const double r = ir * (a / (aR - 1));
+        const double zr = (kmag * nr) * r, zi = (kmag * ni) * r;
+        const double az2 = zr * zr + zi * zi, inv = 1.0 / az2;
+        const double ur = zr * inv, ui = -(zi * inv);
+        zj::zc j0, j1;
+        mie::sph_j01(zr, zi, ur, ui, &j0, &j1);
+        double fr = 1e-100, fi = 0.0, gr = 0.0, gi = 0.0;   // orders k + 1 and k + 2
+        const int top = mie::mie_start_order(nl, sqrt(az2));
+        double c = 2.0 * top + 3.0;
+        for (int k = top; k >= 0; --k) {
+            const double ar = c * ur, ai = c * ui;
+            const double hr = fma(ar, fr, fma(-ai, fi, -gr));
+            const double hi = fma(ar, fi, fma(ai, fr, -gi));
+            gr = fr;
+            gi = fi;
+            fr = hr;
+            fi = hi;
+            c -= 2.0;
+            if (k <= nl) o[k * jl.col] = make_double2(hr, hi);
+            if (fabs(fr) + fabs(fi) > 1e200) {   // small arguments, many orders
+                const double t = 1e-200;
+                fr *= t, fi *= t, gr *= t, gi *= t;
+                for (int l = k; l <= nl; ++l) {
+                    const double2 v = o[l * jl.col];
+                    o[l * jl.col] = make_double2(v.x * t, v.y * t);
+                }
+            }
+        }
+        const bool use0 = j0.r * j0.r + j0.i * j0.i > j1.r * j1.r + j1.i * j1.i;
+        const zj::zc sc = zj::zsc(quirk, use0 ? zj::zdiv(j0, zj::zc{fr, fi})
+                                              : zj::zdiv(j1, zj::zc{gr, gi}));
+#pragma unroll 4
+        for (int l = 0; l <= nl; ++l) {
+            const double2 v = o[l * jl.col];
+            const zj::zc w = zj::zmul(zj::zc{v.x, v.y}, sc);
+            o[l * jl.col] = make_double2(w.r, w.i);
+        }
+        return;
+    }
+    if (ir >= dR) return;
+    const double x = kmag * (ir * dr + lo), inv = 1.0 / x;
+    double* const o = (double*)(h.p + ir * h.row) + blockIdx.y;
+    const long long col = 2 * h.col;
+    double sn, cs;
+    sincos(x, &sn, &cs);
+    const double s0 = sn * inv, c0 = cs * inv;
+    if (blockIdx.y == 0) {
+        const double j1 = fma(s0, inv, -c0);
+        double f = 1e-100, g = 0.0;
+        const int top = mie::mie_start_order(nl, x);
+        double c = 2.0 * top + 3.0;
+        for (int k = top; k >= 0; --k) {
+            const double v = fma(c * inv, f, -g);
+            if (k <= nl) o[k * col] = v;
+            g = f;
+            f = v;
+            c -= 2.0;
+        }
+        const double sc = quirk * (fabs(s0) > fabs(j1) ? s0 / f : j1 / g);
+#pragma unroll 4
+        for (int l = 0; l <= nl; ++l) o[l * col] *= sc;
+    } else {
+        double g = -(quirk * c0), f = fma(g, inv, -(quirk * s0));
+        o[0] = g;
+        o[col] = f;
+        double c = 3.0;
+        for (int l = 2; l <= nl; ++l) {
+            const double v = fma(c * inv, f, -g);
+            o[l * col] = v;
+            g = f;
+            f = v;
+            c += 2.0;
+        }
+    }
+}
+
+// The radii (real arguments x_lo to x_hi, complex ones up to z_hi at steps of
+// z_lo) whose functions lut_radial_kernel forms: no order of j or y leaves the
+// range of a double (the orders belong to the smallest real argument) and
+// neither do sinh and cosh.
+static bool lut_closed_radii(int nl, double x0, double x1, double zr, double zi, int aR) {
+    const double lo = std::min(x0, x1), hi = std::max(x0, x1);
+    const double az = std::hypot(zr, zi);
+    return lo >= 1e-2 && hi <= 4096.0 && (double)nl <= lo + 4.05 * std::cbrt(lo) + 20.0 &&
+           zr >= 0.0 && az <= 4096.0 && std::fabs(zi) <= 100.0 && az >= 1e-8 * std::max(1, aR - 1);
+}
+
+// One table L[it][ir] = sum_l C_l rad(ir, l) P_l(cos(it * dtheta))
+// (sphere.cu:4-99) of nr radii.
 template <class Out>
-__global__ void lut_eval_kernel(int nl, const double2* __restrict__ C, const double2* __restrict__ rad,
-                                int nr, int thetaR, double dtheta, Out* __restrict__ L) {
+struct EvalTable {
+    const double2* C;
+    RadialOut rad;
+    int nr;
+    Out* L;
+};
+
+template <class Out>
+__global__ void lut_eval_kernel(int nl, EvalTable<Out> T, int thetaR, double dtheta) {
     const int ir = blockIdx.x * blockDim.x + threadIdx.x;
     const int it = blockIdx.y;
-    if (ir >= nr) return;
+    if (ir >= T.nr) return;
     const double theta = dtheta * it;
     const double ct = cos(theta);
     double P0 = 1.0, P1 = ct;
     dc acc = {0.0, 0.0};
     for (int l = 0; l <= nl; ++l) {
-        const dc h = ld(rad, (size_t)ir * (nl + 1) + l);
+        const dc h = ld(T.rad.p, ir * T.rad.row + l * T.rad.col);
         if (l == 0) {
-            acc = cadd(acc, cscl(cmul(ld(C, 0), h), P0));
+            acc = cadd(acc, cscl(cmul(ld(T.C, 0), h), P0));
         } else {
             if (l > 1) ref::shift_legendre(l, ct, P0, P1);
-            acc = cadd(acc, cscl(cmul(ld(C, l), h), P1));
+            acc = cadd(acc, cscl(cmul(ld(T.C, l), h), P1));
         }
     }
-    st(L, (size_t)it * nr + ir, acc);
+    st(T.L, (size_t)it * T.nr + ir, acc);
 }
 
-// lut_eval_kernel for kEvalRows angle rows per workgroup, with the same
-// operations in the same order (identical results): the rows' Legendre
-// values are computed once into LDS, and C_l rad[ir][l] once per (ir, l)
-// rather than once per (angle, ir, l).
+// lut_eval_kernel for kEvalRows angle rows per workgroup and two tables
+// (blockIdx.z), with the same operations in the same order (identical
+// results): the rows' Legendre values are computed once into LDS, and
+// C_l rad(ir, l) once per (ir, l) rather than once per (angle, ir, l).
 constexpr int kEvalRows = 16;
 constexpr int kEvalMaxOrders = 512;   // LDS: kEvalRows doubles per order
 
 template <class Out>
-__global__ __launch_bounds__(kThreads) void lut_eval_rows_kernel(
-    int nl, const double2* __restrict__ C, const double2* __restrict__ rad, int nr, int thetaR,
-    double dtheta, Out* __restrict__ L) {
+__global__ __launch_bounds__(kThreads) void lut_eval_rows_kernel(int nl, EvalTable<Out> T0,
+                                                                 EvalTable<Out> T1, int thetaR,
+                                                                 double dtheta) {
     extern __shared__ double Pl[];   // [l][row], (nl + 1) kEvalRows doubles
+    const EvalTable<Out>& T = blockIdx.z ? T1 : T0;
+    if ((int)blockIdx.x * kThreads >= T.nr) return;
     const int it0 = blockIdx.y * kEvalRows;
     if (threadIdx.x < kEvalRows) {
         const int r = threadIdx.x;
@@ -198,20 +323,20 @@ __global__ __launch_bounds__(kThreads) void lut_eval_rows_kernel(
     }
     __syncthreads();
     const int ir = blockIdx.x * kThreads + threadIdx.x;
-    if (ir >= nr) return;
+    if (ir >= T.nr) return;
     dc acc[kEvalRows];
 #pragma unroll
     for (int r = 0; r < kEvalRows; ++r) acc[r] = dc{0.0, 0.0};
-    const double2* h = rad + (size_t)ir * (nl + 1);
+    const double2* h = T.rad.p + ir * T.rad.row;
     for (int l = 0; l <= nl; ++l) {
-        const dc c = cmul(ld(C, l), ld(h, l));
+        const dc c = cmul(ld(T.C, l), ld(h, l * T.rad.col));
         const double* P = Pl + l * kEvalRows;
 #pragma unroll
         for (int r = 0; r < kEvalRows; ++r) acc[r] = cadd(acc[r], cscl(c, P[r]));
     }
 #pragma unroll
     for (int r = 0; r < kEvalRows; ++r)
-        if (it0 + r < thetaR) st(L, (size_t)(it0 + r) * nr + ir, acc[r]);
+        if (it0 + r < thetaR) st(T.L, (size_t)(it0 + r) * T.nr + ir, acc[r]);
 }
 
 // bilinear fetch with clamp addressing at data coordinates (x, y)
@@ -416,26 +541,54 @@ void sphere_lut_dims_host(const QuadArg& q, const bimsim_sphere& s, int R, int d
     *dR = dR_override > 0 ? dR_override : 2 * R;
 }
 
-// L[it][ir] = sum_l C_l rad[ir][l] P_l(cos(it dtheta)) for nr radii
-static int lut_eval_launch(bimsim_ctx* ctx, bool f32, int nl, const double2* C,
-                           const double2* rad, int nr, int thetaR, double dtheta, void* L) {
-    const unsigned gx = (unsigned)((nr + kThreads - 1) / kThreads);
+// The tables of both (or, with T1.nr = 0, of the first).
+template <class Out>
+static int lut_eval_launch(bimsim_ctx* ctx, int nl, const EvalTable<Out>& T0,
+                           const EvalTable<Out>& T1, int thetaR, double dtheta) {
+    const auto blocks = [](int nr) { return (unsigned)((nr + kThreads - 1) / kThreads); };
     if (nl + 1 <= kEvalMaxOrders) {
-        const dim3 grid(gx, (unsigned)((thetaR + kEvalRows - 1) / kEvalRows));
+        const dim3 grid(blocks(std::max(T0.nr, T1.nr)),
+                        (unsigned)((thetaR + kEvalRows - 1) / kEvalRows), T1.nr > 0 ? 2 : 1);
         const size_t lds = sizeof(double) * kEvalRows * (size_t)(nl + 1);
-        if (f32)
-            hipLaunchKernelGGL(lut_eval_rows_kernel<float2>, grid, dim3(kThreads), lds,
-                               ctx->stream, nl, C, rad, nr, thetaR, dtheta, (float2*)L);
-        else
-            hipLaunchKernelGGL(lut_eval_rows_kernel<double2>, grid, dim3(kThreads), lds,
-                               ctx->stream, nl, C, rad, nr, thetaR, dtheta, (double2*)L);
-    } else if (f32) {
-        hipLaunchKernelGGL(lut_eval_kernel<float2>, dim3(gx, thetaR), dim3(kThreads), 0,
-                           ctx->stream, nl, C, rad, nr, thetaR, dtheta, (float2*)L);
+        hipLaunchKernelGGL(lut_eval_rows_kernel<Out>, grid, dim3(kThreads), lds, ctx->stream, nl,
+                           T0, T1, thetaR, dtheta);
     } else {
-        hipLaunchKernelGGL(lut_eval_kernel<double2>, dim3(gx, thetaR), dim3(kThreads), 0,
-                           ctx->stream, nl, C, rad, nr, thetaR, dtheta, (double2*)L);
+        for (const EvalTable<Out>* T : {&T0, &T1})
+            if (T->nr > 0)
+                hipLaunchKernelGGL(lut_eval_kernel<Out>, dim3(blocks(T->nr), thetaR),
+                                   dim3(kThreads), 0, ctx->stream, nl, *T, thetaR, dtheta);
     }
+    BIMSIM_HIP_CHECK(ctx, hipGetLastError());
+    return BIMSIM_OK;
+}
+
+// The radial tables h (dR radii from max(a, dmin) to dmax) and j (aR from 0 to
+// a) of a sphere, either of them optional (p null).
+static int lut_radial_launch(bimsim_ctx* ctx, const bimsim_sphere* s, double kmag, double dmin,
+                             double dmax, int dR, const RadialOut& h, int aR, const RadialOut& j) {
+    const int nl = s->Nl;
+    const double lo = std::max(s->a, dmin), dr = (dmax - lo) / (dR - 1);
+    const double ka = kmag * s->a;
+    // (a missing table's radii are taken as the sphere's edge)
+    const double x0 = h.p ? kmag * lo : ka, x1 = h.p ? kmag * dmax : ka;
+    if (lut_closed_radii(nl, x0, x1, j.p ? s->n[0] * ka : ka, j.p ? s->n[1] * ka : 0.0,
+                         j.p ? aR : 1)) {
+        const int n = std::max(h.p ? dR : 0, j.p ? aR : 0);
+        hipLaunchKernelGGL(lut_radial_kernel, dim3((n + 63) / 64, 3), dim3(64), 0, ctx->stream, nl,
+                           kmag, lo, dr, h.p ? dR : 0, h, s->n[0], s->n[1], s->a, j.p ? aR : 0, j);
+        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
+        return BIMSIM_OK;
+    }
+    const int wstride = nl + 2;
+    const int nmax = std::max(h.p ? dR : 0, j.p ? aR : 0);
+    void* work = nullptr;
+    BIMSIM_TRY(scratch_get(ctx, kSlotMisc, sizeof(zj::zc) * 4 * (size_t)wstride * nmax, &work));
+    if (h.p)
+        hipLaunchKernelGGL(hankel_lut_kernel, dim3((dR + 63) / 64), dim3(64), 0, ctx->stream, nl,
+                           kmag, lo, dr, dR, (double*)work, wstride, h);
+    if (j.p)
+        hipLaunchKernelGGL(bessel_lut_kernel, dim3((aR + 63) / 64), dim3(64), 0, ctx->stream, nl,
+                           kmag, s->n[0], s->n[1], s->a, aR, (zj::zc*)work, wstride, j);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return BIMSIM_OK;
 }
@@ -509,27 +662,23 @@ int bimsim_sphere_lut(bimsim_ctx* ctx, const bimsim_sphere* s, const void* A, co
     BIMSIM_CHECK_ARG(ctx, (long long)dR * thetaR <= (1LL << 30), "LUT too large");
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     const int nl = s->Nl;
-    const int wstride = nl + 2;
-    const int nmax = std::max(dR, aR);
-    void *work = nullptr, *rad = nullptr;
-    BIMSIM_TRY(scratch_get(ctx, kSlotMisc, sizeof(zj::zc) * 4 * (size_t)wstride * nmax, &work));
-    BIMSIM_TRY(scratch_get(ctx, kSlotCoef, sizeof(double2) * (size_t)(nl + 1) * nmax, &rad));
+    // order by order, so that neighbouring radii's lanes read and write side by side
+    const int n_j = Uip ? aR : 0;
+    void* rad = nullptr;
+    BIMSIM_TRY(scratch_get(ctx, kSlotCoef, sizeof(double2) * (size_t)(nl + 1) * ((size_t)dR + n_j),
+                           &rad));
+    const RadialOut h = {(double2*)rad, 1, dR};
+    const RadialOut j = {Uip ? (double2*)rad + (size_t)(nl + 1) * dR : nullptr, 1, aR};
+    BIMSIM_TRY(lut_radial_launch(ctx, s, kmag, dmin, dmax, dR, h, aR, j));
     const double2* Ad = (const double2*)A + s->coeff_off;
     const double2* Bd = (const double2*)B + s->coeff_off;
     // (PI) / (thetaR - 1) is float arithmetic in the reference (sphere.cu:21)
     const double dtheta = (double)(kPIf / (float)(thetaR - 1));
-    const bool f32 = prec == BIMSIM_FP32_FAST;
-    // Usp from the Hankel table
-    const double lo = std::max(s->a, dmin);
-    hipLaunchKernelGGL(hankel_lut_kernel, dim3((dR + 63) / 64), dim3(64), 0, ctx->stream, nl, kmag,
-                       lo, (dmax - lo) / (dR - 1), dR, (double*)work, wstride, (double2*)rad);
-    BIMSIM_TRY(lut_eval_launch(ctx, f32, nl, Bd, (const double2*)rad, dR, thetaR, dtheta, Usp));
-    if (Uip) {
-        hipLaunchKernelGGL(bessel_lut_kernel, dim3((aR + 63) / 64), dim3(64), 0, ctx->stream, nl,
-                           kmag, s->n[0], s->n[1], s->a, aR, (zj::zc*)work, wstride, (double2*)rad);
-        BIMSIM_TRY(lut_eval_launch(ctx, f32, nl, Ad, (const double2*)rad, aR, thetaR, dtheta, Uip));
-    }
-    return BIMSIM_OK;
+    if (prec == BIMSIM_FP32_FAST)
+        return lut_eval_launch(ctx, nl, EvalTable<float2>{Bd, h, dR, (float2*)Usp},
+                               EvalTable<float2>{Ad, j, n_j, (float2*)Uip}, thetaR, dtheta);
+    return lut_eval_launch(ctx, nl, EvalTable<double2>{Bd, h, dR, (double2*)Usp},
+                           EvalTable<double2>{Ad, j, n_j, (double2*)Uip}, thetaR, dtheta);
 }
 
 int bimsim_sphere_radial_lut(bimsim_ctx* ctx, const bimsim_sphere* s, double kmag, double dmin,
@@ -540,22 +689,8 @@ int bimsim_sphere_radial_lut(bimsim_ctx* ctx, const bimsim_sphere* s, double kma
                      "bad radial table sizes");
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     const int nl = s->Nl;
-    const int wstride = nl + 2;
-    const int nmax = std::max(h ? dR : 0, j ? aR : 0);
-    void* work = nullptr;
-    BIMSIM_TRY(scratch_get(ctx, kSlotMisc, sizeof(zj::zc) * 4 * (size_t)wstride * nmax, &work));
-    if (h) {
-        const double lo = std::max(s->a, dmin);
-        hipLaunchKernelGGL(hankel_lut_kernel, dim3((dR + 63) / 64), dim3(64), 0, ctx->stream, nl,
-                           kmag, lo, (dmax - lo) / (dR - 1), dR, (double*)work, wstride, (double2*)h);
-        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    }
-    if (j) {
-        hipLaunchKernelGGL(bessel_lut_kernel, dim3((aR + 63) / 64), dim3(64), 0, ctx->stream, nl,
-                           kmag, s->n[0], s->n[1], s->a, aR, (zj::zc*)work, wstride, (double2*)j);
-        BIMSIM_HIP_CHECK(ctx, hipGetLastError());
-    }
-    return BIMSIM_OK;
+    return lut_radial_launch(ctx, s, kmag, dmin, dmax, dR, RadialOut{(double2*)h, nl + 1, 1}, aR,
+                             RadialOut{(double2*)j, nl + 1, 1});
 }
 
 int bimsim_nf_us_lut(bimsim_ctx* ctx, const bimsim_quad* pos, int uR, int vR,

@@ -166,6 +166,22 @@ __device__ inline int mie_start_order(int n, double az) {
 // ka), j (of n ka, complex, unscaled), w = lmax + 2 each, and the scales.
 __host__ __device__ inline int mie_closed_doubles(int w) { return 4 * w + 4; }
 
+// Spherical j_0 and j_1 of z, u = 1/z.
+__device__ __forceinline__ void sph_j01(double zr, double zi, double ur, double ui, zc* j0, zc* j1) {
+    double sr, cr;
+    sincos(zr, &sr, &cr);
+    const double e = exp(zi), ei = 1.0 / e;
+    const double ch = 0.5 * (e + ei);
+    // sinh near zero by its series (the difference would cancel)
+    const double q = zi * zi;
+    const double sh_s =
+        zi * (1.0 + q * (1.0 / 6.0 + q * (1.0 / 120.0 + q * (1.0 / 5040.0 + q * (1.0 / 362880.0)))));
+    const double shi = fabs(zi) < 0.25 ? sh_s : 0.5 * (e - ei);
+    const zc u = {ur, ui};
+    *j0 = zj::zmul(zc{sr * ch, cr * shi}, u);
+    *j1 = zj::zsub(zj::zmul(*j0, u), zj::zmul(zc{cr * ch, -(sr * shi)}, u));
+}
+
 // Coefficients of cnt <= kClosedSph spheres sh (in LDS); lds as above per
 // sphere.  Waves 0, 1 and 2 run a part each (j of ka, y of ka, j of n ka;
 // lane s: sphere s), then the block's threads take the (sphere, order)
@@ -184,19 +200,8 @@ __device__ __forceinline__ void mie_closed_block(const MieSph* sh, int cnt, int 
             // sin z / z and (sin z / z - cos z) / z at the end
             const double az2 = m.zr * m.zr + m.zi * m.zi, inv = 1.0 / az2;
             const double ur = m.zr * inv, ui = -(m.zi * inv);
-            double sr, cr;
-            sincos(m.zr, &sr, &cr);
-            const double e = exp(m.zi), ei = 1.0 / e;
-            const double ch = 0.5 * (e + ei);
-            // sinh near zero by its series (the difference would cancel)
-            const double q = m.zi * m.zi;
-            const double sh_s =
-                m.zi * (1.0 + q * (1.0 / 6.0 + q * (1.0 / 120.0 + q * (1.0 / 5040.0 +
-                                                                      q * (1.0 / 362880.0)))));
-            const double shi = fabs(m.zi) < 0.25 ? sh_s : 0.5 * (e - ei);
-            const zc u = {ur, ui};
-            const zc j0 = zj::zmul(zc{sr * ch, cr * shi}, u);
-            const zc j1 = zj::zsub(zj::zmul(j0, u), zj::zmul(zc{cr * ch, -(sr * shi)}, u));
+            zc j0, j1;
+            sph_j01(m.zr, m.zi, ur, ui, &j0, &j1);
             double fr = 1e-100, fi = 0.0, gr = 0.0, gi = 0.0;   // orders k + 1 and k + 2
             const int top = mie_start_order(n, sqrt(az2));
             double c = 2.0 * top + 3.0;
