@@ -31,6 +31,8 @@ struct UfInst {
     // diag: pixel (iu, iv) and the transposed (iv, iu) hold the same values
     // too (ncx = ncy), and the canonical pixels with cx <= cy cover the slice.
     int ncx, ncy, mx, my, nlx, nly, hx, hy, diag;
+    int mc_tile;     // Monte-Carlo sum, complex64: pixels per edge of the tiles that have
+                     // nodes, or 0 (each pixel evaluated)
 };
 
 // The mirror axis of one slice direction: positions r(i) = (a + x i/n) - f
@@ -140,14 +142,22 @@ int uf_batch_launch(bimsim_ctx* ctx, const UfInst* d_inst, int n, int items, int
                     const double* tabs, const double* waves, void* Uf,
                     const SumInst* sum = nullptr, void* D = nullptr, void* Di = nullptr);
 
-// Incident fields of the Monte-Carlo instances list[0..n) of d_inst into the
-// complex64 field Uf, in tiles of 64 x 64 pixels (the per-pixel batch
-// kernels leave those instances alone in complex64 fields).
-int uf_mc_batch_launch(bimsim_ctx* ctx, const UfInst* d_inst, const int* list, int n,
-                       int max_tiles, const double* waves, float2* Uf);
+// Sets mc_tile of n Monte-Carlo instances that one launch takes.
+void mc_node_tiles(const bimsim_ctx* ctx, UfInst* const* inst, int n);
+// Blocks of one of them.
+int mc_tiles(const UfInst& I);
 
-// Workgroups of uf_mc_batch_launch for a uR x vR field.
-int mc_tiles(int uR, int vR);
+// Monte-Carlo instances of a batch: those whose pixels are evaluated, then
+// those with nodes, and the blocks of the largest of each.
+struct McList {
+    int* d_list = nullptr;
+    int n_pixel = 0, n_node = 0, pixel_tiles = 0, node_tiles = 0;
+};
+
+// Their incident fields into the complex64 field Uf (the per-pixel batch
+// kernels leave those instances alone in complex64 fields).
+int uf_mc_batch_launch(bimsim_ctx* ctx, const UfInst* d_inst, const McList& L,
+                       const double* waves, float2* Uf);
 
 // U = Uf or U += Uf outside the spheres, for n instances; d_sph holds
 // (x, y, z, a) per sphere.  Also zeroes each instance's images in D and Di

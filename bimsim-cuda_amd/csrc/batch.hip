@@ -60,8 +60,7 @@ struct bimsim_batch {
     double* d_kdirs = nullptr;      // plane-wave directions, one row per instance
     // complex64 batches: the instances whose incident field is the
     // Monte-Carlo sum, evaluated by the tiled kernel after the per-pixel one
-    int* d_mc_list = nullptr;
-    int n_mc_uf = 0, mc_tiles_max = 0;
+    McList mc;
     // complex64 batches: instances with orders beyond the FP32 series
     // kernels, whose scattered field the FP64 form computes
     std::vector<int> wide;
@@ -128,7 +127,7 @@ void release(bimsim_batch* b) {
     series_plan_destroy(&b->plan_pw);
     for (DetBatch& d : b->det) det_batch_destroy(&d);
     void* ptrs[] = {b->d_sph, b->d_kmag, b->d_work, b->d_A, b->d_B, b->d_uf, b->d_uftab,
-                    b->d_sum, b->d_sph4, b->d_Uf, b->d_U, b->d_kdirs, b->d_mc_list,
+                    b->d_sum, b->d_sph4, b->d_Uf, b->d_U, b->d_kdirs, b->mc.d_list,
                     b->d_inside};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -181,8 +180,7 @@ int enqueue(bimsim_batch* b) {
         const bool mc = b->have_mc;
         BIMSIM_TRY(series_plan_launch_prepass(ctx, mc ? b->plan_mc : b->plan_pw,
                                               mc ? b->waves : b->d_kdirs, b->pre));
-        BIMSIM_TRY(uf_mc_batch_launch(ctx, b->d_uf, b->d_mc_list, b->n_mc_uf, b->mc_tiles_max,
-                                      b->waves, (float2*)b->d_Uf));
+        BIMSIM_TRY(uf_mc_batch_launch(ctx, b->d_uf, b->mc, b->waves, (float2*)b->d_Uf));
         BIMSIM_TRY(series_plan_launch_sums(ctx, mc ? b->plan_mc : b->plan_pw, b->d_A, b->d_B,
                                            (float2*)b->d_U));
     } else if (b->f32) {
@@ -203,8 +201,7 @@ int enqueue(bimsim_batch* b) {
             rc = uf_batch_launch(ctx, b->d_uf, b->n, b->uf_items, b->f32, b->d_uftab, b->waves,
                                  b->d_Uf, b->fuse_sum ? b->d_sum : nullptr, b->D, b->Di);
         if (rc == BIMSIM_OK)
-            rc = uf_mc_batch_launch(ctx, b->d_uf, b->d_mc_list, b->n_mc_uf, b->mc_tiles_max,
-                                    b->waves, (float2*)b->d_Uf);
+            rc = uf_mc_batch_launch(ctx, b->d_uf, b->mc, b->waves, (float2*)b->d_Uf);
         if (rc == BIMSIM_OK && hipEventRecord(b->ev_fields, b->side_f) != hipSuccess)
             rc = set_error(ctx, BIMSIM_E_HIP, "hipEventRecord failed");
         ctx->stream = main;
@@ -354,7 +351,6 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         uf_mirror(uf[i]);
         if (b->f32 && I.uf_mode == BIMSIM_UF_MC) {
             mc_list.push_back(i);
-            b->mc_tiles_max = std::max(b->mc_tiles_max, mc_tiles(I.N, I.N));
         }
         // images to clear each pass: those of the instances whose detector
         // adds to them (the batched detector writes its images whole)
@@ -418,6 +414,15 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     BIMSIM_TRY(dev_upload(ctx, &b->d_sph, sph_dev));
     BIMSIM_TRY(dev_upload(ctx, &b->d_kmag, sph_k));
+    std::vector<UfInst*> mc_inst;
+    for (int i : mc_list) mc_inst.push_back(&uf[i]);
+    mc_node_tiles(ctx, mc_inst.data(), (int)mc_inst.size());
+    std::stable_partition(mc_list.begin(), mc_list.end(), [&](int i) { return uf[i].mc_tile == 0; });
+    for (int i : mc_list) {
+        int& most = uf[i].mc_tile ? b->mc.node_tiles : b->mc.pixel_tiles;
+        most = std::max(most, mc_tiles(uf[i]));
+        ++(uf[i].mc_tile ? b->mc.n_node : b->mc.n_pixel);
+    }
     BIMSIM_TRY(dev_upload(ctx, &b->d_uf, uf));
     BIMSIM_TRY(dev_upload(ctx, &b->d_uftab, uftab));
     for (int i = 0; i < n; ++i)
@@ -425,8 +430,7 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     BIMSIM_TRY(dev_upload(ctx, &b->d_sum, sum));
     BIMSIM_TRY(dev_upload(ctx, &b->d_sph4, sph4));
     BIMSIM_TRY(dev_upload(ctx, &b->d_kdirs, kdirs));
-    BIMSIM_TRY(dev_upload(ctx, &b->d_mc_list, mc_list));
-    b->n_mc_uf = (int)mc_list.size();
+    BIMSIM_TRY(dev_upload(ctx, &b->mc.d_list, mc_list));
     b->mie_closed = mie_closed_spheres(ctx, sph_dev.data(), sph_k.data(), b->n_sph);
     if (!b->mie_closed)
         BIMSIM_TRY(dev_alloc(ctx, &b->d_work, sizeof(double2) * 8 * (size_t)(b->lmax + 2) * std::max(1, b->n_sph)));
