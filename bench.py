@@ -58,8 +58,9 @@ def log(msg):
 
 # ------------------------------------------------------------ work counts
 def harmonic_flops(Nl, planar=False):
-    """FLOPs of the harmonic series kernel per (pixel, sphere), with the
-    coefficients B_l (A_l inside) already in the records.  General form,
+    """FLOPs of the harmonic series kernel per (point, sphere; a point is a
+    pixel or, where a sphere is far from a tile of pixels, one of the tile's
+    fewer Chebyshev nodes), with the coefficients B_l (A_l inside) already in the records.  General form,
     P = (Nl+1)(Nl+2)/2 pairs (m, l >= m): per pair the scaled Legendre step
     (3), the rotation by e^{i m phi} (2) and the accumulation (8); per row
     the next diagonal value and phase (8).  Planar form (the slice contains
@@ -82,6 +83,8 @@ def is_planar(inst, s):
 
 
 def series_flops(inst):
+    """The count with every pixel evaluated: what the nodes stand for, not
+    what the kernels execute."""
     n2 = inst["N"] ** 2
     return n2 * sum(harmonic_flops(s["Nl"], is_planar(inst, s)) for s in inst["spheres"])
 
@@ -245,12 +248,16 @@ def headline(pkg, P, W, ctx, torch, args):
     log(f"bench: FP64 plain {t64 * 1e3:.1f} ms/image, hoisted FP64 {t64h * 1e3:.1f} ms/image, "
         f"absorbance error {err:.2e}")
 
-    traffic = None
+    traffic = executed_flops = None
     if os.path.exists(PROFILE_TRAFFIC):
         with open(PROFILE_TRAFFIC) as fh:
             for line in fh:
                 if line.startswith("traffic_bytes_per_pass ="):
                     traffic = int(line.split("=")[1])
+                if line.startswith("fp32_flops_per_pass ="):
+                    executed_flops = float(line.split("=")[1])
+    executed = (executed_flops / (series_ms_pass * 1e-3) / 1e12
+                if executed_flops and series_ms_pass > 0 else None)
     achieved = flops / (series_ms_pass * 1e-3) / 1e12 if series_ms_pass > 0 else None
     ach64 = f64 / us64 / 1e12 if us64 > 0 else None
     return {
@@ -275,7 +282,10 @@ def headline(pkg, P, W, ctx, torch, args):
             "us_kernel_ms_per_image": us64 * 1e3 / len(picks),
             "roofline": {"bound": "valu_fp64", "achieved": ach64, "peak": PEAK_FP64_TFLOPS,
                          "unit": "TFLOP/s", "frac": ach64 / PEAK_FP64_TFLOPS if ach64 else None,
-                         "kernel": "us_parity_kernel (reference per-wave series, FP64)",
+                         "kernel": "us_series64_kernel (per-wave series in the reference's "
+                                   "operations, radial terms formed once, FP64; counted as the "
+                                   "reference's loop, which forms them per wave: 20 per order "
+                                   "for 8)",
                          "flops_per_image": f64 / len(picks)},
         },
         "fp64_hoisted": {"images_per_s": 1.0 / t64h, "ms_per_image": t64h * 1e3},
@@ -286,11 +296,15 @@ def headline(pkg, P, W, ctx, torch, args):
             "bound_note": "compute-bound on the SIMDs, not HBM: the order-sum products run on "
                           "the matrix cores (v_mfma_f32_4x4x1_16b_f32) in the variants the "
                           "tuner picks, the FP64 radial recurrences and phase steps on the "
-                          "VALU, and the two do not issue beside each other on MI355X",
-            "achieved": achieved,
+                          "VALU, and the two do not issue beside each other on MI355X; "
+                          "evaluated at Chebyshev nodes of pixel tiles where a sphere is far",
+            "achieved": executed,
             "peak": PEAK_FP32_TFLOPS,
             "unit": "TFLOP/s",
-            "frac": achieved / PEAK_FP32_TFLOPS if achieved else None,
+            "frac": executed / PEAK_FP32_TFLOPS if executed else None,
+            "achieved_note": "FP32 FLOP per pass that the counters saw executed "
+                             "(profiles/series_harm_cfg4_traffic.md) over this run's time",
+            "pixel_equivalent_tflops": achieved,
             "traffic": traffic,
             "traffic_note": "HBM bytes per pass (the six bucket launches) from rocprofv3 "
                             "FETCH_SIZE x 2 + WRITE_SIZE, scaled by a 256 MiB copy; "
@@ -298,7 +312,8 @@ def headline(pkg, P, W, ctx, torch, args):
             "kernel": "series_harm_kernel (harmonic FP32 scattered-field sums, planar form in "
                       "chunks of orders, products on VALU FMAs or MFMA; one persistent launch "
                       "per order bucket)",
-            "flops_per_pass": flops,
+            "flops_per_pass": executed_flops,
+            "pixel_equivalent_flops_per_pass": flops,
             "series_ms_per_pass": series_ms_pass,
             "peak_note": "157.3 is AMD's published FP32 peak (vector and matrix); this build "
                          "compiles without packed FP32 instructions: plain v_fma_f32 issues "
@@ -358,7 +373,7 @@ def cfg2_image(pkg, P, W, ctx, torch, steps):
         "fp64_plain_ms_per_image": t64 * 1e3, "speedup_vs_fp64_plain": t64 / t_eager,
         "absorbance_max_abs_err_vs_fp64": err,
         "harmonic_series_kernel_ms": res["harmonic"],
-        "harmonic_series_tflops": series_flops(inst) / (res["harmonic"] * 1e-3) / 1e12,
+        "harmonic_series_pixel_equivalent_tflops": series_flops(inst) / (res["harmonic"] * 1e-3) / 1e12,
         "direct_series_kernel_ms": res["direct"],
         "direct_series_flops": dfl,
         "direct_series_tflops_by_reference_count": dfl / (res["direct"] * 1e-3) / 1e12,
@@ -565,8 +580,8 @@ def main():
         "reference_equivalent_terms_per_s": h["terms_per_s"],
         "terms_note": "Mie series terms counted as the reference's per-wave series would evaluate "
                       "them (N^2 nk sum(Nl+1) + N^2 (m+1) per image); the harmonic kernel "
-                      "reaches them with fewer operations (roofline.flops_per_pass is its own "
-                      "count), so this is a reference-equivalent rate",
+                      "reaches them with fewer operations, at fewer points than pixels "
+                      "(roofline.flops_per_pass is what it executes), so this is a reference-equivalent rate",
         "eager_pass": h["eager_pass"],
         "fp64_plain": h["fp64_plain"],
         "fp64_hoisted": h["fp64_hoisted"],

@@ -450,16 +450,15 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         BIMSIM_TRY(mie_batch_launch(ctx, b->d_sph, b->d_kmag, b->n_sph, b->lmax, b->quirks,
                                     b->mie_closed, b->d_work, b->d_A, b->d_B));
         // how far each sphere's own coefficients reach (the tiles of the
-        // harmonic form's nodes)
-        std::vector<double> hB(2 * (size_t)coef);
-        if (coef > 0) {
+        // harmonic form's nodes, which plane-wave instances do not take)
+        std::vector<double> hB(mc.sph.empty() ? 0 : 2 * (size_t)coef);
+        if (!hB.empty()) {
             BIMSIM_HIP_CHECK(ctx, hipMemcpyAsync(hB.data(), b->d_B, sizeof(double) * hB.size(),
                                                  hipMemcpyDeviceToHost, ctx->stream));
             BIMSIM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         }
-        for (SeriesBatch* sb : {&mc, &pw})
-            for (SeriesSph& S : sb->sph)
-                S.reach = node_reach(S.s, sb->inst[S.inst].kmag, hB.data() + 2 * (size_t)S.s.coeff_off);
+        for (SeriesSph& S : mc.sph)
+            S.reach = node_reach(S.s, mc.inst[S.inst].kmag, hB.data() + 2 * (size_t)S.s.coeff_off);
         if (!mc.inst.empty()) {
             BIMSIM_TRY(series_plan_create_tuned(ctx, mc, budget, b->waves, b->d_A, b->d_B, &b->plan_mc));
             b->have_mc = true;

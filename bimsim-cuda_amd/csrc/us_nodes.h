@@ -45,6 +45,12 @@ constexpr int kNodeMaxQ = 64;
 // Instructions of an instance's pixels (point_cost) below which they are
 // evaluated as they are.
 constexpr double kNodeMinWork = 1.0e8;
+// A plan below both of these, instructions of all its pixels and of the longest
+// of them, is bound by latency, and the expansion's launch costs what the
+// points save: one 512 x 512 image of 3 spheres (0.6e9, 2200) takes 95 us by
+// its pixels and 112 by nodes, one 320 x 320 of 6 (0.3e9, 3000) 177 and 162.
+constexpr double kNodeMinPlan = 1.2e9;
+constexpr double kNodeMinChain = 2600.0;
 
 // Host tables of a plan's nodes, uploaded by series_plan_create.
 struct NodeTables {
@@ -58,6 +64,9 @@ struct NodeTables {
     long long n_v = 0, n_w = 0;
     std::map<std::pair<int, int>, std::pair<int, int>> mats;   // (T, q) -> offsets in E, X
 };
+
+// Instructions of one pixel of the instance.
+double node_pixel_chain(const SeriesInst& I, const SeriesSph* sph);
 
 // Adds instance i's nodes to the tables when they cost less than its pixels
 // (else its entry has n_lev = 0).  sph: its spheres in plan order.

@@ -182,12 +182,16 @@ bool node_mask_any(const unsigned long long* m, int begin, int n) {
     return false;
 }
 
+double node_pixel_chain(const SeriesInst& I, const SeriesSph* sph) {
+    double one = 0.0;
+    for (int s = 0; s < I.ns; ++s) one += point_cost(sph[s].s.Nl + 1);
+    return one;
+}
+
 void node_plan_instance(const SeriesInst& I, const SeriesSph* sph, NodeTables* t) {
     const int at = (int)t->inst.size();
     t->inst.push_back(NodeInst{});
-    double pixels = 0.0;
-    for (int s = 0; s < I.ns; ++s) pixels += point_cost(sph[s].s.Nl + 1);
-    pixels *= (double)I.uR * I.vR;
+    const double pixels = node_pixel_chain(I, sph) * I.uR * I.vR;
     // a slice whose pixels are some four waves per SIMD for one small sphere
     // is bound by latency: another launch costs what its points would save
     if (I.ns == 0 || pixels < kNodeMinWork) return;

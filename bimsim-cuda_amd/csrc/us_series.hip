@@ -1029,7 +1029,13 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     // harmonic form: the nodes of the instances they pay for
     NodeTables nt;
     bool any_nodes = false;
-    if (P->harmonic) {
+    double pixel_work = 0.0, chain = 0.0;
+    for (const SeriesInst& I : batch.inst) {
+        const double one = node_pixel_chain(I, batch.sph.data() + I.s_begin);
+        chain = std::max(chain, one);
+        pixel_work += one * I.uR * I.vR;
+    }
+    if (P->harmonic && (pixel_work >= kNodeMinPlan || chain >= kNodeMinChain)) {
         for (const SeriesInst& I : batch.inst) {
             node_plan_instance(I, batch.sph.data() + I.s_begin, &nt);
             any_nodes = any_nodes || nt.inst.back().n_lev > 0;
