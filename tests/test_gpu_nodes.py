@@ -25,9 +25,15 @@ def spheres_of(pkg, lam, rows):
     return out, off
 
 
+# far spheres that lift every call over the work below which a plan keeps to
+# its pixels (their own nodes are the coarsest tiles')
+FAR = [((200.0 + 20.0 * i, 300.0, 0.0), 3.0, 1.4 + 0.01j) for i in range(9)]
+
+
 def both(pkg, ctx, q, uR, vR, lam, rows, nk=20, accumulate=False, seed=0):
     kmag = 2.0 * math.pi / lam
-    spheres, n = spheres_of(pkg, lam, rows)
+    spheres, n = spheres_of(pkg, lam, rows + FAR)
+    assert sum(0.5 * (s["Nl"] + 1) ** 2 + 12 * (s["Nl"] + 1) + 90 for s in spheres) >= 2600
     A = torch.zeros(n, dtype=torch.complex128, device="cuda")
     B = torch.zeros_like(A)
     ctx.mie_coeffs(spheres, kmag, A, B)
@@ -121,10 +127,12 @@ def test_nodes_accumulate(pkg, ctx):
 def test_node_batches_eager_captured_and_per_call(pkg, ctx):
     """Instances with nodes and without (small, no spheres) in one batch: the
     same images eagerly and replayed, with other work between the replays,
-    and the per-call pipeline's."""
+    and the per-call pipeline's, whose plans are small enough to keep to
+    their pixels."""
     import bimsim_amd.pipeline as P
     import bimsim_amd.workloads as W
-    insts = [W.config(2, N=320, nk=32), W.config(1, N=48, nk=32), W.config(2, N=256, nk=48)]
+    insts = [W.config(2, N=512, nk=32), W.config(1, N=48, nk=32), W.config(2, N=512, nk=48),
+             W.config(2, N=320, nk=24)]
     waves = [W.mc_waves(i, pkg.mc_sample_na) for i in insts]
     arr, spheres, Wv, n = P.batch_tables(insts, waves)
     wd = torch.as_tensor(Wv.ravel()).cuda()
