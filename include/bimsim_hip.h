@@ -38,10 +38,10 @@ typedef enum {
 } bimsim_status;
 
 /* Arithmetic form of a call.
- *   FP64_PARITY: the reference algorithm in double, reference operation order
- *                and loop structure (per-wave recurrences), FMA contraction off.
- *   FP64:        same arithmetic, wave-independent Bessel/Hankel terms hoisted
- *                out of the wave loop (identical operation sequence per term).
+ *   FP64_PARITY: the reference algorithm in double, reference operations and
+ *                order per term, FMA contraction off; the Bessel/Hankel terms
+ *                that no wave changes formed once.
+ *   FP64:        the same arithmetic (the scattered field bit for bit).
  *   FP32_FAST:   Bessel terms and Mie products in double, per-wave Legendre
  *                series, plane-wave sum and FFT in float with compensated
  *                accumulation. */
