@@ -142,24 +142,38 @@ __host__ __device__ inline MieSph mie_sph(const SphereDev& S, double kmag) {
     return MieSph{kmag * S.a, z.r, z.i, S.n[0], S.n[1], S.Nl, S.coeff_off};
 }
 
-// The spheres the closed form takes: the order within 20 of the size's own
-// (sphere::calcNl: x + 4 x^(1/3) + 2), so that no order leaves the range of
-// a double, and arguments whose sinh and cosh stay far from overflow.
-__host__ __device__ inline bool mie_closed_form(const MieSph& m) {
-    const double az = sqrt(m.zr * m.zr + m.zi * m.zi);
-    return m.Nl >= 2 && m.x >= 1e-2 && m.x <= 4096.0 && az >= 1e-2 && az <= 4096.0 &&
-           m.zr >= 0.0 && fabs(m.zi) <= 100.0 &&
-           (double)m.Nl <= m.x + 4.05 * cbrt(m.x) + 20.0;
-}
-
 // First order of the downward recurrence for orders up to n of argument
 // magnitude az: far enough past both that what the start leaves out of
 // order n (the ratio of j to y at the start against that at n, which falls
 // as exp(-(2 sqrt(2)/3) 2 (d/az^(1/3))^(3/2)) past the turning point, d
 // orders beyond it) is below 1e-18.
-__device__ inline int mie_start_order(int n, double az) {
+__host__ __device__ inline int mie_start_order(int n, double az) {
     const double c = cbrt(az);
     return (int)(fmax((double)n, az) + 8.0 * c + 16.0);
+}
+
+// Natural log of the growth of that recurrence from its start down to the
+// orders of az's own size: v acosh(v / az) - sqrt(v^2 - az^2), v = k + 1/2
+// (the ratio of j there to j at the start by their Debye expansions).  An
+// absorbing sphere's grows by up to |Im z| more.
+inline double mie_growth(int n, double az) {
+    const double v = std::max(mie_start_order(n, az) + 0.5, az);
+    return v * std::acosh(v / az) - std::sqrt(v * v - az * az);
+}
+
+// The spheres the closed form takes: the order within 20 of the size's own
+// (sphere::calcNl: x + 4 x^(1/3) + 2), arguments whose sinh and cosh stay far
+// from overflow, and recurrences that grow by at most exp(500) = 1e217 from
+// their start of 1e-100, so that neither they nor the scaled j_l leave the
+// range of a double.  Of those orders k a's grows by exp(300) at most, and so
+// does an n k a no smaller; the last condition shuts out orders far beyond
+// |n| k a (at n = 0.1 from k a of about 155 on, at n = 0.5 of 770).
+inline bool mie_closed_form(const MieSph& m) {
+    const double az = std::sqrt(m.zr * m.zr + m.zi * m.zi);
+    return m.Nl >= 2 && m.x >= 1e-2 && m.x <= 4096.0 && az >= 1e-2 && az <= 4096.0 &&
+           m.zr >= 0.0 && std::fabs(m.zi) <= 100.0 &&
+           (double)m.Nl <= m.x + 4.05 * std::cbrt(m.x) + 20.0 &&
+           (az >= m.x || mie_growth(m.Nl, az) + std::fabs(m.zi) <= 500.0);
 }
 
 // LDS of a sphere in doubles: orders 0 .. Nl of j (of ka, unscaled), y (of

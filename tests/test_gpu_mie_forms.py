@@ -72,3 +72,23 @@ def test_orders_past_the_closed_form(pkg, ctx, orc, extra):
         a_, b_ = orc.mie_coeffs(s["Nl"], kmag, s["a"], n, 1)
         assert np.linalg.norm(A[sl] - a_) <= 1e-11 * np.linalg.norm(a_), s
         assert np.linalg.norm(B[sl] - b_) <= 1e-11 * np.linalg.norm(b_), s
+
+
+# k a and an index far below one, whose orders run past |n| k a by far: on both
+# sides of where the closed form's recurrence would leave its range, and past
+# where it would overflow (x = 160, 360 and 800 for these indices)
+@pytest.mark.parametrize("x,n", [(60.0, 0.01), (120.0, 0.01), (160.0, 0.01), (150.0, 0.1),
+                                 (160.0, 0.1), (400.0, 0.1), (350.0, 0.3), (800.0, 0.3)])
+def test_index_far_below_one(pkg, ctx, orc, x, n):
+    kmag = 2.0
+    s = dict(a=x / kmag, n=complex(n), Nl=pkg.sphere_order(x / kmag, 2 * np.pi / kmag))
+    A, B = run(pkg, ctx, [s], kmag, 1)
+    a, b = orc.mie_coeffs(s["Nl"], kmag, s["a"], s["n"], 1)
+    # (the reference's own arrays leave the range at the highest orders)
+    there = np.isfinite(a) & np.isfinite(b)
+    assert there.sum() > 0.5 * len(a)
+    A, B = (g[: s["Nl"] + 1][there] for g in (A, B))
+    a, b = a[there], b[there]
+    assert np.linalg.norm(B - b) <= 1e-11 * np.linalg.norm(b)
+    # A grows over the orders by up to 1e200: each order by itself
+    assert (np.abs(A - a) <= 1e-9 * np.abs(a)).all()
