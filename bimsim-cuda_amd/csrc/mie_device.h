@@ -181,15 +181,19 @@ inline bool mie_closed_form(const MieSph& m) {
 __host__ __device__ inline int mie_closed_doubles(int w) { return 4 * w + 4; }
 
 // Spherical j_0 and j_1 of z, u = 1/z.
-__device__ __forceinline__ void sph_j01(double zr, double zi, double ur, double ui, zc* j0, zc* j1) {
+__host__ __device__ __forceinline__ void sph_j01(double zr, double zi, double ur, double ui, zc* j0,
+                                                 zc* j1) {
     double sr, cr;
     sincos(zr, &sr, &cr);
     const double e = exp(zi), ei = 1.0 / e;
     const double ch = 0.5 * (e + ei);
-    // sinh near zero by its series (the difference would cancel)
+    // sinh near zero by its series (the difference would cancel); what it
+    // leaves out is zi^12 / 13!, 1e-17 at a quarter
     const double q = zi * zi;
     const double sh_s =
-        zi * (1.0 + q * (1.0 / 6.0 + q * (1.0 / 120.0 + q * (1.0 / 5040.0 + q * (1.0 / 362880.0)))));
+        zi * (1.0 + q * (1.0 / 6.0 +
+                         q * (1.0 / 120.0 +
+                              q * (1.0 / 5040.0 + q * (1.0 / 362880.0 + q * (1.0 / 39916800.0))))));
     const double shi = fabs(zi) < 0.25 ? sh_s : 0.5 * (e - ei);
     const zc u = {ur, ui};
     *j0 = zj::zmul(zc{sr * ch, cr * shi}, u);
