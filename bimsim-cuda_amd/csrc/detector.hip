@@ -1390,20 +1390,31 @@ std::mutex g_noalloc_mu;
 void* g_noalloc_ptr[kNoAllocDevices] = {};
 bool g_noalloc_tried[kNoAllocDevices] = {};
 
-// e^{-2 pi i t/n}, t < n, evaluated in double (as the context's tables)
-template <class C>
-__global__ void twiddle_fill_kernel(C* __restrict__ tw, int n) {
+// The tables of a call in one launch: e^{-2 pi i t/n} of both lengths,
+// evaluated in double (as the context's tables), for the forward rows (tu) and
+// past the columns (t2u, t2v; tv where they are the same type), and the
+// pass-band columns, the first n1 and the last n2 of uR.
+template <class C, class C2T>
+__global__ void noalloc_tables_kernel(C* __restrict__ tu, C2T* __restrict__ t2u,
+                                      C2T* __restrict__ t2v, int uR, int vR,
+                                      int* __restrict__ cols, int n1, int n2) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const double ang = -2.0 * M_PI * (double)t / (double)n;
-    tw[t].x = cos(ang);
-    tw[t].y = sin(ang);
-}
-
-// the first n1 and the last n2 of uR columns
-__global__ void band_cols_kernel(int* __restrict__ cols, int n1, int n2, int uR) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < n1 + n2) cols[c] = c < n1 ? c : uR - n2 + (c - n1);
+    if (t < uR) {
+        const double ang = -2.0 * M_PI * (double)t / (double)uR;
+        const double c = cos(ang), s = sin(ang);
+        tu[t].x = c;
+        tu[t].y = s;
+        if (t2u) {
+            t2u[t].x = c;
+            t2u[t].y = s;
+        }
+    }
+    if (t < vR) {
+        const double ang = -2.0 * M_PI * (double)t / (double)vR;
+        t2v[t].x = cos(ang);
+        t2v[t].y = sin(ang);
+    }
+    if (t < n1 + n2) cols[t] = t < n1 ? t : uR - n2 + (t - n1);
 }
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -1447,24 +1458,16 @@ int detector_noalloc_impl(bimsim_ctx* ctx, unsigned char* work, int quirks, cons
                          "entry point has %zu",
                          need, kNoAllocBytes);
     C* tu = (C*)(work + o_tu);
-    C* tv = (C*)(work + o_tv);
     int* cols = (int*)(work + o_cols);
-    hipLaunchKernelGGL(twiddle_fill_kernel<C>, dim3((uR + 255) / 256), dim3(256), 0, ctx->stream,
-                       tu, uR);
-    hipLaunchKernelGGL(twiddle_fill_kernel<C>, dim3((vR + 255) / 256), dim3(256), 0, ctx->stream,
-                       tv, vR);
-    double2 *t2u = (double2*)tu, *t2v = (double2*)tv;
-    if (wide) {
-        t2u = (double2*)(work + o_t2u);
-        t2v = (double2*)(work + o_t2v);
-        hipLaunchKernelGGL(twiddle_fill_kernel<double2>, dim3((uR + 255) / 256), dim3(256), 0,
-                           ctx->stream, t2u, uR);
-        hipLaunchKernelGGL(twiddle_fill_kernel<double2>, dim3((vR + 255) / 256), dim3(256), 0,
-                           ctx->stream, t2v, vR);
-    }
-    if (Nc > 0)
-        hipLaunchKernelGGL(band_cols_kernel, dim3((Nc + 255) / 256), dim3(256), 0, ctx->stream,
-                           cols, n1, n2, uR);
+    void* t2u = wide ? work + o_t2u : work + o_tu;
+    void* t2v = wide ? work + o_t2v : work + o_tv;
+    const dim3 tgrid((std::max(uR, vR) + 255) / 256);   // (Nc <= uR)
+    if (wide)
+        hipLaunchKernelGGL((noalloc_tables_kernel<C, double2>), tgrid, dim3(256), 0, ctx->stream,
+                           tu, (double2*)t2u, (double2*)t2v, uR, vR, cols, n1, n2);
+    else
+        hipLaunchKernelGGL((noalloc_tables_kernel<C, C>), tgrid, dim3(256), 0, ctx->stream, tu,
+                           (C*)nullptr, (C*)t2v, uR, vR, cols, n1, n2);
     BIMSIM_HIP_CHECK(ctx, hipGetLastError());
     return detector_band<R>(ctx, bp, const_cast<void*>(U), const_cast<void*>(Uf), uR, vR, uR, vR,
                             padding, Nd, ss, D, Di, Abs, 0, tu, t2u, t2v, nullptr, cols, Nc,
