@@ -545,6 +545,9 @@ __device__ __forceinline__ void rows_fwd_body(
                 a[tot + t] = or_zero(ok[k], w[k]);
             }
         }
+    } else if (!kBoth && !(kSum && f == 0) && !pad) {
+        const C* F = (f ? Uf : U) + (size_t)row0 * n;
+        for (int t = threadIdx.x; t < tot; t += kThreads) a[t] = F[t];
     } else {
         const C* F = f ? Uf : U;
         for (int t = threadIdx.x; t < tot; t += kThreads) {
@@ -986,8 +989,10 @@ int detector_band(bimsim_ctx* ctx, const PostOp& bp, void* Uin, void* Ufin, int 
     }
     const int B = rows_per_group(nrows, f32 ? cs2 : cs2 / 2);
     const size_t lds = cs2 * 2 * (size_t)B * uR;
-    if (Nc > 0 && ss == 1 && !write_filtered && 2 * lds <= ctx->lds_max) {
+    if (Nc > 0 && ss == 1 && !write_filtered && 2 * lds <= (wide ? ctx->lds_max / 2 : ctx->lds_max)) {
         // both fields' rows per workgroup, detection on them in the same pass
+        // (FP64 rows of an FP32 detector only where two workgroups fit a CU:
+        // 1536 x 1536 in 85 us by two passes, 106 in one; 2048 x 2048 138 and 158)
         with_compute<R>(wide, [&](auto r2) {
             using R2 = decltype(r2);
             using C2T = typename C2<R2>::T;
