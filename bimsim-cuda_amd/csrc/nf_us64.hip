@@ -293,6 +293,103 @@ __global__ void us_combine64_kernel(int n, int ns, const double* __restrict__ pa
     U[i] = acc;
 }
 
+// The few-wave form: a thread a pixel, W >= nk waves of a sphere in registers,
+// the radial chains run beside the waves' own.  The same operations in the same
+// order as us_series64_kernel, whose blocks give a pixel's chains and its waves
+// a wavefront each and leave most of them idle where there are few waves.
+// Bound by FP64 issue.  One wave and one sphere of 18 orders on 256 x 256
+// pixels 11 us (28 in the other form), 512 x 512 22 (85), 1024 x 1024 75 (309);
+// of 116 orders on 512 x 512 79 (574); four waves, four spheres of 39 orders on
+// 512 x 512 217 (433).
+template <int W>
+__global__ __launch_bounds__(kThreads) void us_few64_kernel(
+    QuadArg q, int uR, int vR, d3 f, double kmag, UsSphereBatch batch, int ns,
+    const double2* __restrict__ A, const double2* __restrict__ B,
+    const double* __restrict__ waves, int nk, double sA, double2* __restrict__ U, int accumulate) {
+    __shared__ double2 ph[W];
+    const int npix = uR * vR;
+    const int pix = blockIdx.x * kThreads + (int)threadIdx.x;
+    const int at = min(pix, npix - 1), iv = at / uR, iu = at - iv * uR;
+    const d3 p = quad_at(q, (double)iu / (double)uR, (double)iv / (double)vR);
+    dc acc = {0.0, 0.0};
+    if (accumulate) acc = ld2(U, at);
+    for (int s = 0; s < ns; ++s) {
+        const SphereDev& S = batch.s[s];
+        const d3 ps = mk(S.p), c = sub(ps, f);
+        d3 r = sub(p, ps);
+        const double d = len(r), kd = kmag * d;
+        const dc knd = cscl(dc{S.n[0], S.n[1]}, kd);
+        r = norm(r);
+        const bool inside = d <= S.a, centre = inside && knd.r < (double)kEpsFloat;
+        const double2* const C = (inside ? A : B) + S.coeff_off;
+        __syncthreads();   // the last sphere's phases are used
+        if ((int)threadIdx.x < nk) {
+            const dc e = cscl(cexp_i(kmag * dot(mk(waves + 3 * threadIdx.x), c)), sA);
+            ph[threadIdx.x] = make_double2(e.r, e.i);
+        }
+        __syncthreads();
+        double x[W], P0[W], P1[W], tr[W], ti[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            x[w] = dot(mk(waves + 3 * min(w, nk - 1)), r);
+            P0[w] = 1.0;
+            P1[w] = x[w];
+        }
+        auto first = [&](dc c0, dc c1) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                tr[w] = 0.0 + c0.r;
+                ti[w] = 0.0 + c0.i;
+                tr[w] += c1.r * x[w];
+                ti[w] += c1.i * x[w];
+            }
+        };
+        auto order = [&](int l, dc cl) {
+            const double a = (double)(2 * l - 1), b = (double)(l - 1), n = (double)l, inv = 1.0 / n;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const double Pn = div_int(a * x[w] * P1[w] - b * P0[w], n, inv);
+                P0[w] = P1[w];
+                P1[w] = Pn;
+                tr[w] += cl.r * Pn;
+                ti[w] += cl.i * Pn;
+            }
+        };
+        if (centre) {   // calc_Ui: A_0 for every wave
+            const dc c0 = ld2(C, 0);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                tr[w] = c0.r;
+                ti[w] = c0.i;
+            }
+        } else if (inside) {
+            dc j[2];
+            ref::init_jc(knd, j);
+            first(cmul(ld2(C, 0), j[0]), cmul(ld2(C, 1), j[1]));
+            for (int l = 2; l <= S.Nl; ++l) {
+                ref::shift_jc(l, knd, j);
+                order(l, cmul(ld2(C, l), j[1]));
+            }
+        } else {
+            double j[2], y[2];
+            ref::init_j(kd, j);
+            ref::init_y(kd, y);
+            first(cmul(ld2(C, 0), dc{j[0], y[0]}), cmul(ld2(C, 1), dc{j[1], y[1]}));
+            for (int l = 2; l <= S.Nl; ++l) {
+                ref::shift_j(l, kd, j);
+                ref::shift_y(l, kd, y);
+                order(l, cmul(ld2(C, l), dc{j[1], y[1]}));
+            }
+        }
+        dc sum = {0.0, 0.0};
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+            if (w < nk) sum = cadd(sum, cmul(ld2(ph, w), dc{tr[w], ti[w]}));
+        acc = cadd(acc, sum);
+    }
+    if (pix < npix) U[pix] = make_double2(acc.r, acc.i);
+}
+
 __global__ void clear_c64(double2* U, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) U[i] = make_double2(0.0, 0.0);
@@ -330,6 +427,15 @@ SphereDev to_dev(const bimsim_sphere& S) {
 // with the same operations.
 constexpr int kSplitBlocks = 4096;
 
+// Whether a call takes the few-wave form: up to two waves where the pixels are
+// more than two wavefronts a CU (one wave, 192 x 192: one sphere 12 us and 19
+// in the other form, four of 39 orders 64 and 68; 144 x 144: 13 and 15, 64 and
+// 48), three or four where they are four (256 x 256: 17 and 28, 47 and 60; 224
+// x 224, four spheres: 107 and 95).
+bool few_waves64(const bimsim_ctx* ctx, int npix, int nk) {
+    return (nk <= 2 && npix > 128 * ctx->cu_count) || (nk <= 4 && npix >= 256 * ctx->cu_count);
+}
+
 int us_series64(bimsim_ctx* ctx, const QuadArg& q, int uR, int vR, d3 f, double kmag,
                 const bimsim_sphere* spheres, int ns, const double2* A, const double2* B,
                 const double* waves, int nk, double sA, int lmax, double* U, int accumulate) {
@@ -337,8 +443,9 @@ int us_series64(bimsim_ctx* ctx, const QuadArg& q, int uR, int vR, d3 f, double 
     const int cap = std::min(lmax + 1, kOrders);
     const size_t lds = (size_t)kSumBytes + sizeof(double2) * kPhases +
                        (size_t)cap * (sizeof(StepConst) + 64 * sizeof(double2));
+    const bool few = few_waves64(ctx, npix, nk);
     void* part = nullptr;
-    if (ns > 1 && blocks <= kSplitBlocks)
+    if (!few && ns > 1 && blocks <= kSplitBlocks)
         part = scratch_try(ctx, kSlotSums, sizeof(double2) * (size_t)std::min(ns, kUsBatch) * npix);
     for (int s0 = 0; s0 < ns; s0 += kUsBatch) {
         const int cnt = std::min(kUsBatch, ns - s0), add = (s0 > 0 || accumulate) ? 1 : 0;
@@ -349,7 +456,16 @@ int us_series64(bimsim_ctx* ctx, const QuadArg& q, int uR, int vR, d3 f, double 
                 return spheres[s0 + x].Nl > spheres[s0 + y].Nl;
             });
         for (int i = 0; i < cnt; ++i) b.s[i] = to_dev(spheres[s0 + b.slot[i]]);
-        if (part) {
+        if (few) {
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((npix + kThreads - 1) / kThreads), dim3(kThreads),
+                                   0, ctx->stream, q, uR, vR, f, kmag, b, cnt, A, B, waves, nk, sA,
+                                   (double2*)U, add);
+            };
+            if (nk == 1) launch(us_few64_kernel<1>);
+            else if (nk == 2) launch(us_few64_kernel<2>);
+            else launch(us_few64_kernel<4>);
+        } else if (part) {
             hipLaunchKernelGGL(us_series64_kernel<true>, dim3(blocks, cnt), dim3(kThreads), lds,
                                ctx->stream, q, uR, vR, f, kmag, b, cnt, A, B, waves, nk, sA, cap,
                                (double*)part, U, add);

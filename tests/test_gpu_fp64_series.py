@@ -106,3 +106,29 @@ def test_slices_beyond_the_split(pkg, ctx):
     ctx.nf_us(q, n, 241, (0.0, 0.0, 0.0), kmag, spheres, A, B, waves, 0.7, part, prec=pkg.FP64)
     a, b = whole.view(rows, n)[::17], part.view(241, n)
     assert float((a - b).abs().max()) <= 1e-10 * float(b.abs().max())
+
+
+# both sides of the few-wave form's limits (more than 128 pixels a CU, or from
+# 256 on), spheres that cover part of the slice and one centred on a pixel,
+# orders past those the other form holds at a time, more than 32 spheres
+@pytest.mark.parametrize("ns,nk,ka,uR,vR", [
+    (1, 1, 3.0, 181, 181), (1, 1, 3.0, 182, 182), (3, 2, 2.0, 257, 129), (2, 3, 3.0, 256, 256),
+    (1, 4, 93.0, 300, 219), (1, 1, 93.0, 222, 150), (35, 2, 2.0, 200, 165), (1, 5, 3.0, 256, 256)])
+def test_few_waves(pkg, ctx, orc, ns, nk, ka, uR, vR):
+    spheres, off, kmag, k = setup(pkg, ns, nk, ka)
+    A, B = coefficients(ctx, spheres, off, kmag)
+    waves = torch.as_tensor(k).cuda()
+    width = 5.0 * ka / kmag
+    U0 = torch.view_as_complex(torch.randn(uR * vR, 2, dtype=torch.float64, device="cuda"))
+    for U in (None, U0):
+        got = field(pkg, ctx, spheres, A, B, kmag, waves, uR, vR, width, pkg.FP64, U)
+        parity = field(pkg, ctx, spheres, A, B, kmag, waves, uR, vR, width, pkg.FP64_PARITY, U)
+        assert torch.equal(got, parity)
+        # the first row alone (the same points) takes the other form: the same bits
+        row = field(pkg, ctx, spheres, A, B, kmag, waves, uR, 1, width, pkg.FP64,
+                    None if U is None else U[:uR])
+        assert torch.equal(got[:uR], row)
+    want = orc.nf_us(pkg.Quad.xy(width), uR, vR, (0.1, -0.2, 0.3), kmag, spheres, A.cpu().numpy(),
+                     B.cpu().numpy(), k, 0.7).ravel()
+    got = field(pkg, ctx, spheres, A, B, kmag, waves, uR, vR, width, pkg.FP64).cpu().numpy()
+    assert np.abs(got - want).max() <= 1e-10 * np.abs(want).max()
