@@ -334,6 +334,10 @@ int series_plan_launch_sums(bimsim_ctx* ctx, const SeriesPlan& plan, const doubl
 bool series_few_rows(const bimsim_ctx* ctx, const SeriesPlan& plan);
 
 
+// The class of each of an instance's pixels, for the harmonic form's order of
+// them: 1 + the first sphere that holds it (d <= a), or 0.  False if none does.
+bool pixel_classes(const SeriesInst& I, const SeriesSph* sph, std::vector<int>* cls);
+
 // Order capacity for Nl + 1 orders, or -1.
 int series_capacity(int nl1);
 
