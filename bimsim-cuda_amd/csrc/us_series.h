@@ -334,9 +334,10 @@ int series_plan_launch_sums(bimsim_ctx* ctx, const SeriesPlan& plan, const doubl
 bool series_few_rows(const bimsim_ctx* ctx, const SeriesPlan& plan);
 
 
-// The class of each of an instance's pixels, for the harmonic form's order of
-// them: 1 + the first sphere that holds it (d <= a), or 0.  False if none does.
-bool pixel_classes(const SeriesInst& I, const SeriesSph* sph, std::vector<int>* cls);
+// Appends an instance's pixels in the harmonic form's order: those of each
+// sphere from the first on (d <= a; a pixel of several is the first's), then
+// those of none.  Nothing (false) where no sphere holds one.
+bool pixel_order(const SeriesInst& I, const SeriesSph* sph, std::vector<int>* perm);
 
 // Order capacity for Nl + 1 orders, or -1.
 int series_capacity(int nl1);
