@@ -42,15 +42,38 @@ constexpr int kNearTile = 16;       // a near tile is a block's 256 pixels
 // Nodes per edge: at most 3/4 of the tile's pixels, and 64 (the expansion's
 // LDS).
 constexpr int kNodeMaxQ = 64;
-// Instructions of an instance's pixels (point_cost) below which they are
-// evaluated as they are.
-constexpr double kNodeMinWork = 1.0e8;
-// A plan below both of these, instructions of all its pixels and of the longest
-// of them, is bound by latency, and the expansion's launch costs what the
-// points save: one 512 x 512 image of 3 spheres (0.6e9, 2200) takes 95 us by
-// its pixels and 112 by nodes, one 320 x 320 of 6 (0.3e9, 3000) 177 and 162.
-constexpr double kNodeMinPlan = 1.2e9;
-constexpr double kNodeMinChain = 2600.0;
+// Costs are in units of one order of one planar sphere at one point (some
+// 0.7e-6 us where the chip is full).
+// An instance's pixels below which they are evaluated as they are.
+constexpr double kNodeMinWork = 8.0e6;
+// What a plan's time is but for its points' work: the longest chain of spheres
+// at a point (whatever the number of points), and for nodes the expansion's
+// launch and its phases for each size of tiles.  Fitted to 760 images of 128^2
+// to 1024^2 pixels and 1 to 20 spheres of 13 to 39 orders, planar or not,
+// timed by pixels and by nodes: 15 of them are slower than their pixels by
+// more than 3 per cent (1.2 times at most), and the mean is 2.0 per cent from
+// the better of the two.  (Thresholds on the pixels' work and chain alone: 73,
+// 1.38 times and 6.2 per cent.)  On either side of the line, us by pixels and
+// by nodes: planar spheres of 39 orders, 512 x 512, three 94 and 111, six 155
+// and 135; 256 x 256, six 105 and 120, twenty 288 and 230; of 18 orders, two on
+// 512 x 512 49 and 50, on 768 x 768 78 and 57; off the plane, 256 x 256, one of
+// 39 102 and 118, six of 28 214 and 167.
+constexpr double kNodeChain = 2.0e5;
+constexpr double kNodeLaunch = 1.5e7;
+constexpr double kNodeLevel = 4.0e6;
+
+struct NodeCost {
+    double work = 0.0, chain = 0.0;
+    int levels = 0;
+    double total() const {
+        return work + kNodeChain * chain + (levels > 0 ? kNodeLaunch + kNodeLevel * levels : 0.0);
+    }
+    void add(const NodeCost& c) {
+        work += c.work;
+        chain = chain > c.chain ? chain : c.chain;
+        levels = levels > c.levels ? levels : c.levels;
+    }
+};
 
 // Host tables of a plan's nodes, uploaded by series_plan_create.
 struct NodeTables {
@@ -65,12 +88,14 @@ struct NodeTables {
     std::map<std::pair<int, int>, std::pair<int, int>> mats;   // (T, q) -> offsets in E, X
 };
 
-// Instructions of one pixel of the instance.
-double node_pixel_chain(const SeriesInst& I, const SeriesSph* sph);
+// The instance evaluated at its pixels.  planar: every sphere of the plan is
+// (one that is not puts its order bucket on the general sums).
+NodeCost node_pixel_cost(const SeriesInst& I, const SeriesSph* sph, bool planar);
 
 // Adds instance i's nodes to the tables when they cost less than its pixels
-// (else its entry has n_lev = 0).  sph: its spheres in plan order.
-void node_plan_instance(const SeriesInst& I, const SeriesSph* sph, NodeTables* t);
+// (else its entry has n_lev = 0); returns what the instance then costs.  sph:
+// its spheres in plan order.
+NodeCost node_plan_instance(const SeriesInst& I, const SeriesSph* sph, bool planar, NodeTables* t);
 
 // Whether the tile's mask (words 64-bit words at m) has a sphere of
 // [begin, begin + n).

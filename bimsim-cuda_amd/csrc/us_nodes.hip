@@ -25,9 +25,13 @@ static_assert(kNodeMaxQ / 2 * kNodeMaxQ <= kRoundNodes, "a round of the largest 
 // (found for kh from 0.1 to 40).
 int node_count(double kh) { return (int)std::ceil(kh + 6.0 * std::cbrt(kh) + 2.5); }
 
-// Instructions of one point and a sphere of n = Nl + 1 orders: the order
-// sums' products, the radial steps and products, the set-up.
-double point_cost(int n) { return 0.5 * n * n + 12.0 * n + 90.0; }
+// One point and a sphere of n = Nl + 1 orders (the planar sums' products on the
+// matrix cores hardly show beside the radial steps).
+double point_cost(int n, bool planar) { return planar ? n : 0.155 * n * n + 27.0; }
+// A point's position and its result, whatever its spheres.
+constexpr double kPointCost = 40.0;
+// An FMA of the expansion.
+constexpr double kExpandCost = 0.04;
 
 // Interpolation matrix and node positions of (T, q): offsets in E and X.
 std::pair<int, int> matrix(NodeTables* t, int T, int q) {
@@ -77,9 +81,11 @@ struct Tiling {
     std::vector<double> cu, cv, cz2, reach;
     std::vector<int2> tiles[kNodeLevels + 1];   // the last: near tiles
     std::vector<unsigned long long> mask[kNodeLevels + 1];
-    double cost = 0.0;
+    bool planar;
+    NodeCost cost;
 
-    Tiling(const SeriesInst& inst, const SeriesSph* s, int top) : I(inst), sph(s) {
+    Tiling(const SeriesInst& inst, const SeriesSph* s, bool all_planar, int top)
+        : I(inst), sph(s), planar(all_planar) {
         words = (I.ns + 63) / 64;
         const double lx = len(I.q.X), ly = len(I.q.Y);
         px = lx / I.uR;
@@ -118,8 +124,11 @@ struct Tiling {
     void add(int l, int i0, int j0, const std::vector<unsigned long long>& m, int points) {
         tiles[l].push_back(make_int2(i0, j0));
         mask[l].insert(mask[l].end(), m.begin(), m.end());
+        double one = 0.0;
         for (int t = 0; t < I.ns; ++t)
-            if ((m[t >> 6] >> (t & 63)) & 1) cost += points * point_cost(sph[t].s.Nl + 1);
+            if ((m[t >> 6] >> (t & 63)) & 1) one += point_cost(sph[t].s.Nl + 1, planar);
+        cost.work += points * (one + kPointCost);
+        cost.chain = std::max(cost.chain, one);
     }
     void cut(int l, int i0, int j0, std::vector<unsigned long long> left) {
         if (active[l]) {
@@ -154,10 +163,13 @@ struct Tiling {
         const int T0 = kNodeTile[0];
         for (int j0 = 0; j0 < I.vR; j0 += T0)
             for (int i0 = 0; i0 < I.uR; i0 += T0) cut(0, i0, j0, all);
-        cost += 30.0 * I.uR * I.vR;
-        for (int l = 0; l < kNodeLevels; ++l)
-            cost += (double)tiles[l].size() * kNodeTile[l] * kNodeTile[l] *
-                    (2.0 * q[l] + 2.0 * q[l] * q[l] / std::min(64, kNodeTile[l]));
+        double fma = 30.0 * I.uR * I.vR;
+        for (int l = 0; l < kNodeLevels; ++l) {
+            fma += (double)tiles[l].size() * kNodeTile[l] * kNodeTile[l] *
+                   (2.0 * q[l] + 2.0 * q[l] * q[l] / std::min(64, kNodeTile[l]));
+            cost.levels += !tiles[l].empty();
+        }
+        cost.work += kExpandCost * fma;
     }
 };
 
@@ -182,25 +194,24 @@ bool node_mask_any(const unsigned long long* m, int begin, int n) {
     return false;
 }
 
-double node_pixel_chain(const SeriesInst& I, const SeriesSph* sph) {
-    double one = 0.0;
-    for (int s = 0; s < I.ns; ++s) one += point_cost(sph[s].s.Nl + 1);
-    return one;
+NodeCost node_pixel_cost(const SeriesInst& I, const SeriesSph* sph, bool planar) {
+    NodeCost c;
+    for (int s = 0; s < I.ns; ++s) c.chain += point_cost(sph[s].s.Nl + 1, planar);
+    c.work = (c.chain + kPointCost) * I.uR * I.vR;
+    return c;
 }
 
-void node_plan_instance(const SeriesInst& I, const SeriesSph* sph, NodeTables* t) {
+NodeCost node_plan_instance(const SeriesInst& I, const SeriesSph* sph, bool planar, NodeTables* t) {
     const int at = (int)t->inst.size();
     t->inst.push_back(NodeInst{});
-    const double pixels = node_pixel_chain(I, sph) * I.uR * I.vR;
-    // a slice whose pixels are some four waves per SIMD for one small sphere
-    // is bound by latency: another launch costs what its points would save
-    if (I.ns == 0 || pixels < kNodeMinWork) return;
-    Tiling wide(I, sph, 0), narrow(I, sph, 1);
+    const NodeCost pixels = node_pixel_cost(I, sph, planar);
+    if (I.ns == 0 || pixels.work < kNodeMinWork) return pixels;
+    Tiling wide(I, sph, planar, 0), narrow(I, sph, planar, 1);
     if (narrow.active[1] || narrow.active[2] || narrow.active[3]) narrow.run();
-    else return;
+    else return pixels;
     if (wide.active[0]) wide.run();
-    Tiling& g = wide.active[0] && wide.cost < narrow.cost ? wide : narrow;
-    if (g.cost > 0.8 * pixels) return;
+    Tiling& g = wide.active[0] && wide.cost.work < narrow.cost.work ? wide : narrow;
+    if (g.cost.levels == 0 || g.cost.work > 0.8 * pixels.work) return pixels;
     NodeInst& N = t->inst[at];
     N.words = g.words;
     N.tile_first = (int)t->tiles.size();
@@ -235,10 +246,6 @@ void node_plan_instance(const SeriesInst& I, const SeriesSph* sph, NodeTables* t
         t->tiles.insert(t->tiles.end(), g.tiles[l].begin(), g.tiles[l].end());
         t->mask.insert(t->mask.end(), g.mask[l].begin(), g.mask[l].end());
     }
-    if (N.n_lev == 0) {   // every tile is near every sphere
-        N = NodeInst{};
-        return;
-    }
     N.near0 = (int)t->tiles.size();
     N.n_near = (int)g.tiles[kNodeLevels].size();
     N.near_idx0 = grid(g.tiles[kNodeLevels], kNearTile, &N.near_gw);
@@ -249,6 +256,7 @@ void node_plan_instance(const SeriesInst& I, const SeriesSph* sph, NodeTables* t
     for (int y = 0; y < (I.vR + kBlock - 1) / kBlock; ++y)
         for (int x = 0; x < (I.uR + kBlock - 1) / kBlock; ++x)
             t->blocks.push_back(make_int4(at, x, y, 0));
+    return g.cost;
 }
 
 namespace {

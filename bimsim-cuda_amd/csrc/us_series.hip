@@ -917,8 +917,7 @@ static bool harm_planar(const QuadArg& q, const SphereDev& S) {
 // A row of pixels is A + Y v + X u: only those within two pixels of the ends of
 // a sphere's chord in it are tested, and rows and what lies beyond the chords go
 // in whole.  512 x 512 pixels and three to ten spheres: 0.2 to 0.4 ms of the
-// host's for 2.5 to 4
-// with every pixel tested.
+// host's for 2.5 to 4 with every pixel tested.
 bool pixel_order(const SeriesInst& I, const SeriesSph* sph, std::vector<int>* perm) {
     const int end = I.uR;
     const double xx = dot(I.q.X, I.q.X);
@@ -1126,23 +1125,27 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
             }
         }
     }
-    // harmonic form: the nodes of the instances they pay for
+    // harmonic form: the nodes of the instances they pay for, where the plan as
+    // a whole is then faster
     NodeTables nt;
     bool any_nodes = false;
-    double pixel_work = 0.0, chain = 0.0;
-    for (const SeriesInst& I : batch.inst) {
-        const double one = node_pixel_chain(I, batch.sph.data() + I.s_begin);
-        chain = std::max(chain, one);
-        pixel_work += one * I.uR * I.vR;
-    }
-    if (P->harmonic && (pixel_work >= kNodeMinPlan || chain >= kNodeMinChain)) {
-        for (const SeriesInst& I : batch.inst) {
-            node_plan_instance(I, batch.sph.data() + I.s_begin, &nt);
-            any_nodes = any_nodes || nt.inst.back().n_lev > 0;
-        }
-        if (nt.n_v + nt.n_w >= (1LL << 31) || !any_nodes) {   // (node numbers are ints)
-            any_nodes = false;
-            nt = NodeTables();
+    if (P->harmonic) {
+        bool planar = true;
+        for (const SeriesInst& I : batch.inst)
+            for (int t = I.s_begin; t < I.s_begin + I.ns; ++t)
+                planar = planar && harm_planar(I.q, batch.sph[t].s);
+        NodeCost pixels, nodes;
+        for (const SeriesInst& I : batch.inst)
+            pixels.add(node_pixel_cost(I, batch.sph.data() + I.s_begin, planar));
+        if (pixels.total() > kNodeLaunch + kNodeLevel) {
+            for (const SeriesInst& I : batch.inst) {
+                nodes.add(node_plan_instance(I, batch.sph.data() + I.s_begin, planar, &nt));
+                any_nodes = any_nodes || nt.inst.back().n_lev > 0;
+            }
+            if (nt.n_v + nt.n_w >= (1LL << 31) ||   // (node numbers are ints)
+                nodes.total() >= pixels.total())
+                any_nodes = false;
+            if (!any_nodes) nt = NodeTables();
         }
     }
     // split the waves until the queue holds several items per CU (each
