@@ -1726,24 +1726,32 @@ int series_plan_create_tuned(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_bu
         float best = 1e30f;
         int rc = BIMSIM_OK;
         for (int mult : {1, 2, 4, 8, 16}) {
-            for (int gpc : {2, 4, 8}) {
+            // (a split that no instance takes is the one before it)
+            const bool splits = std::any_of(work.inst.begin(), work.inst.end(), [&](const SeriesInst& I) {
+                return I.nk_pad / mult >= 32;
+            });
+            if (mult > 1 && !splits) break;
+            // the plan there is, or one of its own for another split; the
+            // resident groups are the launch's alone
+            SeriesPlan T;
+            SeriesPlan* const Q = mult == P->split_mult ? P : &T;
+            const int kept = P->groups_per_cu;
+            if (Q == &T) {
                 SeriesBatch cand = batch;
                 for (SeriesInst& I : cand.inst) I.accumulate = 0;
-                SeriesPlan T;
-                rc = series_plan_create(ctx, cand, coef_budget, &T, mult, gpc);
+                rc = series_plan_create(ctx, cand, coef_budget, &T, mult, kept);
                 if (rc != BIMSIM_OK) break;
-                if (mult > 1 && T.split_insts.empty()) {   // no instance splits further
-                    series_plan_destroy(&T);
-                    continue;
-                }
-                rc = series_plan_launch(ctx, T, waves, A, B, tmp);   // warm
+            }
+            for (int gpc : {2, 4, 8}) {
+                Q->groups_per_cu = gpc;
+                rc = series_plan_launch(ctx, *Q, waves, A, B, tmp);   // warm
                 (void)hipEventRecord(e0, ctx->stream);
-                for (int r = 0; r < 2 && rc == BIMSIM_OK; ++r) rc = series_plan_launch(ctx, T, waves, A, B, tmp);
+                for (int r = 0; r < 2 && rc == BIMSIM_OK; ++r)
+                    rc = series_plan_launch(ctx, *Q, waves, A, B, tmp);
                 (void)hipEventRecord(e1, ctx->stream);
                 (void)hipEventSynchronize(e1);
                 float ms = 0.f;
                 (void)hipEventElapsedTime(&ms, e0, e1);
-                series_plan_destroy(&T);
                 if (rc != BIMSIM_OK) break;
                 if (ms < best) {
                     best = ms;
@@ -1751,6 +1759,8 @@ int series_plan_create_tuned(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_bu
                     best_gpc = gpc;
                 }
             }
+            P->groups_per_cu = kept;
+            series_plan_destroy(&T);
             if (rc != BIMSIM_OK) break;
         }
         ctx->timing = timing;
@@ -1763,7 +1773,8 @@ int series_plan_create_tuned(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_bu
         best_mult = hit->second.first;
         best_gpc = hit->second.second;
     }
-    if (best_mult == P->split_mult && best_gpc == P->groups_per_cu) {
+    if (best_mult == P->split_mult) {
+        P->groups_per_cu = best_gpc;
         batch = work;
         return BIMSIM_OK;
     }
