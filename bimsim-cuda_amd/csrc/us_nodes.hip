@@ -78,14 +78,13 @@ struct Tiling {
     // centre in pixels and its squared distance from the plane
     double px, py;
     bool ortho;
-    std::vector<double> cu, cv, cz2, reach;
+    std::vector<double> cu, cv, cz2, reach, one;        // one: its cost at a point
+    std::vector<unsigned long long> cell[kNodeLevels];   // masks of the cell being cut
     std::vector<int2> tiles[kNodeLevels + 1];   // the last: near tiles
     std::vector<unsigned long long> mask[kNodeLevels + 1];
-    bool planar;
     NodeCost cost;
 
-    Tiling(const SeriesInst& inst, const SeriesSph* s, bool all_planar, int top)
-        : I(inst), sph(s), planar(all_planar) {
+    Tiling(const SeriesInst& inst, const SeriesSph* s, bool planar, int top) : I(inst), sph(s) {
         words = (I.ns + 63) / 64;
         const double lx = len(I.q.X), ly = len(I.q.Y);
         px = lx / I.uR;
@@ -105,7 +104,9 @@ struct Tiling {
             cz2.push_back(std::max(0.0, dot(c, c) - a * a - b * b));
             const int order = std::max(sph[t].reach > 0 ? sph[t].reach : S.Nl, 4);
             reach.push_back(std::max(order / I.kmag, S.a) * (1.0 + 1e-9));
+            one.push_back(point_cost(S.Nl + 1, planar));
         }
+        for (auto& c : cell) c.resize(2 * (size_t)words);
     }
     // whether sphere t is far from the tile of level l at pixel (i0, j0): no
     // point of it within reach of the centre, nor within 1.3 half edges
@@ -121,28 +122,37 @@ struct Tiling {
         const d3 p = quad_at(I.q, (i0 + m) / I.uR, (j0 + m) / I.vR);
         return len(sub(p, mk(sph[t].s.p))) - m * (px + py) >= need;
     }
-    void add(int l, int i0, int j0, const std::vector<unsigned long long>& m, int points) {
-        tiles[l].push_back(make_int2(i0, j0));
-        mask[l].insert(mask[l].end(), m.begin(), m.end());
-        double one = 0.0;
-        for (int t = 0; t < I.ns; ++t)
-            if ((m[t >> 6] >> (t & 63)) & 1) one += point_cost(sph[t].s.Nl + 1, planar);
-        cost.work += points * (one + kPointCost);
-        cost.chain = std::max(cost.chain, one);
+    // f(sphere) for each of the mask's
+    template <class F>
+    void each(const unsigned long long* m, F&& f) const {
+        for (int w = 0; w < words; ++w)
+            for (unsigned long long b = m[w]; b; b &= b - 1) f(64 * w + __builtin_ctzll(b));
     }
-    void cut(int l, int i0, int j0, std::vector<unsigned long long> left) {
+    void add(int l, int i0, int j0, const unsigned long long* m, int points) {
+        tiles[l].push_back(make_int2(i0, j0));
+        mask[l].insert(mask[l].end(), m, m + words);
+        double sum = 0.0;
+        each(m, [&](int t) { sum += one[t]; });
+        cost.work += points * (sum + kPointCost);
+        cost.chain = std::max(cost.chain, sum);
+    }
+    // (left and m of a size of tiles are free again once its cell is cut)
+    void cut(int l, int i0, int j0, const unsigned long long* parent) {
+        unsigned long long* const left = cell[l].data();
+        unsigned long long* const m = left + words;
+        std::copy(parent, parent + words, left);
         if (active[l]) {
-            std::vector<unsigned long long> m(words, 0);
+            std::fill(m, m + words, 0);
             bool any = false;
-            for (int t = 0; t < I.ns; ++t)
-                if (((left[t >> 6] >> (t & 63)) & 1) && far(t, l, i0, j0)) {
-                    m[t >> 6] |= 1ull << (t & 63);
-                    any = true;
-                }
+            each(left, [&](int t) {
+                if (!far(t, l, i0, j0)) return;
+                m[t >> 6] |= 1ull << (t & 63);
+                any = true;
+            });
             if (any) add(l, i0, j0, m, (q[l] * q[l] + 63) / 64 * 64);
             for (int w = 0; w < words; ++w) left[w] &= ~m[w];
         }
-        if (std::all_of(left.begin(), left.end(), [](unsigned long long w) { return w == 0; })) return;
+        if (std::all_of(left, left + words, [](unsigned long long w) { return w == 0; })) return;
         if (l == kNodeLevels - 1) {
             add(kNodeLevels, i0, j0, left, kNearTile * kNearTile);
             return;
@@ -162,7 +172,7 @@ struct Tiling {
         }();
         const int T0 = kNodeTile[0];
         for (int j0 = 0; j0 < I.vR; j0 += T0)
-            for (int i0 = 0; i0 < I.uR; i0 += T0) cut(0, i0, j0, all);
+            for (int i0 = 0; i0 < I.uR; i0 += T0) cut(0, i0, j0, all.data());
         double fma = 30.0 * I.uR * I.vR;
         for (int l = 0; l < kNodeLevels; ++l) {
             fma += (double)tiles[l].size() * kNodeTile[l] * kNodeTile[l] *
