@@ -213,8 +213,9 @@ struct DetBatch {
     const void *tw = nullptr, *tw2 = nullptr;   // twiddles of the forward rows, and past them
 };
 bool det_batchable(const bimsim_ctx* ctx, int prec, int N, int ss, int zero_fill);
+// may_wide false: no FP64 columns (DetBatch::wide).
 int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::vector<DetParams>& p,
-                     bool fused, DetBatch* out);
+                     bool fused, bool may_wide, DetBatch* out);
 int det_batch_launch(bimsim_ctx* ctx, const DetBatch& b, const void* U, const void* Uf, void* D,
                      void* Di, void* Abs);
 void det_batch_destroy(DetBatch* b);

@@ -91,6 +91,9 @@ struct bimsim_batch {
     // with another instance)
     std::vector<DetBatch> det;
     std::vector<int> det_single;
+    // without the buffers that only speed or sharpen an FP32 batch (nodes, the
+    // detectors' FP64 columns): where the device has no memory for them
+    bool lean = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -460,11 +463,13 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
         for (SeriesSph& S : mc.sph)
             S.reach = node_reach(S.s, mc.inst[S.inst].kmag, hB.data() + 2 * (size_t)S.s.coeff_off);
         if (!mc.inst.empty()) {
-            BIMSIM_TRY(series_plan_create_tuned(ctx, mc, budget, b->waves, b->d_A, b->d_B, &b->plan_mc));
+            BIMSIM_TRY(series_plan_create_tuned(ctx, mc, budget, b->waves, b->d_A, b->d_B, !b->lean,
+                                                &b->plan_mc));
             b->have_mc = true;
         }
         if (!pw.inst.empty()) {
-            BIMSIM_TRY(series_plan_create_tuned(ctx, pw, budget, b->d_kdirs, b->d_A, b->d_B, &b->plan_pw));
+            BIMSIM_TRY(series_plan_create_tuned(ctx, pw, budget, b->d_kdirs, b->d_A, b->d_B, !b->lean,
+                                                &b->plan_pw));
             b->have_pw = true;
         }
         const int wstride = b->lmax + 2;
@@ -531,38 +536,14 @@ int build(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphe
     for (auto& kv : by_size) {
         b->det.emplace_back();
         BIMSIM_TRY(det_batch_create(ctx, b->prec, b->quirks, kv.first, kv.second, b->fuse_sum,
-                                    &b->det.back()));
+                                    !b->lean, &b->det.back()));
     }
     return BIMSIM_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int bimsim_batch_create(bimsim_ctx* ctx, const bimsim_instance* inst, int n,
-                        const bimsim_sphere* spheres, int n_spheres, const double* waves, int prec,
-                        int quirks, void* D, void* Di, void* Abs, int use_graph, bimsim_batch** out) {
-    if (!ctx || !out) return BIMSIM_E_INVALID;
-    *out = nullptr;
-    BIMSIM_CHECK_ARG(ctx, inst && n >= 1 && D && Di && n_spheres >= 0 && (n_spheres == 0 || spheres),
-                     "bad batch arguments");
-    BIMSIM_CHECK_ARG(ctx, prec >= BIMSIM_FP64_PARITY && prec <= BIMSIM_FP32_FAST, "unknown precision");
-    if (!quirks)
-        return set_error(ctx, BIMSIM_E_UNSUPPORTED, "batches run with the reference recurrences only");
-    bool need_waves = false;
-    for (int i = 0; i < n; ++i)
-        need_waves |= inst[i].uf_mode == BIMSIM_UF_MC ||
-                      (inst[i].uf_mode != BIMSIM_UF_PLANE && inst[i].ns > 0);
-    BIMSIM_CHECK_ARG(ctx, waves || !need_waves, "waves must be given");
-    bimsim_batch* b = new bimsim_batch();
-    b->ctx = ctx;
-    b->prec = prec;
-    b->quirks = quirks;
-    b->waves = waves;
-    b->D = D;
-    b->Di = Di;
-    b->Abs = Abs;
+int create(bimsim_batch* b, const bimsim_instance* inst, int n, const bimsim_sphere* spheres,
+           int n_spheres, int use_graph) {
+    bimsim_ctx* ctx = b->ctx;
     int rc = build(b, inst, n, spheres, n_spheres);
     // one eager pass: results, and every scratch buffer and table the pass
     // needs is in place before a capture
@@ -594,14 +575,52 @@ int bimsim_batch_create(bimsim_ctx* ctx, const bimsim_instance* inst, int n,
             ctx->timing = timing;
         }
     }
-    if (rc != BIMSIM_OK) {
+    return rc;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bimsim_batch_create(bimsim_ctx* ctx, const bimsim_instance* inst, int n,
+                        const bimsim_sphere* spheres, int n_spheres, const double* waves, int prec,
+                        int quirks, void* D, void* Di, void* Abs, int use_graph, bimsim_batch** out) {
+    if (!ctx || !out) return BIMSIM_E_INVALID;
+    *out = nullptr;
+    BIMSIM_CHECK_ARG(ctx, inst && n >= 1 && D && Di && n_spheres >= 0 && (n_spheres == 0 || spheres),
+                     "bad batch arguments");
+    BIMSIM_CHECK_ARG(ctx, prec >= BIMSIM_FP64_PARITY && prec <= BIMSIM_FP32_FAST, "unknown precision");
+    if (!quirks)
+        return set_error(ctx, BIMSIM_E_UNSUPPORTED, "batches run with the reference recurrences only");
+    bool need_waves = false;
+    for (int i = 0; i < n; ++i)
+        need_waves |= inst[i].uf_mode == BIMSIM_UF_MC ||
+                      (inst[i].uf_mode != BIMSIM_UF_PLANE && inst[i].ns > 0);
+    BIMSIM_CHECK_ARG(ctx, waves || !need_waves, "waves must be given");
+    // (what an FP32 batch holds for speed and accuracy alone is left out where
+    // the device has no room for it)
+    for (bool lean : {false, true}) {
+        bimsim_batch* b = new bimsim_batch();
+        b->ctx = ctx;
+        b->prec = prec;
+        b->quirks = quirks;
+        b->waves = waves;
+        b->D = D;
+        b->Di = Di;
+        b->Abs = Abs;
+        b->lean = lean;
+        const int rc = create(b, inst, n, spheres, n_spheres, use_graph);
+        if (rc == BIMSIM_OK) {
+            *out = b;
+            return BIMSIM_OK;
+        }
         (void)hipDeviceSynchronize();
         release(b);
         delete b;
-        return rc;
+        if (rc != BIMSIM_E_NOMEM || prec != BIMSIM_FP32_FAST || lean) return rc;
+        (void)hipGetLastError();
     }
-    *out = b;
-    return BIMSIM_OK;
+    return BIMSIM_E_NOMEM;
 }
 
 int bimsim_batch_launch(bimsim_batch* b) {

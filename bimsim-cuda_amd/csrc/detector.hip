@@ -1104,13 +1104,18 @@ int detector_impl(bimsim_ctx* ctx, void* U, void* Uf, int uR, int vR, int nin, i
     const int nrows = write_filtered ? vR : Nd * ss;
     const int* colsd = nullptr;
     void *G = nullptr, *H = nullptr, *I = nullptr;
-    const bool wide = !dbl && det_wide(ctx, uR, vR);
     BIMSIM_TRY(int_table_get(ctx, cols, &colsd));
     BIMSIM_TRY(scratch_get(ctx, kSlotFftA, sizeof(C) * 2 * (size_t)std::max(Nc, 1) * vR, &G));
-    H = G;
-    if (wide)
-        BIMSIM_TRY(scratch_get(ctx, kSlotDet, sizeof(double2) * 2 * (size_t)std::max(Nc, 1) * vR, &H));
     BIMSIM_TRY(scratch_get(ctx, kSlotFftB, sizeof(R) * 2 * (size_t)nrows * uR, &I));
+    // FP64 past the columns where there is memory for their filtered copy (and,
+    // under capture, where it is there already)
+    H = G;
+    bool wide = !dbl && det_wide(ctx, uR, vR);
+    if (wide) {
+        H = scratch_try(ctx, kSlotDet, sizeof(double2) * 2 * (size_t)std::max(Nc, 1) * vR);
+        wide = H != nullptr;
+        if (!wide) H = G;
+    }
     return detector_band<R>(ctx, bp, U, Uf, uR, vR, nin, nin_v, padding, Nd, ss, D, Di, Abs,
                             write_filtered, dbl ? (const C*)twd_u : (const C*)twf_u,
                             dbl || wide ? (const void*)twd_u : (const void*)twf_u,
@@ -1276,7 +1281,7 @@ bool det_batchable(const bimsim_ctx* ctx, int prec, int N, int ss, int zero_fill
 }
 
 int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::vector<DetParams>& p,
-                     bool fused, DetBatch* out) {
+                     bool fused, bool may_wide, DetBatch* out) {
     *out = DetBatch();
     const bool f32 = prec == BIMSIM_FP32_FAST;
     const size_t cs = f32 ? sizeof(float2) : sizeof(double2);
@@ -1325,7 +1330,7 @@ int det_batch_create(bimsim_ctx* ctx, int prec, int quirks, int N, const std::ve
     // rows (columns) per workgroup, fewer when the batch is small so that
     // each pass still spreads over the chip
     const int n = (int)insts.size();
-    const bool wide = f32 && det_wide(ctx, N, N);
+    const bool wide = f32 && may_wide && det_wide(ctx, N, N);
     int B = rows_per_wg(N), B2 = wide ? rows_per_wg_wide(N) : B, Bc = std::max(1, std::min(8, 2048 / N));
     while (B > 1 && (long long)n * ((max_nin + B - 1) / B) < 512) B /= 2;
     while (B2 > 1 && (long long)n * ((max_nd + B2 - 1) / B2) < 512) B2 /= 2;

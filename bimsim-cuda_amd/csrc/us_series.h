@@ -299,16 +299,16 @@ struct SeriesPlan {
 // the plan's buffers (coefficient storage at most `coef_budget` bytes per
 // chunk unless one instance needs more).  Synchronises the stream.
 // split_mult = 0 picks the split from the queue length; groups_per_cu sets
-// the persistent grid.
+// the persistent grid; nodes false leaves every instance to its pixels.
 int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, SeriesPlan* plan,
-                       int split_mult = 0, int groups_per_cu = 8);
+                       int split_mult = 0, int groups_per_cu = 8, bool nodes = true);
 
 // As series_plan_create, but when the queue is short (a few items per CU)
 // the split and grid are chosen by timing the candidates on these inputs
 // (into a temporary field); the choice is kept in the context per batch
 // shape.  A, B and waves must be ready on the stream.
 int series_plan_create_tuned(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget,
-                             const double* waves, const double2* A, const double2* B,
+                             const double* waves, const double2* A, const double2* B, bool nodes,
                              SeriesPlan* plan);
 void series_plan_destroy(SeriesPlan* plan);
 

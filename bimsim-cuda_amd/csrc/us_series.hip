@@ -1045,7 +1045,7 @@ static void node_items(const NodeTables& nt, int i, int g, int s0, int ns, bool 
 }
 
 int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, SeriesPlan* P,
-                       int split_mult, int groups_per_cu) {
+                       int split_mult, int groups_per_cu, bool may_nodes) {
     *P = SeriesPlan();
     P->groups_per_cu = std::max(1, groups_per_cu);
     const int ni = (int)batch.inst.size();
@@ -1129,7 +1129,7 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     // a whole is then faster
     NodeTables nt;
     bool any_nodes = false;
-    if (P->harmonic) {
+    if (P->harmonic && may_nodes) {
         bool planar = true;
         for (const SeriesInst& I : batch.inst)
             for (int t = I.s_begin; t < I.s_begin + I.ns; ++t)
@@ -1689,10 +1689,11 @@ int harm_tune(bimsim_ctx* ctx, const std::string& shape, const double* waves, co
 }  // namespace
 
 int series_plan_create_tuned(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget,
-                             const double* waves, const double2* A, const double2* B, SeriesPlan* P) {
+                             const double* waves, const double2* A, const double2* B, bool nodes,
+                             SeriesPlan* P) {
     // the heuristic plan first: long queues keep it
     SeriesBatch work = batch;
-    BIMSIM_TRY(series_plan_create(ctx, work, coef_budget, P));
+    BIMSIM_TRY(series_plan_create(ctx, work, coef_budget, P, 0, 8, nodes));
     long long items = 0;
     for (const SeriesPlan::Chunk& ch : P->chunks)
         for (const SeriesPlan::Bucket& K : ch.buckets) items += K.item_count;
@@ -1826,7 +1827,16 @@ int series_cached_plan(bimsim_ctx* ctx, SeriesBatch& batch, const double* waves,
         c->entries.erase(c->entries.begin() + victim);
     }
     SeriesCacheEntry* e = new SeriesCacheEntry();
-    const int rc = series_plan_create_tuned(ctx, batch, (size_t)8 << 30, waves, A, B, &e->plan);
+    // (pixels where there is no memory for the nodes)
+    SeriesBatch again = batch;
+    int rc = series_plan_create_tuned(ctx, batch, (size_t)8 << 30, waves, A, B, true, &e->plan);
+    if (rc == BIMSIM_E_NOMEM) {
+        (void)hipStreamSynchronize(ctx->stream);
+        series_plan_destroy(&e->plan);
+        (void)hipGetLastError();
+        batch = again;
+        rc = series_plan_create_tuned(ctx, batch, (size_t)8 << 30, waves, A, B, false, &e->plan);
+    }
     if (rc != BIMSIM_OK) {
         (void)hipStreamSynchronize(ctx->stream);
         series_plan_destroy(&e->plan);
