@@ -1616,9 +1616,14 @@ int harm_tune(bimsim_ctx* ctx, const std::string& shape, const double* waves, co
         return BIMSIM_OK;
     }
     // the key holds the buckets' orders and planar flags: the variants that
-    // exist differ with them
+    // exist differ with them; and of a plan with nodes, whose items are waves
+    // of nodes and near tiles by the spheres' places, that it has them and each
+    // bucket's number of items within a factor of four
     std::string key = shape;
-    for (const SeriesPlan::Bucket* K : bks) key += "|" + std::to_string(K->L) + (K->planar ? "p" : "g");
+    for (const SeriesPlan::Bucket* K : bks) {
+        key += "|" + std::to_string(K->L) + (K->planar ? "p" : "g");
+        if (P->n_xblocks > 0) key += "n" + std::to_string((31 - __builtin_clz(std::max(1, K->item_count))) / 2);
+    }
     auto hit = ctx->tune_harm.find(key);
     if (hit != ctx->tune_harm.end() && hit->second.size() == bks.size()) {
         for (size_t i = 0; i < bks.size(); ++i) bks[i]->variant = hit->second[i];

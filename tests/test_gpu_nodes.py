@@ -160,3 +160,35 @@ def test_node_batches_eager_captured_and_per_call(pkg, ctx):
         m = i["Nd"] ** 2
         assert (imgs[0][off: off + m] - one.D).norm() <= 2e-6 * one.D.norm()
         off += m
+
+
+def test_plans_with_and_without_nodes_are_tuned_apart(pkg, monkeypatch, capfd):
+    """Two plans of one shape (pixels, spheres, orders, waves), the spheres over
+    a narrow slice and a wide one: without nodes and with them, so that the
+    kernel variant timed for one is not taken for the other; a third like the
+    second takes its."""
+    monkeypatch.setenv("BIMSIM_TUNE_LOG", "1")
+    c = pkg.Context(0)
+    k, N, tuned = 1.5, 512, []
+    rng = np.random.default_rng(5)
+    at = [(0.0, 0.0)] + [tuple(rng.uniform(-0.5, 0.5, 2)) for _ in range(9)]
+    spheres, n = [], 0
+    for i in range(10):
+        a = 8.0 / k / (1.0 + 0.02 * i)
+        spheres.append(dict(a=a, n=1.4 + 0.02j, coeff_off=n, Nl=pkg.sphere_order(a, 2 * math.pi / k)))
+        n += spheres[-1]["Nl"] + 1
+    A, B = (torch.zeros(n, dtype=torch.complex128, device="cuda") for _ in range(2))
+    w = torch.tensor(pkg.mc_sample_na(32, (0.0, 0.0, 1.0), 0.1, 0.6, pkg.RNG_SPLITMIX64, 1),
+                     dtype=torch.float64).cuda()
+    U = torch.empty(N * N, dtype=torch.complex64, device="cuda")
+    capfd.readouterr()
+    for width in (20.0, 60.0, 60.01):
+        for s, (x, y) in zip(spheres, at):
+            s["p"] = (x * width, y * width, 0.0)
+        c.mie_coeffs(spheres, k, A, B)
+        c.nf_us(pkg.Quad.xy(width), N, N, (0.0, 0.0, 0.0), k, spheres, A, B, w, 1.0, U,
+                prec=pkg.FP32_FAST)
+        torch.cuda.synchronize()
+        tuned.append(capfd.readouterr().err.count("harmonic waves per SIMD"))
+    assert tuned == [1, 1, 0]
+    c.close()
