@@ -563,26 +563,31 @@ static int lut_eval_launch(bimsim_ctx* ctx, int nl, const EvalTable<Out>& T0,
 }
 
 // The radial tables h (dR radii from max(a, dmin) to dmax) and j (aR from 0 to
-// a) of a sphere, either of them optional (p null).
+// a) of a sphere, either of them optional (p null).  nmax: the radii that the
+// general form's arrays are held for.
 static int lut_radial_launch(bimsim_ctx* ctx, const bimsim_sphere* s, double kmag, double dmin,
-                             double dmax, int dR, const RadialOut& h, int aR, const RadialOut& j) {
+                             double dmax, int dR, const RadialOut& h, int aR, const RadialOut& j,
+                             int nmax) {
     const int nl = s->Nl;
     const double lo = std::max(s->a, dmin), dr = (dmax - lo) / (dR - 1);
     const double ka = kmag * s->a;
+    const int wstride = nl + 2;
+    const size_t work_bytes = sizeof(zj::zc) * 4 * (size_t)wstride * nmax;
     // (a missing table's radii are taken as the sphere's edge)
     const double x0 = h.p ? kmag * lo : ka, x1 = h.p ? kmag * dmax : ka;
     if (lut_closed_radii(nl, x0, x1, j.p ? s->n[0] * ka : ka, j.p ? s->n[1] * ka : 0.0,
                          j.p ? aR : 1)) {
+        // (the general form's arrays, where there is memory for them: a call of
+        // these sizes with another sphere may be captured next)
+        (void)scratch_try(ctx, kSlotMisc, work_bytes);
         const int n = std::max(h.p ? dR : 0, j.p ? aR : 0);
         hipLaunchKernelGGL(lut_radial_kernel, dim3((n + 63) / 64, 3), dim3(64), 0, ctx->stream, nl,
                            kmag, lo, dr, h.p ? dR : 0, h, s->n[0], s->n[1], s->a, j.p ? aR : 0, j);
         BIMSIM_HIP_CHECK(ctx, hipGetLastError());
         return BIMSIM_OK;
     }
-    const int wstride = nl + 2;
-    const int nmax = std::max(h.p ? dR : 0, j.p ? aR : 0);
     void* work = nullptr;
-    BIMSIM_TRY(scratch_get(ctx, kSlotMisc, sizeof(zj::zc) * 4 * (size_t)wstride * nmax, &work));
+    BIMSIM_TRY(scratch_get(ctx, kSlotMisc, work_bytes, &work));
     if (h.p)
         hipLaunchKernelGGL(hankel_lut_kernel, dim3((dR + 63) / 64), dim3(64), 0, ctx->stream, nl,
                            kmag, lo, dr, dR, (double*)work, wstride, h);
@@ -662,14 +667,16 @@ int bimsim_sphere_lut(bimsim_ctx* ctx, const bimsim_sphere* s, const void* A, co
     BIMSIM_CHECK_ARG(ctx, (long long)dR * thetaR <= (1LL << 30), "LUT too large");
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     const int nl = s->Nl;
-    // order by order, so that neighbouring radii's lanes read and write side by side
+    // order by order, so that neighbouring radii's lanes read and write side by
+    // side (room for both tables in any case: a call with Uip may be captured
+    // after one without)
     const int n_j = Uip ? aR : 0;
     void* rad = nullptr;
-    BIMSIM_TRY(scratch_get(ctx, kSlotCoef, sizeof(double2) * (size_t)(nl + 1) * ((size_t)dR + n_j),
+    BIMSIM_TRY(scratch_get(ctx, kSlotCoef, sizeof(double2) * (size_t)(nl + 1) * ((size_t)dR + aR),
                            &rad));
     const RadialOut h = {(double2*)rad, 1, dR};
     const RadialOut j = {Uip ? (double2*)rad + (size_t)(nl + 1) * dR : nullptr, 1, aR};
-    BIMSIM_TRY(lut_radial_launch(ctx, s, kmag, dmin, dmax, dR, h, aR, j));
+    BIMSIM_TRY(lut_radial_launch(ctx, s, kmag, dmin, dmax, dR, h, aR, j, std::max(dR, aR)));
     const double2* Ad = (const double2*)A + s->coeff_off;
     const double2* Bd = (const double2*)B + s->coeff_off;
     // (PI) / (thetaR - 1) is float arithmetic in the reference (sphere.cu:21)
@@ -690,7 +697,8 @@ int bimsim_sphere_radial_lut(bimsim_ctx* ctx, const bimsim_sphere* s, double kma
     BIMSIM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     const int nl = s->Nl;
     return lut_radial_launch(ctx, s, kmag, dmin, dmax, dR, RadialOut{(double2*)h, nl + 1, 1}, aR,
-                             RadialOut{(double2*)j, nl + 1, 1});
+                             RadialOut{(double2*)j, nl + 1, 1},
+                             std::max(h ? dR : 0, j ? aR : 0));
 }
 
 int bimsim_nf_us_lut(bimsim_ctx* ctx, const bimsim_quad* pos, int uR, int vR,

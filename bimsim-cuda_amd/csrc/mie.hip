@@ -177,6 +177,15 @@ extern "C" int bimsim_mie_coeffs(bimsim_ctx* ctx, const bimsim_sphere* spheres, 
     };
     bool closed = closed_lds(wstride, ns) + 1024 <= ctx->lds_max;
     for (int s = 0; s < ns && closed; ++s) closed = mie_closed_form(mie_sph(dev(spheres[s]), kmag));
+    // very high orders: the general form's arrays in global memory (also for a
+    // call of the closed form, where there is memory for them: one of the same
+    // orders that takes the general form may be captured next)
+    const int spb = mie_spheres_per_block(wstride);
+    size_t lds = sizeof(zj::zc) * 8 * (size_t)wstride * spb;
+    const size_t work_bytes = lds > std::min(kMieLds, ctx->lds_max)
+                                  ? sizeof(zj::zc) * 8 * (size_t)wstride * kSphPerLaunch
+                                  : 0;
+    if (closed && work_bytes > 0) (void)scratch_try(ctx, kSlotMisc, work_bytes);
     if (closed) {
         // (the spheres travel as arguments, so that the call captures: 600
         // of them 1107 us as 19 launches of the general form)
@@ -191,13 +200,10 @@ extern "C" int bimsim_mie_coeffs(bimsim_ctx* ctx, const bimsim_sphere* spheres, 
         }
         return BIMSIM_OK;
     }
-    const int spb = mie_spheres_per_block(wstride);
-    size_t lds = sizeof(zj::zc) * 8 * (size_t)wstride * spb;
     void* work = nullptr;
-    if (lds > std::min(kMieLds, ctx->lds_max)) {   // very high orders: global arrays
+    if (work_bytes > 0) {
         lds = 0;
-        BIMSIM_TRY(scratch_get(ctx, kSlotMisc,
-                               sizeof(zj::zc) * 8 * (size_t)wstride * kSphPerLaunch, &work));
+        BIMSIM_TRY(scratch_get(ctx, kSlotMisc, work_bytes, &work));
     }
     for (int s0 = 0; s0 < ns; s0 += kSphPerLaunch) {
         const int cnt = std::min(kSphPerLaunch, ns - s0);

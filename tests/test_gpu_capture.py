@@ -92,3 +92,48 @@ def test_uncached_plan_is_an_error_under_capture(pkg, W):
         assert np.isfinite(host(U)).all()
     finally:
         c.close()
+
+
+def test_tables_of_other_spheres_captured(pkg):
+    """After one eager call of the same sizes a sphere table captures for any
+    sphere: with its inner table where the eager call had none, and with orders
+    that take the general form's arrays where the eager call's did not."""
+    side = torch.cuda.Stream()
+    c = pkg.Context(0, stream=side.cuda_stream)
+    dR, aR, thetaR, kmag, Nl = 70, 40, 33, 2.0, 40
+    g = torch.Generator(device="cuda").manual_seed(3)
+    A, B = (torch.view_as_complex(torch.randn(Nl + 1, 2, generator=g, device="cuda",
+                                              dtype=torch.float64)) for _ in range(2))
+    small, large = (dict(p=(0.0, 0.0, 0.0), a=a, n=1.4 + 0.1j, Nl=Nl, coeff_off=0)
+                    for a in (2.0, 14.0))
+
+    def tables():
+        return [torch.zeros(thetaR * n, dtype=torch.complex128, device="cuda") for n in (dR, aR)]
+
+    def run(s, out, inner=True):
+        c.sphere_lut(s, A, B, kmag, 0.0, 30.0, dR, aR, thetaR, out[0], out[1] if inner else None,
+                     prec=pkg.FP64)
+
+    torch.cuda.synchronize()
+    run(large, tables(), inner=False)
+    torch.cuda.synchronize()
+    got = [tables(), tables()]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        run(large, got[0])
+        run(small, got[1])
+    for _ in range(3):
+        for t in got[0] + got[1]:
+            t.fill_(1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for s, t in zip((large, small), got):
+            want = tables()
+            torch.cuda.synchronize()
+            run(s, want)
+            torch.cuda.synchronize()
+            assert all(torch.equal(x, y) for x, y in zip(t, want))
+    del graph
+    c.close()
