@@ -230,9 +230,9 @@ def headline(pkg, P, W, ctx, torch, args):
     log(f"bench: FP32 eager pass {t_eager * 1e3:.2f} ms; series kernels {series_ms_pass:.2f} ms "
         f"per pass ({spans // reps} spans); graph and eager images equal: {same}")
 
-    # plain FP64 form (and the hoisted FP64 form) on evenly spaced instances
+    # plain FP64 form on evenly spaced instances
     picks = [round(k * (n - 1) / max(1, args.fp64_images - 1)) for k in range(args.fp64_images)]
-    t64 = t64h = us64 = 0.0
+    t64 = us64 = 0.0
     f64 = 0
     err = 0.0
     for k in picks:
@@ -241,12 +241,8 @@ def headline(pkg, P, W, ctx, torch, args):
         us64 += us
         f64 += fp64_parity_flops(insts[k])
         err = max(err, abs_error(Ab32[k], buf.Abs.cpu().numpy(), buf.Di.cpu().numpy()))
-        th, _, _ = fp64_plain(pkg, P, ctx, torch, insts[k], waves[k], pkg.FP64)
-        t64h += th
     t64 /= len(picks)
-    t64h /= len(picks)
-    log(f"bench: FP64 plain {t64 * 1e3:.1f} ms/image, hoisted FP64 {t64h * 1e3:.1f} ms/image, "
-        f"absorbance error {err:.2e}")
+    log(f"bench: FP64 plain {t64 * 1e3:.1f} ms/image, absorbance error {err:.2e}")
 
     traffic = executed_flops = None
     if os.path.exists(PROFILE_TRAFFIC):
@@ -288,7 +284,6 @@ def headline(pkg, P, W, ctx, torch, args):
                                    "for 8)",
                          "flops_per_image": f64 / len(picks)},
         },
-        "fp64_hoisted": {"images_per_s": 1.0 / t64h, "ms_per_image": t64h * 1e3},
         "speedup_vs_fp64_plain": (n / t32) * t64,
         "absorbance_max_abs_err_vs_fp64": err,
         "roofline": {
@@ -584,7 +579,6 @@ def main():
                       "(roofline.flops_per_pass is what it executes), so this is a reference-equivalent rate",
         "eager_pass": h["eager_pass"],
         "fp64_plain": h["fp64_plain"],
-        "fp64_hoisted": h["fp64_hoisted"],
         "speedup_vs_fp64_plain": h["speedup_vs_fp64_plain"],
         "absorbance_max_abs_err_vs_fp64": h["absorbance_max_abs_err_vs_fp64"],
         "roofline": h["roofline"],

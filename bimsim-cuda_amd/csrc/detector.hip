@@ -87,7 +87,7 @@ __device__ inline bool passband(const PostOp& op, int iu, int iv) {
 }
 
 // One instance of a batched detector pass (band-limited path, ss = 1, the
-// images accumulate): its fields at uoff, pass-band columns at cols_off in
+// images written whole): its fields at uoff, pass-band columns at cols_off in
 // the batch's column table, compact spectrum (2 Nc N values) at g_off,
 // images at image_off; crop rows and columns [off, off + Nd).
 struct DetInst {

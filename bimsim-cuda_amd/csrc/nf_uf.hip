@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kThreads) void uf_mc_kernel(QuadArg q, int uR, int 
 // 8 to 100 pixels a wavelength 10 to 25 nodes stand for 64 or 128 pixels.
 // Otherwise (mc_node_tiles) they are the pixels.
 // Bound by the factors and the products' LDS reads in turn; 48 images of
-// 256^2 to 1024^2, 200 to 2000 waves each: 0.42 ms for 2.65 with every pixel
+// 256^2 to 1024^2, 200 to 2000 waves each: 0.34 ms for 2.65 with every pixel
 // evaluated.
 constexpr int kMcTile = 64;
 constexpr int kMcChunk = 32;

@@ -298,9 +298,9 @@ __global__ void us_combine64_kernel(int n, int ns, const double* __restrict__ pa
 // order as us_series64_kernel, whose blocks give a pixel's chains and its waves
 // a wavefront each and leave most of them idle where there are few waves.
 // Bound by FP64 issue.  One wave and one sphere of 18 orders on 256 x 256
-// pixels 11 us (28 in the other form), 512 x 512 22 (85), 1024 x 1024 75 (309);
-// of 116 orders on 512 x 512 79 (574); four waves, four spheres of 39 orders on
-// 512 x 512 217 (433).
+// pixels 11 us (28 in the other form), 512 x 512 20 (85); two spheres of 18 on
+// 1024 x 1024 121 (545); one of 116 orders on 256 x 256 29 (146); four waves, one
+// of 329 orders on 256 x 256 107 (365).
 template <int W>
 __global__ __launch_bounds__(kThreads) void us_few64_kernel(
     QuadArg q, int uR, int vR, d3 f, double kmag, UsSphereBatch batch, int ns,

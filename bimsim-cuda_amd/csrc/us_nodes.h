@@ -19,7 +19,7 @@
 //
 // The harmonic kernel is bound by the instructions of a (point, sphere), so
 // the points are what it costs: on a 64-image sweep (512 x 512, 20 spheres)
-// its launches take 3.6 ms for 9.5 ms, on one image of 1024 x 1024 and 16
+// its launches take 3.6 ms for 9.5 ms, on one image of 1024 x 1024 and 50
 // spheres 0.39 for 1.2 ms, with 0.42 and 0.03 ms for the expansions.
 // A wave holds nodes of one tile only (its last wave partly filled), so that
 // the spheres it skips are the wave's own.  A plan takes the nodes of an

@@ -33,8 +33,19 @@ constexpr int kThreads = 256;
 constexpr int kW = 2;   // waves in flight per thread
 constexpr int kBuckets[] = {16, 24, 32, 40, 48, 64, 80, 96, 112};
 constexpr int kMaxOrders = 112;
-// Waves of pixels per CU up to which a harmonic plan takes one bucket.
+// Waves of pixels per CU, and the largest sphere's order bucket, up to which a
+// harmonic plan takes one bucket.  Measured on images of 64^2 to 768^2 pixels
+// (0.2 to 36 waves a CU), us a call by buckets and by one: orders 13 and 18, 4
+// waves 34 and 31, 16 waves 69 and 46, 36 waves 123 and 75; five spheres of 13 to
+// 45, 107 and 81, 192 and 101, 171 and 118; 13 and 62, 72 and 65, 114 and 89, 184
+// and 134; 13 and 62 off the plane, 242 and 238, 384 and 360, 613 and 588 (at 9
+// waves 266 and 291, the only one slower).  With orders up to 89 nothing is won
+// on small slices (13, 45 and 89, 0.2 to 4 waves: 1.01 to 1.03 times as long, off
+// the plane 0.98 to 1.0; 16 waves 230 and 198, off the plane 852 and 893).
+// Images of more waves were faster with one bucket as well; plans of that size
+// are mostly batches, whose buckets fill the chip each, and were not measured.
 constexpr long long kOneBucketWaves = 16;
+constexpr int kOneBucketOrders = 64;
 
 __device__ inline dc ld2(const double2* p, int i) {
     const double2 v = p[i];
@@ -54,9 +65,10 @@ __constant__ const LegendreScale kLegendreScale = LegendreScale();
 // Phase 1: c'_l(p) (orders padded with zeros to 8 nb) and r-hat(p) for
 // every sphere of a chunk.  Grid: (pixel blocks, spheres of the chunk).
 // ref::shift_j, shift_y and shift_jc with one reciprocal a pixel in place of
-// a division a step (an ulp's difference, far below the complex64 result):
-// bound by FP64 issue, some 25 operations an order; 384 x 384 pixels
-// 62 us for 95 with the divisions.
+// a division a step (an ulp's difference, far below the complex64 result).
+// Bound by the memory it writes: two images of 384 x 384 pixels and five
+// spheres 236 MB in 62 us (95 with the divisions), some 25 FP64 operations an
+// order beside it.
 __global__ __launch_bounds__(kThreads) void series_coef_kernel(
     const SeriesInst* __restrict__ insts, const SeriesSph* __restrict__ sph, int sph_begin,
     int sph_count, const double2* __restrict__ A, const double2* __restrict__ B,
@@ -1093,7 +1105,7 @@ int series_plan_create(bimsim_ctx* ctx, SeriesBatch& batch, size_t coef_budget, 
     if (P->harmonic) {
         split_mult = 1;
         const int top = *std::max_element(bucket.begin(), bucket.end());
-        if ((blocks_all + 0LL) * (kThreads / 64) <= kOneBucketWaves * ctx->cu_count && top <= 64)
+        if ((blocks_all + 0LL) * (kThreads / 64) <= kOneBucketWaves * ctx->cu_count && top <= kOneBucketOrders)
             one_bucket = top;
     }
     auto order_bucket = [&](const SeriesSph& S) {

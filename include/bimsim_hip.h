@@ -44,7 +44,9 @@ typedef enum {
  *   FP64:        the same arithmetic (the scattered field bit for bit).
  *   FP32_FAST:   Bessel terms and Mie products in double, per-wave Legendre
  *                series, plane-wave sum and FFT in float with compensated
- *                accumulation. */
+ *                accumulation; the detector's band-pass and inverse FFT in
+ *                double where their lines fit LDS and memory (see
+ *                bimsim_detector). */
 typedef enum {
     BIMSIM_FP64_PARITY = 0,
     BIMSIM_FP64 = 1,
@@ -241,7 +243,13 @@ int bimsim_nf_sum_uf(bimsim_ctx* ctx, const bimsim_quad* pos, int uR, int vR,
  * -log10(D/Di).  write_filtered != 0 leaves the band-passed fields in U and
  * Uf like the reference (in-place FFT); otherwise U/Uf are left unchanged.
  * quirks = BIMSIM_QUIRKS_REF keeps the reference's negative-frequency index
- * -(uR-1-iu) of the band-pass (microscope.cu:510-518); 0 uses -(uR-iu). */
+ * -(uR-1-iu) of the band-pass (microscope.cu:510-518); 0 uses -(uR-iu).
+ * BIMSIM_FP32_FAST works in double past the pass-band columns of the forward
+ * rows for uR and vR up to 2560, which takes a complex128 copy of those
+ * columns; longer rows, and calls that have no memory for it (or would have
+ * to allocate it under stream capture), work in float throughout: an
+ * absorbance about ten times as far from the FP64 one (8e-6 for 8e-7 at
+ * 512 x 512).  Batches likewise, for all their detectors together. */
 int bimsim_detector(bimsim_ctx* ctx, int prec, int quirks, void* U, void* Uf, int uR,
                     int vR, double du, double dv, double NAin, double NAout,
                     double lambda, int padding, int Nd, int ss, void* D,
@@ -269,7 +277,9 @@ int bimsim_detector_zero_filled(bimsim_ctx* ctx, int prec, int quirks, const voi
  * fixed 64 MiB device array that each GPU the library runs on holds until
  * the process ends; calls needing more return BIMSIM_E_INVALID.  FFT sizes
  * must have a fixed plan (64..4096 of 2^k and 3 2^k, rows fitting LDS),
- * else BIMSIM_E_UNSUPPORTED.  Every call on one GPU shares that array:
+ * else BIMSIM_E_UNSUPPORTED.  BIMSIM_FP32_FAST works in double past the
+ * pass-band columns where the 64 MiB hold their complex128 copy as well,
+ * else in float throughout (bimsim_detector).  Every call on one GPU shares that array:
  * calls that overlap on one GPU (other streams, other threads or contexts)
  * race and must be serialised by the caller. */
 int bimsim_detector_noalloc(bimsim_ctx* ctx, int prec, int quirks, const void* U, const void* Uf,
@@ -473,8 +483,11 @@ typedef struct bimsim_batch bimsim_batch;
  * wavelength, Nl <= 0 asks for sphere::calcNl, coeff_off is ignored.
  * waves: device, rows of 3 doubles.  D, Di (and Abs unless NULL): device
  * images, float for BIMSIM_FP32_FAST and double otherwise; they are
- * overwritten.  The device buffers must stay valid while the batch lives.
- * Creation runs the pass once (results in D/Di/Abs) and synchronises. */
+ * overwritten.  Instances whose images overlap (image_off) add up there.
+ * The device buffers must stay valid while the batch lives.
+ * Creation runs the pass once (results in D/Di/Abs) and synchronises.  A
+ * BIMSIM_FP32_FAST batch that the device has no memory for is created
+ * without what only speeds it or sharpens its detectors, if that suffices. */
 int bimsim_batch_create(bimsim_ctx* ctx, const bimsim_instance* inst, int n,
                         const bimsim_sphere* spheres, int n_spheres,
                         const double* waves, int prec, int quirks, void* D,

@@ -25,14 +25,19 @@ def test_radial_tables(pkg, ctx, orc, a, n, over, dmin, dmax, dR, aR):
     want_h = orc.lut_hankel(nl, kmag, a, dmin, dmax, dR)
     want_j = orc.lut_bessel(nl, kmag, a, n, aR)
     got_h, got_j = h.cpu().numpy().reshape(dR, nl + 1), j.cpu().numpy().reshape(aR, nl + 1)
-    # per order: the functions span many powers of ten.  The oracle's power
-    # series and recurrences lose up to 5e-12 of an order's largest value
-    for got, want in ((got_h.real, want_h.real), (got_h.imag, want_h.imag), (got_j, want_j)):
+    def close(got, want):
+        # per order: the functions span many powers of ten.  The oracle's power
+        # series and recurrences lose up to 5e-12 of an order's largest value
         top = np.abs(want).max(axis=0)
         assert (np.abs(got - want).max(axis=0) <= 1e-11 * top + 1e-200).all()
-    # either table alone is the same
-    h2, j2 = torch.empty_like(h), torch.empty_like(j)
+
+    for got, want in ((got_h.real, want_h.real), (got_h.imag, want_h.imag), (got_j, want_j)):
+        close(got, want)
+    # either table alone, which may take the other form than both together: each
+    # value written, and to the same bound
+    h2, j2 = torch.full_like(h, np.nan), torch.full_like(j, np.nan)
     ctx.sphere_radial_lut(s, kmag, dmin, dmax, dR, 0, h2, None)
     ctx.sphere_radial_lut(s, kmag, dmin, dmax, 0, aR, None, j2)
-    for one, both in ((h2, h), (j2, j)):
-        assert float((one - both).abs().max()) <= 1e-11 * float(both.abs().max())
+    one_h, one_j = h2.cpu().numpy().reshape(got_h.shape), j2.cpu().numpy().reshape(got_j.shape)
+    for one, both in ((one_h.real, got_h.real), (one_h.imag, got_h.imag), (one_j, got_j)):
+        close(one, both)
