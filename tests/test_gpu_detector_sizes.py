@@ -76,6 +76,62 @@ def test_detector_at_any_length(pkg, ctx, N, prec):
             assert (F - D.to(torch.float64)).norm() <= 2 * tol * F.norm()
 
 
+@pytest.mark.parametrize("uR,vR", [(60, 90), (128, 45), (64, 512), (375, 96)])
+@pytest.mark.parametrize("prec", [1, 2])
+def test_rectangular_fields(pkg, ctx, uR, vR, prec):
+    """Rows and columns of different lengths, with a compiled plan or without."""
+    cd, rd = (torch.complex64, torch.float32) if prec == 2 else (torch.complex128, torch.float64)
+    rng = np.random.default_rng(uR)
+    U, Uf = [rng.normal(size=(vR, uR)) + 1j * rng.normal(size=(vR, uR)) for _ in range(2)]
+    lam, Lu, Lv, ss = 4.0, 100.0, 130.0, 1 if uR % 2 else 2
+    Nd = min(uR, vR) // ss
+    na = (0.02, 0.3 * lam * min(uR / Lu, vR / Lv))
+
+    def axis(n, L):
+        i = np.arange(n)
+        return np.where(i <= n // 2, i, -(n - 1 - i)) / L
+
+    f = np.sqrt(axis(uR, Lu)[None, :] ** 2 + axis(vR, Lv)[:, None] ** 2)
+    keep = ~((f < na[0] / lam) | (f > na[1] / lam))
+    ud, ufd = (torch.as_tensor(F.ravel()).to(cd).cuda() for F in (U, Uf))
+    D, Di = (torch.zeros(Nd * Nd, dtype=rd, device="cuda") for _ in range(2))
+    ctx.detector(ud, ufd, uR, vR, 1 / Lu, 1 / Lv, *na, lam, 0, Nd, ss, D, Di, None, prec=prec,
+                 write_filtered=False)
+    tol = 2e-6 if prec == 2 else 1e-13
+    for got, F in ((D, U), (Di, Uf)):
+        G = np.abs(np.fft.ifft2(np.fft.fft2(F) * keep)[: Nd * ss, : Nd * ss]) ** 2
+        want = G.reshape(Nd, ss, Nd, ss).mean(axis=(1, 3)).ravel()
+        got = got.cpu().numpy().astype(np.float64)
+        assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("prec", [1, 2])
+def test_one_transform_size_of_different_fields(pkg, ctx, prec):
+    """Zero-filled and plain instances whose FFTs are of one size share their
+    launches: fields of 50, 100 and 25 samples at 100 points, and two others."""
+    import bimsim_amd.pipeline as P
+    import bimsim_amd.workloads as W
+    insts = []
+    for N, fill in ((50, 2), (100, 0), (25, 4), (40, 0), (50, 0)):
+        i = W.config(1, N=N, nk=20)
+        i["zero_fill"] = fill
+        insts.append(i)
+    waves = [W.mc_waves(i, pkg.mc_sample_na) for i in insts]
+    arr, spheres, Wv, n = P.batch_tables(insts, waves)
+    rd = torch.float32 if prec == 2 else torch.float64
+    D, Di, Ab = (torch.zeros(n, dtype=rd, device="cuda") for _ in range(3))
+    b = ctx.batch(arr, spheres, torch.as_tensor(Wv.ravel()).cuda(), D, Di, Ab, prec=prec)
+    b.launch()
+    at, tol = 0, 2e-6 if prec == 2 else 1e-13
+    for inst, w in zip(insts, waves):
+        one = P.simulate(ctx, inst, torch.as_tensor(w).cuda(), prec)
+        m = inst["Nd"] ** 2
+        for got, want in ((D, one.D), (Di, one.Di)):
+            assert (got[at: at + m] - want).norm() <= tol * want.norm(), inst["N"]
+        at += m
+    b.close()
+
+
 def test_length_with_another_factor_is_refused(pkg, ctx):
     N = 28
     U = torch.zeros(N * N, dtype=torch.complex128, device="cuda")
