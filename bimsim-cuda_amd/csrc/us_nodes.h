@@ -44,8 +44,12 @@ constexpr int kNearTile = 16;       // a near tile is a block's 256 pixels
 constexpr int kNodeMaxQ = 64;
 // Costs are in units of one order of one planar sphere at one point (some
 // 0.7e-6 us where the chip is full).
-// An instance's pixels below which they are evaluated as they are.
-constexpr double kNodeMinWork = 8.0e6;
+// An instance's pixels below which they are evaluated as they are (64 images a
+// batch, one sphere, us by pixels and by nodes: 192 x 192, 39 orders, 2.9e6, 322
+// and 339, 21 orders, 2.2e6, 242 and 241 or on a wide slice 281 and 267; above
+// it 256 x 256, 12 orders, 3.4e6, 345 and 264, 21, 4e6, 362 and 297; 320 x 320,
+// 21, 6.2e6, 633 and 503; 384 x 384, 12, 7.7e6, 752 and 537).
+constexpr double kNodeMinWork = 3.0e6;
 // What a plan's time is but for its points' work: the longest chain of spheres
 // at a point (whatever the number of points), and for nodes the expansion's
 // launch and its phases for each size of tiles.  Fitted to 760 images of 128^2
